@@ -556,20 +556,57 @@ __global__ __launch_bounds__(256) void kda_bwd_zero_outside_kernel(BwdArgs a) {
 // ---- gate parameters ---------------------------------------------------------------
 // g = lb sigmoid(e^A_log (z + b)): dA_log = sum dz (z + b), ddt_bias = sum dz,
 // over the rows the sequences cover.
-__global__ __launch_bounds__(kD) void kda_bwd_gate_partial_kernel(BwdArgs a) {
-  const int h = blockIdx.x, part = blockIdx.y, c = threadIdx.x;
+//
+// Bound by reading dg (fp32) and g once.  One channel per thread and kGateLanes
+// tokens side by side, kGateBatch tokens of loads in flight per thread: 105 ->
+// 21 us at 8,192 tokens x 16 heads (100 MB; one token after the other left one
+// pair of 4-byte loads in flight per thread).  Fixed order: each lane sums its
+// tokens in turn, then lanes, then parts in order.
+constexpr int kGateLanes = 4;
+constexpr int kGateBatch = 8;
+
+template <int G_DT>
+__global__ __launch_bounds__(kGateLanes * kD) void kda_bwd_gate_partial_kernel(BwdArgs a) {
+  const int h = blockIdx.x, part = blockIdx.y, c = threadIdx.x & (kD - 1), lane = threadIdx.x / kD;
+  __shared__ float s_b[kGateLanes][kD], s_a[kGateLanes][kD];
   int64_t lo, hi;
   covered_rows(a, lo, hi);
   const int64_t per = (hi - lo + kGateParts - 1) / kGateParts;
   const int64_t t_lo = imin64(lo + static_cast<int64_t>(part) * per, hi);
   const int64_t t_hi = imin64(t_lo + per, hi);
   const float b = a.dt_bias[h * kD + c];
+  const float *dg = a.dg + static_cast<int64_t>(h) * kD + c;
+  const int64_t dg_stride = static_cast<int64_t>(a.num_heads) * kD;
+  const int64_t gc = static_cast<int64_t>(h) * kD + c;
   float sb = 0.f, sa = 0.f;
-  for (int64_t tok = t_lo; tok < t_hi; ++tok) {
-    const float dz = a.dg[(tok * a.num_heads + h) * kD + c];
-    const float z = load_elem(a.g, tok * a.g_stride + static_cast<int64_t>(h) * kD + c, a.g_dtype);
+  int64_t tok = t_lo + lane;
+  for (; tok + (kGateBatch - 1) * kGateLanes < t_hi; tok += kGateBatch * kGateLanes) {
+    float dz[kGateBatch];
+    uint32_t raw[kGateBatch];
+#pragma unroll
+    for (int i = 0; i < kGateBatch; ++i) {
+      dz[i] = dg[(tok + i * kGateLanes) * dg_stride];
+      raw[i] = load_raw(a.g, (tok + i * kGateLanes) * a.g_stride + gc, G_DT);
+    }
+#pragma unroll
+    for (int i = 0; i < kGateBatch; ++i) {
+      sb += dz[i];
+      sa = fmaf(dz[i], raw_to_f32(raw[i], G_DT) + b, sa);
+    }
+  }
+  for (; tok < t_hi; tok += kGateLanes) {
+    const float dz = dg[tok * dg_stride];
     sb += dz;
-    sa = fmaf(dz, z + b, sa);
+    sa = fmaf(dz, load_elem(a.g, tok * a.g_stride + gc, G_DT) + b, sa);
+  }
+  s_b[lane][c] = sb;
+  s_a[lane][c] = sa;
+  __syncthreads();
+  if (lane != 0) return;
+#pragma unroll
+  for (int l = 1; l < kGateLanes; ++l) {
+    sb += s_b[l][c];
+    sa += s_a[l][c];
   }
   const int64_t o = (static_cast<int64_t>(part) * a.num_heads + h) * kD + c;
   a.gpb[o] = sb;
@@ -580,6 +617,7 @@ __global__ __launch_bounds__(kD) void kda_bwd_gate_final_kernel(BwdArgs a) {
   const int h = blockIdx.x, c = threadIdx.x;
   __shared__ float s_red[2];
   float sb = 0.f, sa = 0.f;
+#pragma unroll 16   // a batch of partials in flight (kGateParts dependent round trips otherwise)
   for (int part = 0; part < kGateParts; ++part) {
     const int64_t o = (static_cast<int64_t>(part) * a.num_heads + h) * kD + c;
     sb += a.gpb[o];
@@ -759,7 +797,12 @@ extern "C" int sophia_kda_chunk_bwd(const void *q, const void *k, const void *v,
     if (const int rc = check_launch("kda_bwd_zero_outside")) return rc;
   }
   if (gate && (dA_log || ddt_bias)) {
-    hipLaunchKernelGGL(kda_bwd_gate_partial_kernel, dim3(num_heads, kGateParts), dim3(kD), 0, st, a);
+    if (g_dtype == SOPHIA_DTYPE_BF16)
+      hipLaunchKernelGGL((kda_bwd_gate_partial_kernel<SOPHIA_DTYPE_BF16>), dim3(num_heads, kGateParts),
+                         dim3(kGateLanes * kD), 0, st, a);
+    else
+      hipLaunchKernelGGL((kda_bwd_gate_partial_kernel<SOPHIA_DTYPE_F32>), dim3(num_heads, kGateParts),
+                         dim3(kGateLanes * kD), 0, st, a);
     if (const int rc = check_launch("kda_bwd_gate_partial")) return rc;
     hipLaunchKernelGGL(kda_bwd_gate_final_kernel, dim3(num_heads), dim3(kD), 0, st, a);
     if (const int rc = check_launch("kda_bwd_gate_final")) return rc;

@@ -442,12 +442,44 @@ struct GateBwdArgs {
   int dtype;
 };
 
+// Eight consecutive elements as loaded, converted to fp32 only when used, so
+// that the loads of several rows are in flight together.
+template <int DT>
+struct Raw8 {
+  u4 w[DT == SOPHIA_DTYPE_BF16 ? 1 : 2];
+  __device__ __forceinline__ void load(const void *base, int64_t idx) {
+    if constexpr (DT == SOPHIA_DTYPE_BF16) {
+      w[0] = *reinterpret_cast<const u4 *>(static_cast<const uint16_t *>(base) + idx);
+    } else {
+      w[0] = *reinterpret_cast<const u4 *>(static_cast<const float *>(base) + idx);
+      w[1] = *reinterpret_cast<const u4 *>(static_cast<const float *>(base) + idx + 4);
+    }
+  }
+  __device__ __forceinline__ void get(float (&v)[8]) const {
+    if constexpr (DT == SOPHIA_DTYPE_BF16) {
+      unpack8(w[0], v);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = __uint_as_float(w[i >> 2][i & 3]);
+    }
+  }
+};
+
+// Bound by memory (o, gate, dy read, d_o and d_gate written once).  A thread's
+// rows are loaded kGnbBatch at a time before any is used: with one row in
+// flight the kernel waited for every row in turn (62 -> 39 us at 8,192 rows x
+// 2,048 columns in bf16, 168 MB: 4.3 TB/s).
+constexpr int kGnbBatch = 4;
+static_assert(kGnbRows % kGnbBatch == 0, "whole batches");
+
+template <int O_DT, int DT>
 __global__ __launch_bounds__(256) void gated_head_norm_bwd_kernel(GateBwdArgs a) {
   __shared__ float s_dw[256][9];
   const int rb = blockIdx.x / a.blocks_per_row;
   const int c = (blockIdx.x - rb * a.blocks_per_row) * 256 + threadIdx.x;
   const int G = a.head_dim >> 3;
   const bool valid = 8 * c < a.width;   // whole heads are valid or not
+  const int cl = valid ? 8 * c : 0;     // lanes past the row read (and never write) its first elements
   const bool norm = a.norm_w != nullptr;
   const int e0 = 8 * (c & (G - 1));
   float w[8], dwacc[8];
@@ -457,55 +489,61 @@ __global__ __launch_bounds__(256) void gated_head_norm_bwd_kernel(GateBwdArgs a)
     dwacc[i] = 0.f;
   }
   const int r_end = min(a.rows, (rb + 1) * kGnbRows);
-  for (int row = rb * kGnbRows; row < r_end; ++row) {   // uniform over the work-group
-    float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, g[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f},
-          dy[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (valid) {
-      load8(static_cast<const uint8_t *>(a.o) + static_cast<int64_t>(row) * a.o_stride * (a.o_dtype == SOPHIA_DTYPE_BF16 ? 2 : 4),
-            8 * c, a.o_dtype, o);
-      load8(static_cast<const uint8_t *>(a.gate) + static_cast<int64_t>(row) * a.gate_stride * (a.dtype == SOPHIA_DTYPE_BF16 ? 2 : 4),
-            8 * c, a.dtype, g);
-      load8(static_cast<const uint8_t *>(a.dy) + static_cast<int64_t>(row) * a.dy_stride * (a.dtype == SOPHIA_DTYPE_BF16 ? 2 : 4),
-            8 * c, a.dtype, dy);
-      if (a.o_dtype != a.dtype) {
+  for (int row0 = rb * kGnbRows; row0 < r_end; row0 += kGnbBatch) {   // uniform over the work-group
+    Raw8<O_DT> ro[kGnbBatch];
+    Raw8<DT> rg[kGnbBatch], rd[kGnbBatch];
+#pragma unroll
+    for (int k = 0; k < kGnbBatch; ++k) {
+      const int64_t row = min(row0 + k, r_end - 1);
+      ro[k].load(a.o, row * a.o_stride + cl);
+      rg[k].load(a.gate, row * a.gate_stride + cl);
+      rd[k].load(a.dy, row * a.dy_stride + cl);
+    }
+#pragma unroll
+    for (int k = 0; k < kGnbBatch; ++k) {
+      const int64_t row = row0 + k;
+      if (row >= r_end) break;   // uniform
+      float o[8], g[8], dy[8];
+      ro[k].get(o);
+      rg[k].get(g);
+      rd[k].get(dy);
+      if constexpr (O_DT != DT) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) o[i] = __uint_as_float(static_cast<uint32_t>(f32_to_bf16_bits(o[i])) << 16);
       }
-    }
-    float sg[8], d_o[8], d_g[8];
+      float sg[8], d_o[8], d_g[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) sg[i] = 1.0f / (1.0f + __expf(-g[i]));
-    if (norm) {   // uniform
-      float ss = 0.f;
+      for (int i = 0; i < 8; ++i) sg[i] = 1.0f / (1.0f + __expf(-g[i]));
+      if (norm) {   // uniform
+        float ss = 0.f;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) ss = fmaf(o[i], o[i], ss);
-      for (int off = G >> 1; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
-      const float r = rsqrtf(ss / static_cast<float>(a.head_dim) + a.eps);
-      float n[8], dn[8], dot = 0.f;
+        for (int i = 0; i < 8; ++i) ss = fmaf(o[i], o[i], ss);
+        for (int off = G >> 1; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+        const float r = rsqrtf(ss / static_cast<float>(a.head_dim) + a.eps);
+        float n[8], dn[8], dot = 0.f;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        n[i] = o[i] * r;
-        dn[i] = dy[i] * sg[i] * w[i];
-        dot = fmaf(dn[i], n[i], dot);
-        d_g[i] = dy[i] * n[i] * w[i] * sg[i] * (1.f - sg[i]);
-        dwacc[i] = fmaf(dy[i] * sg[i], n[i], dwacc[i]);
+        for (int i = 0; i < 8; ++i) {
+          n[i] = o[i] * r;
+          dn[i] = dy[i] * sg[i] * w[i];
+          dot = fmaf(dn[i], n[i], dot);
+          d_g[i] = dy[i] * n[i] * w[i] * sg[i] * (1.f - sg[i]);
+          dwacc[i] = fmaf(dy[i] * sg[i], n[i], dwacc[i]);
+        }
+        for (int off = G >> 1; off > 0; off >>= 1) dot += __shfl_xor(dot, off, 64);
+        const float m = dot / static_cast<float>(a.head_dim);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) d_o[i] = r * (dn[i] - n[i] * m);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          d_o[i] = dy[i] * sg[i];
+          d_g[i] = dy[i] * o[i] * sg[i] * (1.f - sg[i]);
+        }
       }
-      for (int off = G >> 1; off > 0; off >>= 1) dot += __shfl_xor(dot, off, 64);
-      const float m = dot / static_cast<float>(a.head_dim);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) d_o[i] = r * (dn[i] - n[i] * m);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        d_o[i] = dy[i] * sg[i];
-        d_g[i] = dy[i] * o[i] * sg[i] * (1.f - sg[i]);
+      if (valid) {
+        store8(a.d_o, row * a.do_stride + 8 * c, O_DT, d_o);
+        store8(a.d_gate, row * a.dg_stride + 8 * c, DT, d_g);
       }
-    }
-    if (valid) {
-      store8(static_cast<uint8_t *>(a.d_o) + static_cast<int64_t>(row) * a.do_stride * (a.o_dtype == SOPHIA_DTYPE_BF16 ? 2 : 4),
-             8 * c, a.o_dtype, d_o);
-      store8(static_cast<uint8_t *>(a.d_gate) + static_cast<int64_t>(row) * a.dg_stride * (a.dtype == SOPHIA_DTYPE_BF16 ? 2 : 4),
-             8 * c, a.dtype, d_g);
     }
   }
   if (!norm) return;
@@ -521,11 +559,23 @@ __global__ __launch_bounds__(256) void gated_head_norm_bwd_kernel(GateBwdArgs a)
   }
 }
 
-__global__ __launch_bounds__(256) void gated_head_norm_dw_reduce_kernel(GateBwdArgs a) {
-  const int e = blockIdx.x * 256 + threadIdx.x;
-  if (e >= a.head_dim) return;
+// Sums the partials over work-groups: 32 weight positions per work-group, 32
+// lanes of partials side by side (each in order, then the lanes in order), so
+// that 32 x 4 loads are in flight per position instead of one: 119 -> 5 us
+// over the 512 partials of 8,192 rows.
+__global__ __launch_bounds__(1024) void gated_head_norm_dw_reduce_kernel(GateBwdArgs a) {
+  __shared__ float s_part[32][33];
+  const int e = blockIdx.x * 32 + threadIdx.x;
   float acc = 0.f;
-  for (int b = 0; b < a.n_blocks; ++b) acc += a.dw_part[static_cast<int64_t>(b) * a.head_dim + e];
+  if (e < a.head_dim) {
+#pragma unroll 4
+    for (int b = threadIdx.y; b < a.n_blocks; b += 32) acc += a.dw_part[static_cast<int64_t>(b) * a.head_dim + e];
+  }
+  s_part[threadIdx.y][threadIdx.x] = acc;
+  __syncthreads();
+  if (threadIdx.y != 0 || e >= a.head_dim) return;
+#pragma unroll
+  for (int l = 1; l < 32; ++l) acc += s_part[l][threadIdx.x];
   a.dw[e] = acc;
 }
 
@@ -1347,11 +1397,18 @@ extern "C" int sophia_gated_head_norm_bwd(const void *d_out, int64_t d_out_strid
                 static_cast<int>(width), head_dim, blocks_per_row, static_cast<int>(blocks), dtype};
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (blocks > 0) {
-    hipLaunchKernelGGL(gated_head_norm_bwd_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, st, a);
+    constexpr int F = SOPHIA_DTYPE_F32, B = SOPHIA_DTYPE_BF16;
+    const dim3 grid(static_cast<unsigned>(blocks)), block(256);
+    if (dtype == F)
+      hipLaunchKernelGGL((gated_head_norm_bwd_kernel<F, F>), grid, block, 0, st, a);
+    else if (o_dtype == F)
+      hipLaunchKernelGGL((gated_head_norm_bwd_kernel<F, B>), grid, block, 0, st, a);
+    else
+      hipLaunchKernelGGL((gated_head_norm_bwd_kernel<B, B>), grid, block, 0, st, a);
     if (const int rc = check_launch("gated_head_norm_bwd")) return rc;
   }
   if (norm_weight) {
-    hipLaunchKernelGGL(gated_head_norm_dw_reduce_kernel, dim3((head_dim + 255) / 256), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(gated_head_norm_dw_reduce_kernel, dim3((head_dim + 31) / 32), dim3(32, 32), 0, st, a);
     return check_launch("gated_head_norm_dw_reduce");
   }
   return SOPHIA_OK;

@@ -146,6 +146,24 @@ def test_gated_head_norm_backward_matches_float64_autograd(o_dtype, dtype, with_
         assert d_w is None
 
 
+@pytest.mark.parametrize("rows,heads,hd", [(1, 1, 8), (15, 2, 256), (613, 16, 128), (18, 20, 128)])
+def test_gated_head_norm_backward_sizes(rows, heads, hd):
+    """The smallest and largest head sizes, rows that end inside a batch of
+    rows, more partials than lanes of the weight sum, rows of several work-groups."""
+    from sophia_amd import ops
+    dev = _dev()
+    gen = torch.Generator().manual_seed(rows)
+    o, gate, dy = (torch.randn(rows, heads * hd, generator=gen) for _ in range(3))
+    w = torch.rand(hd, generator=gen) + 0.5
+    d_o, d_g, d_w = ops.gated_head_norm_bwd(dy.to(dev), o.to(dev), gate.to(dev), heads, hd, norm_weight=w.to(dev),
+                                            eps=1e-5)
+    o64, g64, w64 = (t.double().requires_grad_(True) for t in (o, gate, w))
+    v = torch.nn.functional.rms_norm(o64.view(rows, heads, hd), (hd,), w64, 1e-5)
+    ((v.reshape(rows, heads * hd) * torch.sigmoid(g64)) * dy.double()).sum().backward()
+    # fp32 arithmetic; the weight's gradient sums rows * heads terms
+    assert _rel(d_o, o64.grad) <= 1e-5 and _rel(d_g, g64.grad) <= 1e-5 and _rel(d_w, w64.grad) <= 1e-4
+
+
 def _trained_like(module, gen):
     """Move A_log, dt_bias and the norm weight off their init values."""
     with torch.no_grad():

@@ -83,6 +83,33 @@ def test_short_conv_backward_matches_float64_autograd(dtype, kernel, with_histor
     assert bool((dx[total:] == 0).all()), "rows past the last sequence"
 
 
+@pytest.mark.parametrize("kernel", [1, 2, 3, 4])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("lens", [[29, 38, 300], [30, 37, 33, 200], [7], [64, 64, 128]])
+def test_short_conv_backward_strip_edges(kernel, dtype, lens):
+    """Sequence starts and ends exactly at, and one row off, the K-1 rows
+    around a 32-row strip (the strips that take the branch-free path and the
+    ones beside them), channels past one work-group (260 = 256 + 4)."""
+    from sophia_amd import ops
+    dev = _dev()
+    gen = torch.Generator().manual_seed(kernel)
+    cu = [0] + np.cumsum(lens).tolist()
+    total, channels = cu[-1], 260
+    x = torch.randn(total, channels, generator=gen).to(dtype)
+    dy = torch.randn(total, channels, generator=gen).to(dtype)
+    w = torch.randn(channels, kernel, generator=gen) * 0.5
+    dx, dw = ops.short_conv_bwd(dy.to(dev), x.to(dev), w.to(dev), torch.tensor(cu, dtype=torch.int32, device=dev))
+    torch.cuda.synchronize()
+    w_r = w.to(dtype).double().requires_grad_(True)
+    x64 = x.double().requires_grad_(True)
+    for a, b in zip(cu[:-1], cu[1:]):
+        y = short_conv_ref(x64[None, a:b], w_r, None)
+        (y[0] * dy[a:b].double()).sum().backward()
+    # fp32 sums of up to 332 terms, exp and rcp at 1 ulp; bf16 dx is rounded once (2^-9)
+    tol = 1e-5 if dtype == torch.float32 else 1e-2
+    assert _rel(dx, x64.grad) <= tol and _rel(dw, w_r.grad) <= 1e-4
+
+
 def test_short_conv_autograd_and_opcheck():
     """sophia::short_conv under autograd gives the backward op's gradients,
     and torch.library.opcheck accepts the op (schema, fake, autograd)."""

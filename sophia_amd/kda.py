@@ -329,10 +329,11 @@ class SophiaKDA(nn.Module):
         y = F.linear(x2, self._input_weight(x2.dtype))
         i, r, h = self.inner_dim, self.decay_rank, self.num_heads
         g = i if self.output_gate_full_rank else self.output_gate_rank
-        qkv = y[:, : 3 * i]
-        gate = y[:, 3 * i: 3 * i + g]
-        dd = y[:, 3 * i + g: 3 * i + g + r]
-        beta = y[:, 3 * i + g + r: 3 * i + g + r + h]
+        # One split, whose backward writes the gradient of y once; a slice per
+        # part would each write a whole zero-padded row set and add it up.
+        sizes = [3 * i, g, r, h]
+        pad = int(y.size(1)) - sum(sizes)
+        qkv, gate, dd, beta = y.split(sizes + [pad] if pad else sizes, 1)[:4]
         if not self.output_gate_full_rank:
             gate = self.output_gate_up(gate)
         return qkv, dd, beta, gate
@@ -422,12 +423,10 @@ class SophiaKDA(nn.Module):
         cu = ops.cu_for_batch(bsz, seqlen, x.device)
         qkv = self._short_convolution_flat(qkv, cu, None, read=cached, write=self.use_cache,
                                            step=(seqlen == 1 and cached and self.use_cache))
-        i = self.inner_dim
         shape4 = (bsz, seqlen, self.num_heads, self.head_dim)
-        # Strided views of the conv output (no copies): the kernels take row strides.
-        q = qkv[:, :i].view(shape4)
-        k = qkv[:, i: 2 * i].view(shape4)
-        v = qkv[:, 2 * i:].view(shape4)
+        # Strided views of the conv output (no copies): the kernels take row
+        # strides.  One unbind: its backward writes the gradient of qkv once.
+        q, k, v = qkv.view(bsz, seqlen, 3, self.num_heads, self.head_dim).unbind(2)
         decay = self.decay_up(dd).view(shape4)
         beta_logits = beta_logits.reshape(bsz, seqlen, self.num_heads)
         if pad_mask is not None:

@@ -585,14 +585,23 @@ __global__ __launch_bounds__(1024) void gated_head_norm_dw_reduce_kernel(GateBwd
 // One work-group (4 wavefronts) per (decode row, key split).  A wavefront takes
 // 16-key tiles of its range in turn and, per tile, on bf16 MFMAs:
 //   S^T[16 keys x 16 heads] = lat[16 x R] . qa^T          (R / 32 MFMAs, K = rank)
-//   lat^T blocks for the value sum: D = lat . I_sel        (one MFMA per 16 ranks)
-//   ctx[16 heads x 16 ranks] += P[16 x 16 keys] . lat      (16x16x16 MFMAs, K = keys)
+//   lat^T tiles for the value sum: D = lat . I_sel         (one MFMA per 16 ranks)
+//   ctx^T[16 ranks x 16 heads] += lat^T . P^T[16 keys]     (16x16x16 MFMAs, K = keys)
 // The accumulator layout of S^T (lane: head = lane % 16, keys 4 (lane / 16) + i)
-// is exactly the A-operand layout of P for the 16x16x16 product, and the
+// is exactly the B-operand layout of P^T for the 16x16x16 product, and the
 // accumulator layout of lat . I_sel (lane: rank column, keys 4 (lane / 16) + i) is
-// its B operand, so no value passes through LDS inside the loop.  Softmax is
-// online (running max and sum per head); the four wavefronts merge through LDS
-// at the end, and key splits, when there are several, in a second kernel.
+// its A operand, so no value passes through LDS inside the loop; in ctx^T a
+// lane's column is its own head, so the running maximum's factor needs no
+// exchange either.  Softmax is online (running max and sum per head); the four
+// wavefronts merge through LDS at the end, and key splits, when there are
+// several, in a second kernel.
+//
+// Bound by reading the latents: two tiles (16 KB) are in flight per wavefront,
+// never under a branch (the prefetch under one made every tile wait for the
+// next), as non-temporal loads of whole 128-byte lines (each latent is read
+// once; 64 bytes of a row per instruction fetch a line twice: 84 us).  240 rows
+// of U[1, 4096) keys, 251 MB: 100 -> 69 us, 3.7 TB/s, where a plain reduction of
+// 1 GiB reads 3.9 TB/s on the same card.
 struct MlaArgs {
   const void *qa;        // [rows, heads, R]
   int64_t qa_stride;     // elements between rows
@@ -629,10 +638,19 @@ __device__ __forceinline__ int mla_keys(const MlaArgs &a, int row, int64_t &slot
   return static_cast<int>(p < 0 ? 0 : (p + 1 > a.max_seq ? a.max_seq : p + 1));
 }
 
+// 16-key tiles per split of a row of `tiles` tiles: an even division, but at
+// least one tile for each wavefront, so that a short row of a long batch does
+// not write (and merge) partials of a few keys each.  The splits past the last
+// tile leave at once and the merge does not read them.
+constexpr int kMlaMinTiles = 4;
+__device__ __forceinline__ int mla_tiles_per_split(int tiles, int splits) {
+  return max((tiles + splits - 1) / splits, kMlaMinTiles);
+}
+
 template <int R>
-__global__ __launch_bounds__(256) void mla_decode_kernel(MlaArgs a) {
+__global__ __launch_bounds__(256, R <= 128 ? 3 : 1) void mla_decode_kernel(MlaArgs a) {
   constexpr int KS = R / 32, NT = R / 16;
-  __shared__ float s_acc[4][16][R];
+  __shared__ __attribute__((aligned(16))) float s_acc[4][16][R + 4];   // rows 4 floats apart in banks
   __shared__ float s_ml[4][2][16];
   const int row = blockIdx.x, split = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -640,22 +658,23 @@ __global__ __launch_bounds__(256) void mla_decode_kernel(MlaArgs a) {
   int64_t slot;
   const int n = mla_keys(a, row, slot);
   const int tiles = (n + 15) >> 4;
-  const int per = (tiles + a.splits - 1) / a.splits;
+  const int per = mla_tiles_per_split(tiles, a.splits);
   const int t0 = split * per, t1 = min(tiles, t0 + per);
+  if (split > 0 && t0 >= tiles) return;   // (split 0 of a row without keys writes its zeros)
   const float *lat = a.latent + slot * a.slot_stride;
 
   // qa^T as B operands (lane: head ln, ranks 32 ks + 8 g + j); heads >= a.heads are zero.
   bf8 qb[KS];
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
-    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (ln < a.heads)
-      load8(static_cast<const uint8_t *>(a.qa) +
-                (static_cast<int64_t>(row) * a.qa_stride + static_cast<int64_t>(ln) * R) *
-                    (a.qa_dtype == SOPHIA_DTYPE_BF16 ? 2 : 4),
-            32 * ks + 8 * g, a.qa_dtype, v);
+    f4 v[2] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
+    if (ln < a.heads) {
+      const int64_t q0 = static_cast<int64_t>(row) * a.qa_stride + static_cast<int64_t>(ln) * R + 32 * ks + 8 * g;
+      v[0] = load4(a.qa, q0, a.qa_dtype);
+      v[1] = load4(a.qa, q0 + 4, a.qa_dtype);
+    }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) qb[ks][j] = static_cast<__bf16>(v[j]);
+    for (int j = 0; j < 8; ++j) qb[ks][j] = static_cast<__bf16>(v[j >> 2][j & 3]);
   }
   // Selection operands: I_h picks ranks 16 h + n of a 32-rank block.
   bf8 sel[2];
@@ -665,33 +684,42 @@ __global__ __launch_bounds__(256) void mla_decode_kernel(MlaArgs a) {
     for (int j = 0; j < 8; ++j)
       sel[hf][j] = static_cast<__bf16>((8 * g + j == 16 * hf + ln) ? 1.0f : 0.0f);
 
-  f4 acc[NT];
+  f4 acc[NT];   // ctx^T: ranks 16 nt + 4 g + i of head ln
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) acc[nt] = f4{0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY, l_run = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;   // of head ln; l_run over this lane's keys alone
 
-  f4 raw[2][KS][2];
-  auto load_tile = [&](int t, f4 (&dst)[KS][2]) {
-    const int key = min(16 * t + ln, n - 1);  // rows past the end are read in bounds and masked
-    const float *rp = lat + static_cast<int64_t>(key) * R + 8 * g;
+  // A load instruction reads 128 whole bytes of eight rows: lane (g, b = bit 3,
+  // k = bits 0..2) takes ranks 32 ks + 8 g + 4 b .. + 3 of keys 16 t + k and
+  // 16 t + 8 + k.  Exchanging bit 3 with the key half (after the conversion to
+  // bf16) then leaves the A operand: ranks 32 ks + 8 g .. + 7 of key 16 t + ln.
+  f4 raw[2][NT];   // [buffer][2 ks + key half]
+  const auto load_tile = [&](int t, f4 (&dst)[NT]) {
+    const int k = 16 * t + (lane & 7);  // rows past the end are read in bounds and masked
+    const float *r0 = lat + static_cast<int64_t>(min(k, n - 1)) * R + 8 * g + ((lane & 8) >> 1);
+    const float *r1 = lat + static_cast<int64_t>(min(k + 8, n - 1)) * R + 8 * g + ((lane & 8) >> 1);
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      dst[ks][0] = *reinterpret_cast<const f4 *>(rp + 32 * ks);
-      dst[ks][1] = *reinterpret_cast<const f4 *>(rp + 32 * ks + 4);
+      dst[2 * ks] = __builtin_nontemporal_load(reinterpret_cast<const f4 *>(r0 + 32 * ks));
+      dst[2 * ks + 1] = __builtin_nontemporal_load(reinterpret_cast<const f4 *>(r1 + 32 * ks));
     }
   };
-  int t = t0 + wave;
-  if (t < t1) load_tile(t, raw[0]);
-  for (; t < t1; t += 4) {
-    if (t + 4 < t1) load_tile(t + 4, raw[1]);
+  // One tile from its buffer, which is refilled (tile `next`) as soon as it is converted.
+  const auto step = [&](int t, int next, f4 (&buf)[NT]) {
     bf8 af[KS];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
+    for (int ks = 0; ks < KS; ++ks) {
+      u2 x = pack4_bf16(buf[2 * ks]), y = pack4_bf16(buf[2 * ks + 1]);
+      u4 w;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        af[ks][j] = static_cast<__bf16>(raw[0][ks][0][j]);
-        af[ks][4 + j] = static_cast<__bf16>(raw[0][ks][1][j]);
+      for (int d = 0; d < 2; ++d) {
+        // row_ror:8 reads lane ^ 8; bank masks 0xc / 0x3 write the lanes with bit 3 set / clear
+        w[d] = __builtin_amdgcn_update_dpp(x[d], y[d], 0x128, 0xf, 0xc, false);
+        w[2 + d] = __builtin_amdgcn_update_dpp(y[d], x[d], 0x128, 0xf, 0x3, false);
       }
+      af[ks] = bits_to_bf8(w);
+    }
+    load_tile(next, buf);
     f4 st = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) st = mfma32(af[ks], qb[ks], st);
@@ -702,8 +730,8 @@ __global__ __launch_bounds__(256) void mla_decode_kernel(MlaArgs a) {
       p[i] = (16 * t + 4 * g + i < n) ? st[i] * a.scale : -INFINITY;
       mx = fmaxf(mx, p[i]);
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = fmaxf(mx, lane_xor16(mx));
+    mx = fmaxf(mx, lane_xor32(mx));
     const float m_new = fmaxf(m_run, mx);  // finite: every tile holds a key < n
     const float alpha = __expf(m_run - m_new);
     float ps = 0.f;
@@ -712,36 +740,39 @@ __global__ __launch_bounds__(256) void mla_decode_kernel(MlaArgs a) {
       p[i] = __expf(p[i] - m_new);
       ps += p[i];
     }
-    ps += __shfl_xor(ps, 16, 64);
-    ps += __shfl_xor(ps, 32, 64);
     l_run = l_run * alpha + ps;
     m_run = m_new;
-    // ctx rows of this lane are heads 4 g + i: their factors live in lanes 4 g + i.
-    float al[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) al[i] = __shfl(alpha, 4 * g + i, 64);
     const bf4 pa = bf4{static_cast<__bf16>(p[0]), static_cast<__bf16>(p[1]), static_cast<__bf16>(p[2]),
                        static_cast<__bf16>(p[3])};
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-      const f4 tr = mfma32(af[nt >> 1], sel[nt & 1], f4{0.f, 0.f, 0.f, 0.f});
-      const bf4 lb = bf4{static_cast<__bf16>(tr[0]), static_cast<__bf16>(tr[1]), static_cast<__bf16>(tr[2]),
+      const f4 tr = mfma32(af[nt >> 1], sel[nt & 1], f4{0.f, 0.f, 0.f, 0.f});   // lat^T: rank 16 nt + ln, keys 4 g + i
+      const bf4 lt = bf4{static_cast<__bf16>(tr[0]), static_cast<__bf16>(tr[1]), static_cast<__bf16>(tr[2]),
                          static_cast<__bf16>(tr[3])};
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[nt][i] *= al[i];
-      acc[nt] = mfma16(pa, lb, acc[nt]);
+      for (int i = 0; i < 4; ++i) acc[nt][i] *= alpha;
+      acc[nt] = mfma16(lt, pa, acc[nt]);
     }
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      raw[0][ks][0] = raw[1][ks][0];
-      raw[0][ks][1] = raw[1][ks][1];
+  };
+  int t = t0 + wave;
+  if (t < t1) {   // wave-uniform
+    // The loads are never under a branch (the wait for one buffer would then be
+    // a wait for both): past the wave's last tile they read it again, unused.
+    const int last = t + ((t1 - 1 - t) & ~3);
+    load_tile(t, raw[0]);
+    load_tile(min(t + 4, last), raw[1]);
+    for (; t + 4 < t1; t += 8) {
+      step(t, min(t + 8, last), raw[0]);
+      step(t + 4, min(t + 12, last), raw[1]);
     }
+    if (t < t1) step(t, last, raw[0]);
   }
-  // Merge the four wavefronts: acc[nt][i] is ctx[head 4 g + i][rank 16 nt + ln].
+  l_run += lane_xor16(l_run);
+  l_run += lane_xor32(l_run);
+  // Merge the four wavefronts.
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) s_acc[wave][4 * g + i][16 * nt + ln] = acc[nt][i];
+    *reinterpret_cast<f4 *>(&s_acc[wave][ln][16 * nt + 4 * g]) = acc[nt];
   if (g == 0) {
     s_ml[wave][0][ln] = m_run;
     s_ml[wave][1][ln] = l_run;
@@ -781,30 +812,53 @@ __global__ __launch_bounds__(256) void mla_decode_kernel(MlaArgs a) {
 }
 
 // Merge of the key splits of one row: ctx = sum_s e^{m_s - M} acc_s / sum_s e^{m_s - M} l_s.
+// One work-group per row and 256 / R heads (one rank of one head per thread), so
+// that a small batch still spreads the partials' reads over the chip, and
+// batches of splits are loaded together: the loop over the splits of all heads
+// by one work-group per row waited for one partial after the other (15 us at
+// 96 rows x 3 splits, 33 us at 8 rows x 8 splits, now about 4).
 template <int R>
 __global__ __launch_bounds__(256) void mla_decode_merge_kernel(MlaArgs a) {
+  constexpr int HPB = 256 / R;
   const int row = blockIdx.x;
-  for (int idx = threadIdx.x; idx < a.heads * R; idx += 256) {
-    const int h = idx / R, r = idx - h * R;
-    const float *pp = a.part + (static_cast<int64_t>(row) * a.splits * 16 + h) * (R + 2);
-    const int64_t step = 16 * static_cast<int64_t>(R + 2);
-    float M = -INFINITY;
-    for (int s = 0; s < a.splits; ++s) M = fmaxf(M, pp[s * step + R]);
-    float num = 0.f, den = 0.f;
-    if (M != -INFINITY) {
-      for (int s = 0; s < a.splits; ++s) {
-        const float e = __expf(pp[s * step + R] - M);
-        num = fmaf(e, pp[s * step + r], num);
-        den = fmaf(e, pp[s * step + R + 1], den);
-      }
+  const int h = blockIdx.y * HPB + threadIdx.x / R, r = threadIdx.x % R;
+  if (h >= a.heads) return;
+  int64_t slot;
+  const int tiles = (mla_keys(a, row, slot) + 15) >> 4;
+  const int per = mla_tiles_per_split(tiles, a.splits);
+  const int used = max(1, (tiles + per - 1) / per);   // splits that wrote a partial
+  const float *pp = a.part + (static_cast<int64_t>(row) * a.splits * 16 + h) * (R + 2);
+  const int64_t step = 16 * static_cast<int64_t>(R + 2);
+  float M = -INFINITY, num = 0.f, den = 0.f;
+  for (int s0 = 0; s0 < used; s0 += 8) {
+    float m[8], l[8], v[8], top = M;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float *q = pp + static_cast<int64_t>(min(s0 + i, used - 1)) * step;   // the last one again, unused
+      m[i] = q[R];
+      l[i] = q[R + 1];
+      v[i] = q[r];
     }
-    const float y = den > 0.f ? num / den : 0.f;
-    const int64_t o = static_cast<int64_t>(row) * a.out_stride + static_cast<int64_t>(h) * R + r;
-    if (a.out_dtype == SOPHIA_DTYPE_BF16)
-      static_cast<uint16_t *>(a.out)[o] = f32_to_bf16_bits(y);
-    else
-      static_cast<float *>(a.out)[o] = y;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) top = fmaxf(top, m[i]);
+    if (top == -INFINITY) continue;   // no keys
+    const float e0 = __expf(M - top);
+    num *= e0;
+    den *= e0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float e = s0 + i < used ? __expf(m[i] - top) : 0.f;
+      num = fmaf(e, v[i], num);
+      den = fmaf(e, l[i], den);
+    }
+    M = top;
   }
+  const float y = den > 0.f ? num / den : 0.f;
+  const int64_t o = static_cast<int64_t>(row) * a.out_stride + static_cast<int64_t>(h) * R + r;
+  if (a.out_dtype == SOPHIA_DTYPE_BF16)
+    static_cast<uint16_t *>(a.out)[o] = f32_to_bf16_bits(y);
+  else
+    static_cast<float *>(a.out)[o] = y;
 }
 
 // ---------------------------------------------------------------------------
@@ -1311,8 +1365,9 @@ extern "C" int sophia_mla_decode_attn(const void *qa, int64_t qa_stride, int qa_
 #define SOPHIA_MLA_CASE(r)                                                                         \
   case r:                                                                                          \
     hipLaunchKernelGGL(mla_decode_kernel<r>, grid, dim3(256), 0, st, a);                           \
-    if (splits > 1) hipLaunchKernelGGL(mla_decode_merge_kernel<r>, dim3(static_cast<unsigned>(rows)), \
-                                       dim3(256), 0, st, a);                                       \
+    if (splits > 1)                                                                                \
+      hipLaunchKernelGGL(mla_decode_merge_kernel<r>,                                               \
+                         dim3(static_cast<unsigned>(rows), (heads + 256 / r - 1) / (256 / r)), dim3(256), 0, st, a); \
     break;
     SOPHIA_MLA_CASE(32) SOPHIA_MLA_CASE(64) SOPHIA_MLA_CASE(128) SOPHIA_MLA_CASE(256)
 #undef SOPHIA_MLA_CASE

@@ -1086,11 +1086,18 @@ def mla_decode_attn(qa: torch.Tensor, latent_cache: torch.Tensor, slots: torch.T
         raise RuntimeError("slots and pos must hold one entry per row")
     n_slots, max_seq = int(latent_cache.size(0)), int(latent_cache.size(1))
     if splits is None:
-        # One work-group per row once the rows fill the chip (the merge of
-        # split partials costs more than it saves there); fewer rows split
-        # their keys so that about 256 work-groups run.
+        # One work-group reads a row's keys at 12.5 ns a key, the chip reads all
+        # rows' keys (about half the bound each) at 0.07 ns a key and row: splits
+        # pay where the longest row's time past the chip's exceeds the merge's 5 us
+        # (96 rows of 1,024 keys: 21.2 us in one part, 17.2 in 8; 160 rows of 600:
+        # 15.5 and 21.9; 240 rows of 4,096: 69 and 71).  Then about three
+        # work-groups per CU, at least one 16-key tile per wavefront, and no more
+        # partials than the merge loads at once (8; the few rows of a small batch
+        # still gain from 16: 8 rows of 2,048 keys 11.3 -> 10.4 us).
         bound = max_seq if max_len is None else min(int(max_len), max_seq)
-        splits = 1 if rows >= 128 else max(1, min(-(-256 // max(rows, 1)), -(-bound // 256)))
+        splits = 1
+        if bound * (180 - rows) > 72000:
+            splits = max(1, min(-(-768 // max(rows, 1)), -(-bound // 64), 16 if rows <= 16 else 8))
     dt = qa.dtype if out_dtype is None else out_dtype
     if out is not None and (not out.is_contiguous() or out.dtype != dt
                             or tuple(out.shape) != (rows, heads, rank)):

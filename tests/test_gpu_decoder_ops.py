@@ -295,6 +295,28 @@ def test_mla_decode_attn_matches_fp64_reference(rank, heads, rows, splits, dtype
         assert float(y[3].abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("rank,rows,splits", [(128, 5, 24), (128, 5, None), (64, 3, 9), (256, 4, 11), (32, 130, 8)])
+def test_mla_decode_attn_many_splits(rank, rows, splits):
+    """More splits than the merge loads at once, rows too short to fill every
+    split (the ones past the last tile write nothing and are not merged), one
+    tile per wavefront, an odd number of tiles per wavefront, a row of one key,
+    a row outside the cache.  Tolerance as above (bf16 probabilities)."""
+    from sophia_amd import ops
+    dev = _dev()
+    g = torch.Generator(device="cpu").manual_seed(rank + rows)
+    max_seq, heads = 1500, 16
+    cache = torch.randn(rows, max_seq, rank, generator=g).to(dev)
+    qa = (torch.randn(rows, heads, rank, generator=g) * 0.3).to(dev, torch.bfloat16)
+    slots = torch.arange(rows, dtype=torch.int32)
+    pos = torch.randint(0, max_seq, (rows,), generator=g)
+    pos[0], pos[1], pos[2] = max_seq - 1, 0, 16 * 4 * 5 + 3
+    if rows > 3:
+        slots[3] = rows
+    y = ops.mla_decode_attn(qa, cache, slots.to(dev), pos.to(dev), 128 ** -0.5, max_len=max_seq, splits=splits)
+    ref = _mla_ref(qa, cache, slots, pos, 128 ** -0.5)
+    assert float((y.double().cpu() - ref).abs().max()) <= 1e-2 * float(ref.abs().max())
+
+
 def _causal_ref(q, k, v, cu, scale):
     """Causal softmax attention per packed sequence, float32 on the host from
     the same bf16 inputs (scaled_dot_product_attention(is_causal=True) per

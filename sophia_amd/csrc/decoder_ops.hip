@@ -19,6 +19,8 @@
 // normalised keys, the softmax weights and the products to the activation
 // dtype in between).  Every kernel is bound by HBM traffic: each input byte
 // is read once and each output byte written once.
+#include <type_traits>
+
 #include "common.hpp"
 
 #include "../../include/sophia_decoder.h"
@@ -870,21 +872,29 @@ __global__ __launch_bounds__(256) void mla_decode_merge_kernel(MlaArgs a) {
 // 0 .. i + (keys - queries).
 //
 // One work-group (4 wavefronts) per (128-query block, head, sequence); a
-// wavefront owns 32 queries.  Per 64-key block, K (row-major) and V (transposed,
-// keys along rows) are staged in LDS by the four wavefronts, then each
-// wavefront forms
+// wavefront owns 32 queries.  Per 64-key block, K and V rows go to LDS as they
+// lie in memory (copies that pass no registers), and each wavefront forms
 //   S^T[keys x queries] = K . Q^T            (A = K rows from LDS, B = Q^T in registers)
-//   O^T[d x queries]   += V^T . P^T          (A = V^T from LDS, B = P^T from the S^T tiles)
-// with v_mfma_f32_16x16x32_bf16.  The S^T accumulators of two 16-key tiles pair
-// into the B operand of the second product (k order 4g..4g+3, 16+4g..16+4g+3,
-// matched by the V^T reads), and O^T puts 4 consecutive head dims of one query
-// in a lane, so the softmax state is per lane and the stores are 8 bytes.  V is
-// transposed on its way into LDS by products with a 0/1 selection matrix.
+//   O^T[d x queries]   += V^T . P^T          (A = V^T by transposing LDS reads, B = P^T from the S^T tiles)
+// with v_mfma_f32_32x32x16_bf16.  A lane of S^T holds one query's scores at half
+// of the keys, so the softmax state is one pair of registers and a row maximum
+// takes one exchange between lane halves; eight consecutive S^T accumulators are
+// the B operand of the second product (k order 8 (j / 4) + 4 (lane / 32) + j % 4,
+// matched by the V^T reads).
+//
+// What bounds it: short sequences wait for memory (16 x 1,024 tokens x 16 heads
+// read and write 268 MB, 67 us at 4 TB/s, before any block is used twice; 177 ->
+// 125 us), long ones the vector instructions of the softmax (an exponential per
+// score at a quarter of the rate; 8 x 4,096 tokens 588 us, 936 TFLOP/s, 37 % of
+// the matrix peak; 1 x 8,192 379 -> 291 us).  Against 16x16x32 tiles, V
+// transposed by matrix products and a register round trip for K and V: half the
+// vector instructions per score, and no registers held by the copies.  Measured
+// and not kept: key blocks from the last one down (132 us; each query block
+// then fetches its own keys first), 64-bit row products in the copies (131 us).
 constexpr int kFaD = 128;          // head dim
 constexpr int kFaQ = 128;          // queries per work-group
 constexpr int kFaK = 64;           // keys per block
-constexpr int kFaLdK = kFaD + 8;   // bf16 row stride of the K tile
-constexpr int kFaLdV = kFaK + 8;   // bf16 row stride of the V^T tile
+constexpr float kFaSlack = 8.f;    // see the running maximum
 
 struct FaArgs {
   const uint16_t *q, *k, *v;       // bf16 rows: token t, head h at t * stride + h * 128
@@ -901,11 +911,31 @@ struct FaArgs {
   float scale_log2;                // softmax scale * log2(e)
 };
 
-__global__ __launch_bounds__(256, 2) void causal_attn_kernel(FaArgs a) {
-  __shared__ __attribute__((aligned(16))) uint16_t sK[kFaK * kFaLdK];
-  __shared__ __attribute__((aligned(16))) uint16_t sVt[kFaD * kFaLdV];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int ln = lane & 15, g = lane >> 4;
+typedef float f16v __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ f16v mfma32x32(const bf8 &a, const bf8 &b, const f16v &c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// Transposing LDS read: the 16 lanes of a group read four rows of 16 elements
+// (lane j: row j / 4, elements 4 (j % 4) .. + 3) and lane j gets column j.
+__device__ __forceinline__ u2 lds_read_tr(const uint16_t *p) {
+  return __builtin_bit_cast(u2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                    (__attribute__((address_space(3))) s4 *)(p)));
+}
+
+// NARROW: 64 rows of k and v span less than 2 GiB, so that a lane's byte offsets
+// within a block are 32-bit constants added to a scalar base (64-bit products
+// per row and block took a quarter of the vector instructions).
+template <bool NARROW>
+__device__ __forceinline__ void causal_attn(const FaArgs &a) {
+  // Two buffers of a block's K and V rows (256 bytes each, as 16-byte chunks:
+  // chunk c of K row r at place c ^ (r % 16), of V row r at c ^ 2 (r % 8), which
+  // keeps both kinds of read free of bank conflicts).
+  __shared__ __attribute__((aligned(1024))) uint16_t sK0[kFaK * kFaD], sK1[kFaK * kFaD];
+  __shared__ __attribute__((aligned(1024))) uint16_t sV0[kFaK * kFaD], sV1[kFaK * kFaD];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ln = lane & 31, half = lane >> 5, l16 = lane & 15;
   // XCD-aware order: work-group b runs on XCD b % 8, and every query block of
   // one (sequence, head) gets the same b % 8, so its K and V rows are fetched
   // from HBM once and then served by that XCD's L2.  Heavy (late) query blocks
@@ -942,147 +972,164 @@ __global__ __launch_bounds__(256, 2) void causal_attn_kernel(FaArgs a) {
   const int wq0 = q0 + 32 * w;                    // first query of this wavefront
   const int wq_last = min(wq0 + 31, len - 1) + off;  // position of the last query it stores
 
-  // Q^T as B operands: lane (query ln of tile qt, g) holds dims 32 ks + 8 g .. +7.
-  bf8 qf[2][4];
+  // Q^T as B operands: lane (query ln, half) holds dims 16 ks + 8 half .. + 7.
+  const int qi = wq0 + ln;
+  bf8 qf[8];
+  {
+    const uint16_t *qp = a.q + (start + min(qi, len - 1)) * a.q_stride + static_cast<int64_t>(h) * kFaD + 8 * half;
 #pragma unroll
-  for (int qt = 0; qt < 2; ++qt) {
-    const int qi = min(wq0 + 16 * qt + ln, len - 1);
-    const uint16_t *qp = a.q + (start + qi) * a.q_stride + static_cast<int64_t>(h) * kFaD + 8 * g;
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) qf[qt][ks] = bits_to_bf8(*reinterpret_cast<const u4 *>(qp + 32 * ks));
+    for (int ks = 0; ks < 8; ++ks) qf[ks] = bits_to_bf8(*reinterpret_cast<const u4 *>(qp + 16 * ks));
   }
-  bf8 sel[2];
+  // Element offsets of this lane's reads within a block (kt / key block added
+  // as constants): K row ln, chunk 2 ks + half; V^T dims 32 dt + 16 (lane / 16 % 2) + l16
+  // of the four rows from 4 half on.
+  int ko[8], vo[4];
 #pragma unroll
-  for (int hf = 0; hf < 2; ++hf)
+  for (int ks = 0; ks < 8; ++ks) ko[ks] = ln * kFaD + 8 * ((2 * ks + half) ^ l16);
+  {
+    const int vrow = 4 * half + (l16 >> 2);
+    const int chunk = 2 * ((lane >> 4) & 1) + ((l16 & 3) >> 1);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) sel[hf][j] = static_cast<__bf16>((8 * g + j == 16 * hf + ln) ? 1.0f : 0.0f);
+    for (int dt = 0; dt < 4; ++dt) vo[dt] = vrow * kFaD + 8 * ((4 * dt + chunk) ^ (2 * vrow)) + 4 * (l16 & 1);
+  }
+  f16v ot[4];
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) ot[dt][i] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;   // l_run over this lane's keys alone
 
-  f4 ot[2][8];
+  // Copies block kb into LDS, 16 rows of K and V per wavefront, four rows (1 KB)
+  // per instruction; in the last block the rows past the last key copy the
+  // block's first 16 bytes (masked below).
+  using Off = typename std::conditional<NARROW, uint32_t, uint64_t>::type;
+  const uint8_t *kbase = reinterpret_cast<const uint8_t *>(a.k + kstart * a.k_stride + static_cast<int64_t>(h) * kFaD);
+  const uint8_t *vbase = reinterpret_cast<const uint8_t *>(a.v + kstart * a.v_stride + static_cast<int64_t>(h) * kFaD);
+  const int r0 = 16 * w + (lane >> 4);
+  Off kofs[4], vofs[4];
 #pragma unroll
-  for (int qt = 0; qt < 2; ++qt)
+  for (int t = 0; t < 4; ++t) {
+    const int r = r0 + 4 * t;
+    kofs[t] = static_cast<Off>(2 * (r * a.k_stride + 8 * (l16 ^ (r & 15))));
+    vofs[t] = static_cast<Off>(2 * (r * a.v_stride + 8 * (l16 ^ (2 * (r & 7)))));
+  }
+  const auto stage = [&](int kb, uint16_t *dk, uint16_t *dv) {
+    const uint8_t *kp = kbase + 2 * kFaK * a.k_stride * kb, *vp = vbase + 2 * kFaK * a.v_stride * kb;
+    const int rows = klen - kb * kFaK;
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt) ot[qt][dt] = f4{0.f, 0.f, 0.f, 0.f};
-  float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.f, 0.f};
-
-  // This lane's K / V rows of a block: key 16 w + ln, dims 32 ks + 8 g .. +7.
-  u4 kr[4], vr[4];
-  auto load_block = [&](int kb) {
-    const int key = min(kb * kFaK + 16 * w + ln, klen - 1);
-    const uint16_t *kp = a.k + (kstart + key) * a.k_stride + static_cast<int64_t>(h) * kFaD + 8 * g;
-    const uint16_t *vp = a.v + (kstart + key) * a.v_stride + static_cast<int64_t>(h) * kFaD + 8 * g;
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      kr[ks] = *reinterpret_cast<const u4 *>(kp + 32 * ks);
-      vr[ks] = *reinterpret_cast<const u4 *>(vp + 32 * ks);
+    for (int t = 0; t < 4; ++t) {
+      const bool in = r0 + 4 * t < rows;
+      __builtin_amdgcn_global_load_lds(kp + (in ? kofs[t] : Off{0}), dk + (16 * w + 4 * t) * kFaD, 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(vp + (in ? vofs[t] : Off{0}), dv + (16 * w + 4 * t) * kFaD, 16, 0, 0);
     }
   };
-  load_block(0);
-  for (int kb = 0; kb < nkb; ++kb) {
+  // One block; `edge`: it may reach past a query or the last key (a constant at
+  // each use, so that the blocks before the edge have no mask and no branch).
+  const auto block = [&](int kb, const uint16_t *sK, const uint16_t *sV, bool edge) {
     const int k0 = kb * kFaK;
-    __syncthreads();  // the previous block's LDS reads are done
+    // st[kt][i] = score(key k0 + 32 kt + 8 (i / 4) + 4 half + i % 4, query qi).
+    f16v st[2];
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      *reinterpret_cast<u4 *>(&sK[(16 * w + ln) * kFaLdK + 32 * ks + 8 * g]) = kr[ks];
+    for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-      for (int hf = 0; hf < 2; ++hf) {
-        const f4 tr = mfma32(bits_to_bf8(vr[ks]), sel[hf], f4{0.f, 0.f, 0.f, 0.f});
-        // tr[i] = V[key 16 w + 4 g + i][dim 32 ks + 16 hf + ln]
-        *reinterpret_cast<u2 *>(&sVt[(32 * ks + 16 * hf + ln) * kFaLdV + 16 * w + 4 * g]) = pack4_bf16(tr);
+      for (int i = 0; i < 16; ++i) st[kt][i] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks)
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+        st[kt] = mfma32x32(bits_to_bf8(*reinterpret_cast<const u4 *>(sK + ko[ks] + 32 * kt * kFaD)), qf[ks], st[kt]);
+    if (edge) {
+      const int last = min(qi + off, klen - 1) - k0 - 4 * half;   // last key of the block this query sees
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          st[kt][i] = 32 * kt + 8 * (i >> 2) + (i & 3) <= last ? st[kt][i] : -INFINITY;
+    }
+    // Raw scores; the scale (times log2 e, > 0) enters through the running max
+    // and one fused multiply-add per exponent.
+    float mx = st[0][0];
+#pragma unroll
+    for (int i = 1; i < 32; ++i) mx = fmaxf(mx, st[i >> 4][i & 15]);
+    mx = fmaxf(mx, lane_xor32(mx));
+    // The reference point m_run follows the maximum only where a score rises
+    // more than 2^kFaSlack above it (the exact same quotient, P up to 2^kFaSlack): after
+    // the first blocks the accumulators then need no rescaling.  m_run is finite
+    // once key 0 has been seen, and key 0 is in the first block.
+    mx *= a.scale_log2;
+    if (__any(mx > m_run + kFaSlack)) {
+      const float m_new = fmaxf(m_run, mx);
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) ot[dt] *= alpha;
+    }
+    float ps = 0.f;
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        st[kt][i] = __builtin_amdgcn_exp2f(fmaf(st[kt][i], a.scale_log2, -m_run));
+        ps += st[kt][i];
+      }
+    l_run += ps;
+#pragma unroll
+    for (int kp = 0; kp < 4; ++kp) {   // 16 keys: k0 + 16 kp ..
+      const f16v &sv = st[kp >> 1];
+      u4 pw;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) pw[i] = pack_bf16x2(sv[8 * (kp & 1) + 2 * i], sv[8 * (kp & 1) + 2 * i + 1]);
+      const bf8 pf = bits_to_bf8(pw);
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) {
+        const u2 lo = lds_read_tr(sV + vo[dt] + 16 * kp * kFaD);
+        const u2 hi = lds_read_tr(sV + vo[dt] + (16 * kp + 8) * kFaD);
+        ot[dt] = mfma32x32(bits_to_bf8(u4{lo.x, lo.y, hi.x, hi.y}), pf, ot[dt]);
       }
     }
+  };
+  // Block kb + 1 is copied while block kb is used; before a block every wavefront
+  // waits for its own copies (nothing else does: the compiler does not tie LDS
+  // reads behind a barrier to copies issued before it) and then for the others'.
+  const auto arrive = [&]() {
+    __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    if (kb + 1 < nkb) load_block(kb + 1);
-    if (k0 > wq_last) continue;  // every key of the block is after this wavefront's queries
-    // Only a block that reaches past this wavefront's first query, or past the
-    // last key, needs the causal / length mask (uniform over the wavefront).
-    const bool masked = k0 + kFaK - 1 > wq0 + off || k0 + kFaK > klen;
-    // S^T tiles: st[kt][qt][i] = score(key k0 + 16 kt + 4 g + i, query wq0 + 16 qt + ln).
-    f4 st[4][2];
-#pragma unroll
-    for (int kt = 0; kt < 4; ++kt) {
-      st[kt][0] = st[kt][1] = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        const bf8 kf = bits_to_bf8(*reinterpret_cast<const u4 *>(&sK[(16 * kt + ln) * kFaLdK + 32 * ks + 8 * g]));
-        st[kt][0] = mfma32(kf, qf[0][ks], st[kt][0]);
-        st[kt][1] = mfma32(kf, qf[1][ks], st[kt][1]);
-      }
-    }
-    bf8 pf[2][2];  // [kp][qt]: P^T as B operands of the value product
-#pragma unroll
-    for (int qt = 0; qt < 2; ++qt) {
-      // Raw scores here; the scale (times log2 e, > 0) enters through the
-      // running max and one fused multiply-add per exponent.
-      float mx = -INFINITY;
-      if (masked) {
-        const int qpos = wq0 + 16 * qt + ln + off;
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int key = k0 + 16 * kt + 4 * g + i;
-            const float sv = (key <= qpos && key < klen) ? st[kt][qt][i] : -INFINITY;
-            st[kt][qt][i] = sv;
-            mx = fmaxf(mx, sv);
-          }
-      } else {
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) mx = fmaxf(mx, st[kt][qt][i]);
-      }
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      const float m_new = fmaxf(m_run[qt], mx * a.scale_log2);
-      // m_new is finite once key 0 has been seen, and key 0 is in the first block.
-      const float alpha = __builtin_amdgcn_exp2f(m_run[qt] - m_new);
-      float ps = 0.f;
-#pragma unroll
-      for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float pv = __builtin_amdgcn_exp2f(fmaf(st[kt][qt][i], a.scale_log2, -m_new));
-          st[kt][qt][i] = pv;
-          ps += pv;
-        }
-      ps += __shfl_xor(ps, 16, 64);
-      ps += __shfl_xor(ps, 32, 64);
-      l_run[qt] = l_run[qt] * alpha + ps;
-      m_run[qt] = m_new;
-#pragma unroll
-      for (int dt = 0; dt < 8; ++dt) ot[qt][dt] *= alpha;
-#pragma unroll
-      for (int kp = 0; kp < 2; ++kp)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          pf[kp][qt][i] = static_cast<__bf16>(st[2 * kp][qt][i]);
-          pf[kp][qt][4 + i] = static_cast<__bf16>(st[2 * kp + 1][qt][i]);
-        }
-    }
-    // O^T += V^T P^T: A = V^T rows dims 16 dt + ln, keys 32 kp + {4g..4g+3, 16+4g..16+4g+3}.
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-      for (int kp = 0; kp < 2; ++kp) {
-        const uint16_t *vrow = &sVt[(16 * dt + ln) * kFaLdV + 32 * kp + 4 * g];
-        const u2 lo = *reinterpret_cast<const u2 *>(vrow);
-        const u2 hi = *reinterpret_cast<const u2 *>(vrow + 16);
-        const bf8 vf = bits_to_bf8(u4{lo.x, lo.y, hi.x, hi.y});
-        ot[0][dt] = mfma32(vf, pf[kp][0], ot[0][dt]);
-        ot[1][dt] = mfma32(vf, pf[kp][1], ot[1][dt]);
-      }
+  };
+  const int nfull = (q0 + off + 1) / kFaK & ~1;   // blocks (in pairs) before every query of the work-group
+  stage(0, sK0, sV0);
+  for (int kb = 0; kb < nfull; kb += 2) {
+    arrive();
+    stage(kb + 1, sK1, sV1);
+    block(kb, sK0, sV0, false);
+    arrive();
+    if (kb + 2 < nkb) stage(kb + 2, sK0, sV0);
+    block(kb + 1, sK1, sV1, false);
   }
-  // ot[qt][dt][i] = O[query wq0 + 16 qt + ln][dim 16 dt + 4 g + i] before the 1 / l.
-#pragma unroll
-  for (int qt = 0; qt < 2; ++qt) {
-    const int qi = wq0 + 16 * qt + ln;
-    if (qi >= len) continue;
-    const float rl = 1.0f / l_run[qt];
-    uint16_t *op = a.out + (start + qi) * a.out_stride + static_cast<int64_t>(h) * kFaD + 4 * g;
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) *reinterpret_cast<u2 *>(op + 16 * dt) = pack4_bf16(ot[qt][dt] * rl);
+  for (int kb = nfull; kb < nkb; kb += 2) {   // at most four blocks
+    arrive();
+    if (kb + 1 < nkb) stage(kb + 1, sK1, sV1);
+    if (kb * kFaK <= wq_last) block(kb, sK0, sV0, true);   // else: after every query of this wavefront
+    if (kb + 1 >= nkb) break;
+    arrive();
+    if (kb + 2 < nkb) stage(kb + 2, sK0, sV0);
+    if ((kb + 1) * kFaK <= wq_last) block(kb + 1, sK1, sV1, true);
   }
+  // ot[dt][i] = O[query qi][dim 32 dt + 8 (i / 4) + 4 half + i % 4] before the 1 / l.
+  l_run += lane_xor32(l_run);
+  if (qi >= len) return;
+  const float rl = 1.0f / l_run;
+  uint16_t *op = a.out + (start + qi) * a.out_stride + static_cast<int64_t>(h) * kFaD + 4 * half;
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      *reinterpret_cast<u2 *>(op + 32 * dt + 8 * i) =
+          pack4_bf16(f4{ot[dt][4 * i] * rl, ot[dt][4 * i + 1] * rl, ot[dt][4 * i + 2] * rl, ot[dt][4 * i + 3] * rl});
 }
+
+__global__ __launch_bounds__(256, 2) void causal_attn_kernel(FaArgs a) { causal_attn<true>(a); }
+__global__ __launch_bounds__(256, 2) void causal_attn_wide_kernel(FaArgs a) { causal_attn<false>(a); }
 
 // ---- MLA latent norms -----------------------------------------------------------
 // The normalisations that follow MLA's down projections (attention.py:611-614):
@@ -1400,8 +1447,12 @@ extern "C" int sophia_causal_attention(const void *q, int64_t q_stride, const vo
   const int64_t pair_groups = (static_cast<int64_t>(heads) * n_seqs + 7) / 8;
   const int64_t blocks = pair_groups * 8 * a.q_blocks;
   SOPHIA_REQUIRE(blocks <= 0x7fffffff, "causal_attention: grid too large");
-  hipLaunchKernelGGL(causal_attn_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), a);
+  const bool narrow = k_stride < (int64_t{1} << 24) && v_stride < (int64_t{1} << 24);
+  const dim3 grid(static_cast<unsigned>(blocks)), block(256);
+  if (narrow)
+    hipLaunchKernelGGL(causal_attn_kernel, grid, block, 0, static_cast<hipStream_t>(stream), a);
+  else
+    hipLaunchKernelGGL(causal_attn_wide_kernel, grid, block, 0, static_cast<hipStream_t>(stream), a);
   return check_launch("causal_attention");
 }
 

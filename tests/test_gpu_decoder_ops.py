@@ -398,6 +398,43 @@ def test_causal_attention_after_cached_keys_matches_reference(queries, keys, hea
     assert err <= 1e-2, err
 
 
+@pytest.mark.parametrize("queries,cached,ramp,wide", [
+    ((128, 64, 1, 130), (63, 64, 65, 0), 0.0, False),   # key offsets around a block: every parity of the edge blocks
+    ((200, 500), (0, 129), 0.2, False),                 # scores that rise by more than 2^8 from block to block
+    ((200, 500), (0, 129), -0.2, False),                # and that fall away: the early keys keep all the weight
+    ((70,), (0,), 0.0, True)])                          # rows 2^24 elements apart: 64-bit row offsets
+def test_causal_attention_edges(queries, cached, ramp, wide):
+    """Block edges, the running maximum's slack in both directions and wide row
+    strides, against float32 on the host.  Tolerance as above."""
+    from sophia_amd import ops
+    dev = _dev()
+    heads = 1 if wide else 2
+    g = torch.Generator(device="cpu").manual_seed(sum(queries) + sum(cached))
+    keys = [a + b for a, b in zip(queries, cached)]
+    cu = torch.tensor([0] + list(np.cumsum(queries)), dtype=torch.int32)
+    cuk = torch.tensor([0] + list(np.cumsum(keys)), dtype=torch.int32)
+    q, k, v = (torch.randn(n, heads, 128, generator=g) for n in (sum(queries), sum(keys), sum(keys)))
+    q[..., 0] = 8.0                                      # a common direction: k[..., 0] shifts every score
+    for s in range(len(keys)):
+        k[int(cuk[s]):int(cuk[s + 1]), :, 0] = ramp * torch.arange(keys[s])[:, None]
+    q, k, v = (t.to(torch.bfloat16) for t in (q, k, v))
+    kd, vd = k.to(dev), v.to(dev)
+    if wide:
+        stride = 1 << 24
+        big = torch.empty(keys[0] * stride, dtype=torch.bfloat16, device=dev)
+        kd, vd = (big.as_strided((keys[0], 1, 128), (stride, 128, 1), at) for at in (0, 4096))
+        kd.copy_(k)
+        vd.copy_(v)
+    y = ops.causal_attention(q.to(dev), kd, vd, cu.to(dev), max(queries), scale=1.0, cu_seqlens_k=cuk.to(dev))
+    ref = torch.zeros(sum(queries), heads, 128)
+    for s in range(len(queries)):
+        a, b, ka, kb = int(cu[s]), int(cu[s + 1]), int(cuk[s]), int(cuk[s + 1])
+        sc = torch.einsum("thd,shd->hts", q[a:b].float(), k[ka:kb].float())
+        sc = sc.masked_fill(~torch.ones(b - a, kb - ka, dtype=torch.bool).tril(kb - ka - (b - a)), float("-inf"))
+        ref[a:b] = torch.einsum("hts,shd->thd", torch.softmax(sc, dim=-1), v[ka:kb].float())
+    assert float((y.float().cpu() - ref).abs().max()) <= 1e-2 * float(ref.abs().max())
+
+
 def test_causal_attention_with_fewer_keys_than_queries():
     """A sequence with fewer keys than queries (0 keys, or 3 keys for 200
     queries) has no causal alignment: with device offsets only, the kernel

@@ -171,6 +171,27 @@ int sophia_causal_attention(const void *q, int64_t q_stride, const void *k, int6
                             const int32_t *cu_seqlens_k, int n_seqs, int64_t total, int64_t total_k, int max_len,
                             int heads, int head_dim, float scale, int dtype, void *stream);
 
+/*
+ * Projections of a few rows (a decode step's): y = x . w^T with x [rows, k],
+ * w [n, k] and y [rows, n] in bf16 (RuntimeLinear.forward,
+ * ml/runtime/model/runtime_linear.py:32-33, without a bias), fp32 sums rounded
+ * once.  rows <= 32; k a multiple of 32; n a multiple of 16; row strides in
+ * elements (x, w: multiples of 8, 16-byte aligned; y: multiple of 4, 8-byte
+ * aligned).  y may not overlap x or w.
+ */
+int sophia_row_linear(const void *x, int64_t x_stride, const void *w, int64_t w_stride, void *y, int64_t y_stride,
+                      int64_t rows, int64_t n, int64_t k, void *stream);
+
+/*
+ * sophia_row_linear of the fused [gate | up] weight w [2 * hidden, k] and
+ * sophia_situ_glu of its result in one launch (FeedForward.forward up to
+ * down_proj, ml/runtime/model/blocks.py:12-27): h [rows, hidden], formed on
+ * the fp32 sums and rounded once.  hidden a multiple of 8; soft caps positive.
+ */
+int sophia_row_linear_situ_glu(const void *x, int64_t x_stride, const void *w, int64_t w_stride, void *h,
+                               int64_t h_stride, int64_t rows, int64_t hidden, int64_t k, float gate_softcap,
+                               float up_softcap, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

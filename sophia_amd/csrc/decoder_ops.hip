@@ -22,6 +22,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "situ.hpp"
 
 #include "../../include/sophia_decoder.h"
 
@@ -274,31 +275,8 @@ __global__ __launch_bounds__(256) void attn_res_mix_kernel(MixArgs a) {
   }
 }
 
-// tanh(x) for x = |z| / cap >= 0 as a fraction num / den: with t = e^{-2x},
-// (1 - t) / (1 + t); below x = 1/8, where 1 - t cancels, the Taylor series
-// x (1 - x^2/3 + 2x^4/15 - 17x^6/315) over 1 (truncation below 2e-9
-// relative).  t is returned for the sigmoid (cap 4: e^{-|z|} = t^2).
-struct Frac {
-  float num, den, t;
-};
-
-__device__ __forceinline__ Frac tanh_frac(float x) {
-  constexpr float kM2Log2e = -2.0f * 1.44269504088896341f;
-  const float t = __builtin_amdgcn_exp2f(kM2Log2e * x);
-  const float x2 = x * x;
-  const float poly = x * fmaf(x2, fmaf(x2, fmaf(x2, -17.0f / 315.0f, 2.0f / 15.0f), -1.0f / 3.0f), 1.0f);
-  const bool small = x < 0.125f;
-  return Frac{small ? poly : 1.0f - t, small ? 1.0f : 1.0f + t, t};
-}
-
-// One 8-element chunk per thread; a block covers 256 chunks of one row.
-//   h = cg tanh(g/cg) sigmoid(g) * cu tanh(u/cu)
-//     = cg cu sgn(g) sgn(u) num_g num_u s / (den_g den_u (1 + e))
-// with e = e^{-|g|} <= 1 and s = 1 (g >= 0) or e (g < 0): every factor of the
-// denominator lies in [1, 2], so one reciprocal serves the element.  With the
-// reference's gate cap of 4 (CAP4), e = t_g^2 and no third exponential is
-// needed.  Arguments are pre-scaled on the host: xg = -2 log2(e) / cg,
-// xu = -2 log2(e) / cu (exponent factors) and rcg = 1 / cg, rcu = 1 / cu.
+// One 8-element chunk per thread; a block covers 256 chunks of one row
+// (situ.hpp has the arithmetic).
 template <bool BF16, bool CAP4>
 __global__ __launch_bounds__(256) void situ_glu_kernel(const void *gu, int64_t gu_stride, void *h, int64_t h_stride,
                                                        int hidden, int blocks_per_row, float rcg, float rcu,
@@ -311,7 +289,6 @@ __global__ __launch_bounds__(256) void situ_glu_kernel(const void *gu, int64_t g
   float g[8], u[8], o[8];
   load8(base, 8 * c, kDt, g);
   load8(base, hidden + 8 * c, kDt, u);
-  constexpr float kM2Log2e = -2.0f * 1.44269504088896341f;
   // With the up cap of 25 nearly every |u| / cu is below 1/8, where tanh_frac
   // takes its series: when that holds for the whole wavefront, the u side
   // skips the exponential and the selects (the same values either way).
@@ -321,24 +298,9 @@ __global__ __launch_bounds__(256) void situ_glu_kernel(const void *gu, int64_t g
   const auto element = [&](auto u_series) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const float ag = fabsf(g[i]);
-      const Frac fg = tanh_frac(ag * rcg);
-      Frac fu;
-      if constexpr (decltype(u_series)::value) {
-        const float x = fabsf(u[i]) * rcu, x2 = x * x;
-        fu = Frac{x * fmaf(x2, fmaf(x2, fmaf(x2, -17.0f / 315.0f, 2.0f / 15.0f), -1.0f / 3.0f), 1.0f), 1.0f, 0.f};
-      } else {
-        fu = tanh_frac(fabsf(u[i]) * rcu);
-      }
-      float e;
-      if constexpr (CAP4)
-        e = fg.t * fg.t;
-      else
-        e = __builtin_amdgcn_exp2f(0.5f * kM2Log2e * ag);
-      const float s = g[i] >= 0.f ? 1.0f : e;
-      const float mag = scale * fg.num * fu.num * s * __builtin_amdgcn_rcpf(fg.den * fu.den * (1.0f + e));
-      // sign of g times sign of u, as a flip of the sign bit
-      o[i] = __uint_as_float(__float_as_uint(mag) ^ ((__float_as_uint(g[i]) ^ __float_as_uint(u[i])) & 0x80000000u));
+      const float x = fabsf(u[i]) * rcu;
+      const Frac fu = decltype(u_series)::value ? Frac{tanh_series(x), 1.0f, 0.f} : tanh_frac(x);
+      o[i] = situ_value<CAP4>(g[i], u[i], fu, rcg, scale);
     }
   };
   if (__all(umax < 0.125f))

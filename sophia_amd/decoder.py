@@ -292,7 +292,7 @@ class SophiaMLA(nn.Module):
         cache = self.latent_cache
         # q_down, kv_down and output_gate in one GEMM; q_norm, kv_norm and the
         # latent-cache writes of every row in one kernel
-        y = F.linear(x, self._input_weight(x.dtype))
+        y = ops.linear(x, self._input_weight(x.dtype))
         q_lat, latent, gate = y[:, :self.q_rank], y[:, self.q_rank:self.q_rank + r], y[:, self.q_rank + r:]
         rect = npre > 0 and bool(step["rectangular"])
         if (self.q_rank % 8 == 0 and r % 8 == 0 and self.q_rank + r <= 512 and int(y.stride(0)) % 8 == 0
@@ -358,7 +358,15 @@ class FeedForward(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         # gate_softcap tanh(g / gate_softcap) sigmoid(g) * up_softcap tanh(u / up_softcap)
         # as one HIP kernel over the fused [gate | up] projection.
-        hidden = ops.situ_glu(self.gate_up_proj(x), self.gate_softcap, self.up_softcap)
+        # For the few rows of a decode step the projection and the activation
+        # are one launch.  A projection with hooks or in another module's place
+        # is called as a module.
+        proj = self.gate_up_proj
+        if type(proj) is RuntimeLinear and proj.bias is None and not (
+                proj._forward_hooks or proj._forward_pre_hooks or proj._backward_hooks or proj._backward_pre_hooks):
+            hidden = ops.linear_situ_glu(x, proj.weight, self.gate_softcap, self.up_softcap)
+        else:
+            hidden = ops.situ_glu(proj(x), self.gate_softcap, self.up_softcap)
         return self.down_proj(hidden)
 
 

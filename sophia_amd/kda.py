@@ -60,7 +60,7 @@ class RuntimeLinear(nn.Module):
             nn.init.zeros_(self.bias)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return F.linear(x, self.weight, self.bias)
+        return ops.linear(x, self.weight, self.bias)
 
 
 class RMSNorm(nn.Module):
@@ -326,7 +326,7 @@ class SophiaKDA(nn.Module):
 
     def _project(self, x2: torch.Tensor):
         """x2: [N, dim] -> views (qkv [N, 3*inner], decay_down, beta, gate_logits)."""
-        y = F.linear(x2, self._input_weight(x2.dtype))
+        y = ops.linear(x2, self._input_weight(x2.dtype))
         i, r, h = self.inner_dim, self.decay_rank, self.num_heads
         g = i if self.output_gate_full_rank else self.output_gate_rank
         # One split, whose backward writes the gradient of y once; a slice per

@@ -807,6 +807,99 @@ def fused_recurrent_kda(q, k, v, g, beta, *, A_log=None, dt_bias=None, scale=Non
     return o.view(bsz, 1, heads, HEAD_DIM), (state if output_final_state else None)
 
 
+# ------------------------------------------------------------------ projections of a few rows
+ROW_LINEAR_MAX = 32   # rows the few-row projection kernel takes
+
+
+def row_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """``F.linear(x, weight)`` of at most ROW_LINEAR_MAX rows in bf16
+    (sophia_row_linear): x [rows, k] with dense rows, weight [n, k] contiguous,
+    k a multiple of 32, n of 16.  Returns [rows, n]."""
+    rows, k = int(x.size(0)), int(x.size(1))
+    n = int(weight.size(0))
+    y = torch.empty((rows, n), dtype=x.dtype, device=x.device)
+    rc = nat.lib().sophia_row_linear(x.data_ptr(), x.stride(0) if rows > 1 else k, weight.data_ptr(), k, y.data_ptr(),
+                                     n, rows, n, k, nat.stream_handle(x.device))
+    nat.check(rc, "sophia_row_linear")
+    return y
+
+
+def _row_linear_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether ``F.linear(x, weight)`` may run on the few-row kernel, and gains
+    by it.  It may when nothing else than the values is asked of the call (no
+    gradient, trace, transform, mode or autocast) and the layout fits.  It gains
+    up to 32 rows and 512 tiles of outputs: with more rows than that each
+    work-group's reads of x weigh as much as the weight's, and past two tiles per
+    CU the library's GEMM is as fast (8,384 x 1,536: 12.1 us against 11.3 at 8
+    rows, the vocabulary's 65,536: 54 against 39)."""
+    if not _values_only(x, weight):   # (first: a wrapped tensor has no pointer to look at)
+        return False
+    k = x.shape[-1]
+    if (x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or x.device.type != "cuda"
+            or weight.device != x.device or x.numel() > ROW_LINEAR_MAX * k or x.numel() == 0
+            or k % 32 or weight.shape[0] % 16 or weight.shape[0] > 512 * 16):
+        return False
+    return (weight.is_contiguous() and x.stride(-1) == 1 and x.data_ptr() % 16 == 0
+            and weight.data_ptr() % 16 == 0)
+
+
+def _values_only(*tensors) -> bool:
+    """True when a call on ``tensors`` computes plain values only: not traced,
+    transformed (functorch, forward-mode), under a dispatch or function mode or
+    autocast, and with no gradient to record."""
+    if torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda"):
+        return False
+    if (torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+            or torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0):
+        return False
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+        return False
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)
+
+
+def _few_rows(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor | None:
+    """x as the [rows, k] view (or copy) that the few-row kernel takes, or None
+    where ``F.linear`` runs."""
+    if weight.dim() != 2 or x.dim() < 2 or x.shape[-1] != weight.shape[1] or not _row_linear_takes(x, weight):
+        return None
+    rows = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
+    if rows.size(0) > 1 and (rows.stride(0) % 8 or rows.stride(0) < rows.size(1)):
+        return None
+    return rows
+
+
+def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
+    """``F.linear``, on the few-row kernel where that applies and gains."""
+    rows = _few_rows(x, weight) if bias is None else None
+    if rows is None:
+        return torch.nn.functional.linear(x, weight, bias)
+    y = row_linear(rows, weight)
+    return y if x.dim() == 2 else y.view(*x.shape[:-1], weight.shape[0])
+
+
+def linear_situ_glu(x: torch.Tensor, weight: torch.Tensor, gate_softcap: float, up_softcap: float) -> torch.Tensor:
+    """``situ_glu(F.linear(x, weight), ...)``: for a few rows in one launch."""
+    rows = _few_rows(x, weight)
+    if rows is None:
+        return situ_glu(torch.nn.functional.linear(x, weight), gate_softcap, up_softcap)
+    h = row_linear_situ_glu(rows, weight, gate_softcap, up_softcap)
+    return h if x.dim() == 2 else h.view(*x.shape[:-1], h.size(1))
+
+
+def row_linear_situ_glu(x: torch.Tensor, weight: torch.Tensor, gate_softcap: float, up_softcap: float) -> torch.Tensor:
+    """``situ_glu(F.linear(x, weight), ...)`` of at most ROW_LINEAR_MAX rows in
+    one launch (sophia_row_linear_situ_glu), the activation formed on the fp32
+    sums: x [rows, k], weight [2H, k] ([gate | up], H a multiple of 8)."""
+    rows, k = int(x.size(0)), int(x.size(1))
+    hidden = int(weight.size(0)) // 2
+    h = torch.empty((rows, hidden), dtype=x.dtype, device=x.device)
+    rc = nat.lib().sophia_row_linear_situ_glu(
+        x.data_ptr(), x.stride(0) if rows > 1 else k, weight.data_ptr(), k, h.data_ptr(), hidden, rows, hidden, k,
+        float(gate_softcap), float(up_softcap), nat.stream_handle(x.device))
+    nat.check(rc, "sophia_row_linear_situ_glu")
+    return h
+
+
 # ------------------------------------------------------------------ decoder layers
 def _aligned(t: torch.Tensor, name: str) -> None:
     if t.data_ptr() % 16:

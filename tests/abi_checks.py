@@ -136,6 +136,17 @@ def check_host_side(lib, nat) -> None:
     rc = lib.sophia_mla_decode_attn(16, 2048, 1, 32, 2048 * 128, 8, 2048, 48, 64, 0.1, 80, 2048, 1, 4,
                                     16, 128, 3, None, 0, None)
     assert rc == nat.SOPHIA_ERR_INVALID and "workspace" in nat.last_error()
+    # Few-row projections: at most 32 rows, k in whole MFMA steps, aligned rows.
+    rc = lib.sophia_row_linear(16, 64, 32, 64, 48, 16, 33, 16, 64, None)
+    assert rc == nat.SOPHIA_ERR_INVALID and "rows" in nat.last_error()
+    rc = lib.sophia_row_linear(16, 64, 32, 64, 48, 16, 4, 16, 40, None)
+    assert rc == nat.SOPHIA_ERR_INVALID and "multiple of 32" in nat.last_error()
+    rc = lib.sophia_row_linear(16, 60, 32, 64, 48, 16, 4, 16, 64, None)
+    assert rc == nat.SOPHIA_ERR_INVALID and "stride" in nat.last_error()
+    rc = lib.sophia_row_linear_situ_glu(16, 64, 32, 64, 48, 16, 4, 12, 64, 4.0, 25.0, None)
+    assert rc == nat.SOPHIA_ERR_INVALID and "multiple of 16" in nat.last_error()
+    rc = lib.sophia_row_linear_situ_glu(16, 64, 32, 64, 48, 16, 4, 16, 64, 0.0, 25.0, None)
+    assert rc == nat.SOPHIA_ERR_INVALID and "soft caps" in nat.last_error()
     # Causal attention: bf16 and head_dim 128 only.
     rc = lib.sophia_causal_attention(16, 2048, 32, 2048, 48, 2048, 64, 2048, 80, None, 2, 100, 0, 64,
                                      16, 128, 0.08, 0, None)

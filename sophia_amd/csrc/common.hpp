@@ -145,6 +145,24 @@ __device__ __forceinline__ float lane_xor32(float v) {
   return __uint_as_float((threadIdx.x & 32) ? r[0] : r[1]);
 }
 
+// Sum over the wavefront, in every lane, without the LDS crossbar: the row
+// swaps, then rotations within the rows of 16 lanes (DPP).  Ten vector
+// instructions where the shuffles of wave_sum are six round trips through LDS,
+// and bit for bit its result: the lanes are added in the same butterfly (a
+// rotation by 4 of values that repeat every 8 lanes is the lane ^ 4, and so on).
+template <int CTRL>
+__device__ __forceinline__ float dpp_rotate(float v) {
+  return __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float wave_sum_dpp(float v) {
+  v += lane_xor32(v);
+  v += lane_xor16(v);
+  v += dpp_rotate<0x128>(v);   // row_ror:8
+  v += dpp_rotate<0x124>(v);
+  v += dpp_rotate<0x122>(v);
+  return v + dpp_rotate<0x121>(v);
+}
+
 // Butterfly sum over the whole 64-lane wavefront.
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll

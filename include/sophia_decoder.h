@@ -192,6 +192,19 @@ int sophia_row_linear_situ_glu(const void *x, int64_t x_stride, const void *w, i
                                int64_t h_stride, int64_t rows, int64_t hidden, int64_t k, float gate_softcap,
                                float up_softcap, void *stream);
 
+/*
+ * Per-head projections: y[r, h, :] = x[r, h, :] . w[h]^T with x [rows, heads,
+ * k], w [heads, n, k] (contiguous) and y [rows, heads, n] in bf16, fp32 sums
+ * rounded once: the products of MLA's decode rows with the head blocks of k_up
+ * and v_up (ml/runtime/model/attention.py:623-628 folded into latent space).
+ * Strides in elements (x: multiples of 8, x and w 16-byte aligned; y: multiples
+ * of 4, 8-byte aligned), rows at least as far apart as their heads reach; k a
+ * multiple of 32, n of 16.  y may not overlap x or w.
+ */
+int sophia_head_linear(const void *x, int64_t x_row_stride, int64_t x_head_stride, const void *w, void *y,
+                       int64_t y_row_stride, int64_t y_head_stride, int64_t rows, int heads, int n, int k,
+                       void *stream);
+
 #ifdef __cplusplus
 }
 #endif

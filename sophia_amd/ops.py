@@ -900,6 +900,30 @@ def row_linear_situ_glu(x: torch.Tensor, weight: torch.Tensor, gate_softcap: flo
     return h
 
 
+def head_linear(x: torch.Tensor, weight: torch.Tensor, *, out: torch.Tensor | None = None) -> torch.Tensor:
+    """Per-head projection (sophia_head_linear): out[r, h] = x[r, h] . weight[h]^T
+    in bf16, x [rows, heads, k] with dense last dim, weight [heads, n, k]
+    contiguous, k a multiple of 32, n of 16.  Returns [rows, heads, n] (or
+    ``out``, whose rows and heads may be strided)."""
+    _gpu(x, "x")
+    _gpu(weight, "weight")
+    rows, heads, k = (int(v) for v in x.shape)
+    n = int(weight.size(1))
+    if tuple(weight.shape) != (heads, n, k) or not weight.is_contiguous() or x.stride(2) != 1 \
+            or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or weight.device != x.device:
+        raise RuntimeError(f"head_linear takes bf16 x [rows, {heads}, {k}] and contiguous weight [{heads}, n, {k}]")
+    y = out if out is not None else torch.empty((rows, heads, n), dtype=x.dtype, device=x.device)
+    if y.dtype != x.dtype or tuple(y.shape) != (rows, heads, n) or y.stride(2) != 1 or y.device != x.device:
+        raise RuntimeError(f"out must be bf16 [{rows}, {heads}, {n}]")
+    xh = x.stride(1) if heads > 1 else k
+    yh = y.stride(1) if heads > 1 else n
+    rc = nat.lib().sophia_head_linear(
+        x.data_ptr(), x.stride(0) if rows > 1 else (heads - 1) * xh + k, xh, weight.data_ptr(), y.data_ptr(),
+        y.stride(0) if rows > 1 else (heads - 1) * yh + n, yh, rows, heads, n, k, nat.stream_handle(x.device))
+    nat.check(rc, "sophia_head_linear")
+    return y
+
+
 # ------------------------------------------------------------------ decoder layers
 def _aligned(t: torch.Tensor, name: str) -> None:
     if t.data_ptr() % 16:

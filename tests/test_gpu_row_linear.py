@@ -133,3 +133,23 @@ def test_feed_forward_few_rows_and_graph(rows):
             x.copy_(torch.randn(rows, 256, generator=torch.Generator().manual_seed(seed)))
             graph.replay()
             assert torch.equal(out, m(x))
+
+
+@pytest.mark.parametrize("rows,heads,n,k", [(1, 1, 16, 32), (8, 16, 128, 128), (240, 16, 128, 128), (17, 3, 144, 96),
+                                            (5, 2, 32, 320)])
+def test_head_linear_matches_float64(rows, heads, n, k):
+    """Rows and outputs that end inside a tile, more than one work-group of
+    outputs, k past one batch of steps; x a slice of a wider row, the output a
+    view of one (nothing written beside it)."""
+    from sophia_amd import ops
+    dev = _dev()
+    g = torch.Generator().manual_seed(rows)
+    wide = torch.randn(rows, heads, k + 8, generator=g).to(torch.bfloat16)
+    w = (torch.randn(heads, n, k, generator=g) * k ** -0.5).to(torch.bfloat16)
+    big = torch.full((rows + 2, heads, n + 4), 3.0, dtype=torch.bfloat16, device=dev)
+    y = ops.head_linear(wide.to(dev)[:, :, 8:], w.to(dev), out=big[1:-1, :, :n])
+    ref = torch.einsum("rhk,hnk->rhn", wide[:, :, 8:].double(), w.double())
+    assert _close(y, ref) and _close(ops.head_linear(wide.to(dev)[:, :, 8:], w.to(dev)), ref)
+    assert bool((big[0] == 3).all() and (big[-1] == 3).all() and (big[1:-1, :, n:] == 3).all())
+    with pytest.raises(RuntimeError):
+        ops.head_linear(wide.to(dev)[:, :, 8:].float(), w.to(dev))

@@ -20,6 +20,14 @@
 // weight rows, so that the activation (SiTU-GLU, blocks.py:12-27 of
 // ml/runtime/model) is formed on the fp32 sums of one tile: the projection is
 // neither rounded nor written.
+//
+// For at most eight rows half of a tile's columns would be empty, and 1,536
+// outputs are 96 tiles on 256 CUs.  The half-tile form puts eight outputs in a
+// work-group: A holds their weights over two parts of k (rows 0-7 and 8-15), B
+// the rows of x over the same two parts, and of the product the two diagonal
+// quadrants are the sums over the parts.  Twice the work-groups, the same bytes
+// per load instruction: under the profiler 1,536 x 3,968 9.0 -> 7.3 us, 1,536 x
+// 2,048 5.3 -> 4.8.
 #include "common.hpp"
 #include "situ.hpp"
 
@@ -48,34 +56,40 @@ struct RowLinearArgs {
 __device__ __forceinline__ bf8 as_bf8(u4 w) { return __builtin_bit_cast(bf8, w); }
 
 // NW wavefronts, NT tiles of outputs (sharing the loads of x), MT tiles of 16
-// rows of x.
-template <int NW, int NT, int MT, bool GLU, bool CAP4>
+// rows of x.  HALF: eight outputs per tile for at most eight rows, k split over
+// 2 NW parts, a lane's part by its half of the 16.
+template <int NW, int NT, int MT, bool GLU, bool CAP4, bool HALF>
 __global__ __launch_bounds__(NW * 64) void row_linear_kernel(RowLinearArgs a) {
   __shared__ f4 s_part[NW][NT * MT][64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ln = lane & 15, g = lane >> 4;
+  static_assert(!HALF || (MT == 1 && !GLU), "half tiles: at most eight rows, plain outputs");
+  constexpr int kOut = HALF ? 8 : 16;   // outputs per tile
   const uint16_t *wp[NT], *xp[MT];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
     const int64_t tile = imin64(static_cast<int64_t>(blockIdx.x) * NT + nt, a.tiles - 1);   // the last again, unused
-    const int64_t wrow = GLU ? (ln < 8 ? 8 * tile + ln : a.hidden + 8 * tile + ln - 8) : 16 * tile + ln;
+    const int64_t wrow = GLU ? (ln < 8 ? 8 * tile + ln : a.hidden + 8 * tile + ln - 8) : kOut * tile + ln % kOut;
     wp[nt] = a.w + wrow * a.w_stride + 8 * g;
   }
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
-    xp[mt] = a.x + static_cast<int64_t>(min(16 * mt + ln, a.rows - 1)) * a.x_stride + 8 * g;
-  const int per = (a.ksteps + NW - 1) / NW;
-  const int s0 = wave * per, s1 = min(s0 + per, a.ksteps);
+    xp[mt] = a.x + static_cast<int64_t>(min(16 * mt + ln % kOut, a.rows - 1)) * a.x_stride + 8 * g;
+  constexpr int kParts = HALF ? 2 * NW : NW;
+  const int per = (a.ksteps + kParts - 1) / kParts;
+  const int s0 = (HALF ? 2 * wave + ln / 8 : wave) * per, s1 = min(s0 + per, a.ksteps);
   f4 acc[NT][MT];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = f4{0.f, 0.f, 0.f, 0.f};
-  for (int s = s0; s < s1; s += kRlBatch) {
+  // (HALF: the bounds differ between the lanes' halves, the trip count is the
+  // same; loads past a part's end are inside the row and replaced by zeros.)
+  for (int s = s0; HALF ? s < s0 + per : s < s1; s += kRlBatch) {
     u4 wr[NT][kRlBatch], xr[MT][kRlBatch];
 #pragma unroll
     for (int i = 0; i < kRlBatch; ++i) {
-      const int at = 32 * min(s + i, s1 - 1);   // past the wave's last step: the last again, unused
+      const int at = 32 * min(s + i, (HALF ? a.ksteps : s1) - 1);   // past the wave's last step: the last again, unused
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) wr[nt][i] = *reinterpret_cast<const u4 *>(wp[nt] + at);
 #pragma unroll
@@ -85,7 +99,16 @@ __global__ __launch_bounds__(NW * 64) void row_linear_kernel(RowLinearArgs a) {
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < kRlBatch; ++i) {
-      if (s + i >= s1) break;   // wave-uniform
+      if constexpr (HALF) {
+        if (s + i >= s0 + per) break;   // wave-uniform (s - s0 is)
+        if (s + i >= s1) {
+          xr[0][i] = u4{0, 0, 0, 0};
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) wr[nt][i] = u4{0, 0, 0, 0};
+        }
+      } else {
+        if (s + i >= s1) break;   // wave-uniform
+      }
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
@@ -107,7 +130,15 @@ __global__ __launch_bounds__(NW * 64) void row_linear_kernel(RowLinearArgs a) {
   const int row = 16 * (wave % MT) + ln;
   const int64_t tile = static_cast<int64_t>(blockIdx.x) * NT + wave / MT;
   if (tile >= a.tiles) return;
-  if constexpr (GLU) {
+  if constexpr (HALF) {
+    // outputs 8 tile + (4 g + i) % 8: lanes ln < 8, g < 2 hold the sums over the
+    // first parts of k, lanes ln + 8, g + 2 the same outputs' over the second
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sum[i] += lane_xor32(dpp_rotate<0x128>(sum[i]));
+    if (g < 2 && row < a.rows)
+      *reinterpret_cast<u2 *>(a.y + row * a.y_stride + 8 * tile + 4 * g) =
+          u2{pack_bf16x2(sum[0], sum[1]), pack_bf16x2(sum[2], sum[3])};
+  } else if constexpr (GLU) {
     // rows 4 g + i of the tile: g < 2 gate columns, g + 2 their up columns
     f4 up;
 #pragma unroll
@@ -123,9 +154,9 @@ __global__ __launch_bounds__(NW * 64) void row_linear_kernel(RowLinearArgs a) {
   }
 }
 
-template <int NW, int NT, int MT, bool GLU, bool CAP4>
+template <int NW, int NT, int MT, bool GLU, bool CAP4, bool HALF = false>
 int launch(const RowLinearArgs &a, hipStream_t st) {
-  hipLaunchKernelGGL((row_linear_kernel<NW, NT, MT, GLU, CAP4>), dim3(static_cast<unsigned>((a.tiles + NT - 1) / NT)),
+  hipLaunchKernelGGL((row_linear_kernel<NW, NT, MT, GLU, CAP4, HALF>), dim3(static_cast<unsigned>((a.tiles + NT - 1) / NT)),
                      dim3(NW * 64), 0, st, a);
   return check_launch(GLU ? "row_linear_situ_glu" : "row_linear");
 }
@@ -144,6 +175,16 @@ int dispatch_tiles(const RowLinearArgs &a, hipStream_t st) {
 template <bool GLU, bool CAP4>
 int dispatch(const RowLinearArgs &a, hipStream_t st) {
   const int need = (a.ksteps + kRlBatch - 1) / kRlBatch;
+  // Half tiles while they are at most one per CU; past that whole tiles fill
+  // the chip.  k over 8 parts up to 2,048, over 16 beyond.
+  if constexpr (!GLU) {
+    if (a.rows <= 8 && a.tiles <= 128) {
+      RowLinearArgs half = a;
+      half.tiles = 2 * a.tiles;
+      if (need <= 8) return launch<4, 1, 1, false, false, true>(half, st);
+      return launch<8, 1, 1, false, false, true>(half, st);
+    }
+  }
   if (a.rows <= 16) {
     if (need <= 4) return dispatch_tiles<4, 1, GLU, CAP4>(a, st);
     if (need <= 8) return dispatch_tiles<8, 1, GLU, CAP4>(a, st);

@@ -254,6 +254,27 @@ int sophia_kda_decode_conv_step(const void *x_q, const void *x_k, const void *x_
                                 void *stream);
 
 /*
+ * sophia_kda_decode_conv_step and what a mixer runs around it, in one launch, all
+ * in bf16 with the gate in the kernel (flags hold SOPHIA_KDA_GATE_IN_KERNEL):
+ *   decay_weight  : NULL, or [H * 128, 128] contiguous: g is then the low-rank row
+ *                   [batch, 128] (row stride a multiple of 8; both 16-byte
+ *                   aligned) and the decay logits g . decay_weight^T, rounded to
+ *                   bf16 (decay_up, attention.py:402-404).  Every row reads the
+ *                   weight: meant for few rows.
+ *   out_gate      : [batch, H, 128] logits; o = RMSNorm(o; norm_weight [128] fp32,
+ *                   norm_eps) sigmoid(out_gate) per head, as
+ *                   sophia_gated_head_norm gives it for the step's bf16 output.
+ */
+int sophia_kda_decode_mixer_step(const void *x_q, const void *x_k, const void *x_v, int64_t x_row_stride,
+                                 const float *conv_weight, float *conv_state, const void *g,
+                                 int64_t g_row_stride, const void *decay_weight, const void *beta,
+                                 int64_t beta_row_stride, const float *A_log, const float *dt_bias, float scale,
+                                 float lower_bound, unsigned flags, float *state, int n_state_slots,
+                                 const int32_t *state_slots, int read_state, const void *out_gate,
+                                 int64_t out_gate_row_stride, const float *norm_weight, float norm_eps, int batch,
+                                 int num_heads, int head_dim, void *o, int64_t o_row_stride, void *stream);
+
+/*
  * The prefill of a KDA layer with its ShortConv: the causal conv + SiLU of the
  * q, k and v channels over each sequence (CausalDepthwiseConv1d.forward,
  * attention.py:32-60, as SophiaKDA._short_convolution drives it, 226-258)

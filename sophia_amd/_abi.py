@@ -57,6 +57,9 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "sophia_kda_decode_conv_step": (_i32, [_vp, _vp, _vp, _i64, _i32, _vp, _vp, _i32, _vp, _i64, _i32,
                                            _vp, _i64, _i32, _vp, _vp, _f32, _f32, _u32, _vp, _i32,
                                            _vp, _i32, _i32, _i32, _i32, _vp, _i64, _vp]),
+    "sophia_kda_decode_mixer_step": (_i32, [_vp, _vp, _vp, _i64, _vp, _vp, _vp, _i64, _vp, _vp, _i64, _vp, _vp,
+                                            _f32, _f32, _u32, _vp, _i32, _vp, _i32, _vp, _i64, _vp, _f32, _i32, _i32,
+                                            _i32, _vp, _i64, _vp]),
     "sophia_kda_conv_chunk_fwd": (_i32, [_vp, _vp, _vp, _i64, _i32, _vp, _vp, _i32, _i32, _vp, _i64, _i32,
                                          _vp, _i64, _i32, _vp, _vp, _f32, _f32, _u32, _vp, _vp, _i32,
                                          _i64, _i32, _i32, _vp, _vp, _i32, _vp, _vp, _i64, _vp, _sz, _vp]),

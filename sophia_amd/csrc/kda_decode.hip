@@ -26,6 +26,17 @@
 // history back: a decode layer is then one launch.  It keeps one work-group
 // per (sequence, head) (128 value columns): with two, both would read a
 // channel's history while one of them rewrites it.
+//
+// Its DECAY form also makes the decay logits (decay_up, attention.py:402-404):
+// g is then the low-rank row [128], and the work-group forms its head's 128
+// logits on MFMAs from the head's 32 KB of the weight, rounded to bf16 as a
+// launch of its own writes them.  Every row reads that weight (from L2), so it
+// is for few rows.  Its GATED form ends with the head's RMSNorm and output gate
+// (attention.py:411-420), o rounded to bf16 before them as it is between two
+// launches: the work-group holds the whole head, and the barrier that its sum
+// of squares needs is there already.
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace sophia {
@@ -38,11 +49,19 @@ constexpr int kDecodeCols = 64;   // value columns per work-group
 // Conv history samples per channel (kernel size 4).
 constexpr int kConvHist = 3;
 
+// The GATED epilogue: o = RMSNorm(o; w, eps) sigmoid(gate), gate rows like o's.
+struct GatedOut {
+  const uint16_t *gate;
+  int64_t gate_stride;
+  const float *norm_w;   // [128]
+  float eps;
+};
+
 // Dtypes and the gate switch are template parameters so that the load batch
 // below has no branches: the wave then waits for the token inputs alone
 // (issued first) before the prologue, while the state is still in flight.
 
-template <int QKV_DT, int G_DT, int B_DT, bool GATE, int NC, bool CONV>
+template <int QKV_DT, int G_DT, int B_DT, bool GATE, int NC, bool CONV, bool DECAY = false, bool GATED = false>
 __global__ __launch_bounds__(kThreads) void kda_decode_kernel(
     const void *__restrict__ q, const void *__restrict__ k, const void *__restrict__ v,
     int64_t qkv_stride, const void *__restrict__ g, int64_t g_stride,
@@ -50,7 +69,8 @@ __global__ __launch_bounds__(kThreads) void kda_decode_kernel(
     const float *__restrict__ A_log, const float *__restrict__ dt_bias, float scale, float lb,
     unsigned flags, float *__restrict__ state, int n_slots, const int32_t *__restrict__ slots,
     int read_state, int num_heads, void *__restrict__ o, int64_t o_stride,
-    const float *__restrict__ conv_w, float *__restrict__ conv_state) {
+    const float *__restrict__ conv_w, float *__restrict__ conv_state, const uint16_t *__restrict__ decay_w,
+    GatedOut out) {
   constexpr int CG = NC / 4;           // column groups of 4 columns
   constexpr int RG = kThreads / CG;    // row groups
   constexpr int RPT = kD / RG;         // rows per thread
@@ -67,6 +87,8 @@ __global__ __launch_bounds__(kThreads) void kda_decode_kernel(
   __shared__ float s_red[4][3];
   __shared__ float s_p[4][NC], s_r[4][NC];
   __shared__ float s_u[NC];
+  __shared__ float s_ss[2];
+  __shared__ __align__(8) uint16_t s_z[DECAY ? kD : 4];
 
   const int slot = slots ? slots[b] : b;
   if (slot < 0 || slot >= n_slots) {  // no cache slot: output 0, no state touched
@@ -86,12 +108,36 @@ __global__ __launch_bounds__(kThreads) void kda_decode_kernel(
   const uint32_t raw_q = load_raw(q, row + c, QKV_DT);
   const uint32_t raw_k = load_raw(k, row + c, QKV_DT);
   const uint32_t raw_v = load_raw(v, row + c, QKV_DT);
-  const uint32_t raw_g = load_raw(g, grow + c, G_DT);
+  static_assert(!DECAY || (CONV && G_DT == SOPHIA_DTYPE_BF16), "");
+  constexpr int kSteps = kD / 32;   // MFMA k-steps of the low rank
+  uint32_t raw_g = 0;
+  u4 dw[DECAY ? 2 : 1][kSteps], dx[kSteps];
+  if constexpr (DECAY) {
+    // A = 2 x 16 weight rows of this wavefront's 32 channels, B = the low-rank
+    // row in all 16 columns
+    const uint16_t *dr = static_cast<const uint16_t *>(g) + static_cast<int64_t>(b) * g_stride + 8 * (lane >> 4);
+    const uint16_t *wr = decay_w + (static_cast<int64_t>(h) * kD + 32 * wave + (lane & 15)) * kD + 8 * (lane >> 4);
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+      dx[s] = *reinterpret_cast<const u4 *>(dr + 32 * s);
+#pragma unroll
+      for (int m = 0; m < 2; ++m) dw[m][s] = *reinterpret_cast<const u4 *>(wr + 16 * kD * m + 32 * s);
+    }
+  } else {
+    raw_g = load_raw(g, grow + c, G_DT);
+  }
   const uint32_t raw_b = load_raw(beta, static_cast<int64_t>(b) * beta_stride + h, B_DT);
   float alog = 0.f, bias = 0.f;
   if constexpr (GATE) {
     bias = dt_bias[h * kD + c];
     alog = A_log[h];
+  }
+  static_assert(!GATED || (CONV && NC == kD && QKV_DT == SOPHIA_DTYPE_BF16), "whole bf16 heads");
+  uint32_t raw_og = 0;
+  float norm_w = 0.f;
+  if constexpr (GATED) {
+    raw_og = out.gate[static_cast<int64_t>(b) * out.gate_stride + static_cast<int64_t>(h) * kD + c];
+    norm_w = out.norm_w[c];
   }
   // Conv taps and history of channel c of q, k and v: channels
   // h*128 + c, inner + h*128 + c and 2*inner + h*128 + c of the fused
@@ -145,6 +191,21 @@ __global__ __launch_bounds__(kThreads) void kda_decode_kernel(
     xq = conv1(wq, hq, xq);
     xk = conv1(wk, hk, xk);
     xv = conv1(wv, hv, xv);
+  }
+  if constexpr (DECAY) {
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      f4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < kSteps; ++s)
+        z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, dw[m][s]), __builtin_bit_cast(bf8, dx[s]),
+                                                    z, 0, 0, 0);
+      if ((lane & 15) == 0)   // all columns are alike; rows 4 (lane / 16) + i
+        *reinterpret_cast<u2 *>(&s_z[32 * wave + 16 * m + 4 * (lane >> 4)]) =
+            u2{pack_bf16x2(z[0], z[1]), pack_bf16x2(z[2], z[3])};
+    }
+    lds_barrier();
+    raw_g = s_z[c];
   }
   const float qv = own ? xq : 0.f;
   const float kv = own ? xk : 0.f;
@@ -230,15 +291,31 @@ __global__ __launch_bounds__(kThreads) void kda_decode_kernel(
     }
   }
   lds_barrier();
+  const int64_t o_at = static_cast<int64_t>(b) * o_stride + static_cast<int64_t>(h) * kD + col0 + t;
+  float oj = 0.f;
   if (t < NC) {
     const float pj = s_p[0][t] + s_p[1][t] + s_p[2][t] + s_p[3][t];
     const float rj = s_r[0][t] + s_r[1][t] + s_r[2][t] + s_r[3][t];
     const float u = bt * (s_v[col0 + t] - pj);
     s_u[t] = u;
-    store_elem(o, static_cast<int64_t>(b) * o_stride + static_cast<int64_t>(h) * kD + col0 + t, QKV_DT,
-               rj + qk * u);
+    oj = rj + qk * u;
+    if constexpr (GATED) {
+      oj = as_dtype(oj, QKV_DT);
+      const float ss = wave_sum_dpp(oj * oj);
+      if (lane == 0) s_ss[wave] = ss;
+    } else {
+      store_elem(o, o_at, QKV_DT, oj);
+    }
   }
   lds_barrier();
+  if constexpr (GATED) {
+    if (own) {
+      const float r = rsqrtf((s_ss[0] + s_ss[1]) / static_cast<float>(kD) + out.eps);
+      oj *= r * norm_w;
+      oj *= __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896341f * raw_to_f32(raw_og, QKV_DT)));
+      store_elem(o, o_at, QKV_DT, oj);
+    }
+  }
   const f4 u4v = *reinterpret_cast<const f4 *>(&s_u[4 * cg]);
 #pragma unroll
   for (int r = 0; r < RPT; ++r) {
@@ -289,7 +366,7 @@ extern "C" int sophia_kda_decode_step(const void *q, const void *k, const void *
     hipLaunchKernelGGL((kda_decode_kernel<QD, GD, BD, GT, kDecodeCols, false>), grid, dim3(kThreads), 0, st, q, \
                        k, v, qkv_row_stride, g, g_row_stride, beta, beta_row_stride, A_log, dt_bias,   \
                        scale, lower_bound, flags, state, n_state_slots, state_slots, read_state, \
-                       num_heads, o, o_row_stride, nullptr, nullptr);                            \
+                       num_heads, o, o_row_stride, nullptr, nullptr, nullptr, GatedOut{});                            \
     break;
   constexpr int F = SOPHIA_DTYPE_F32, B = SOPHIA_DTYPE_BF16;
   switch (key) {
@@ -354,7 +431,7 @@ extern "C" int sophia_kda_decode_conv_step(const void *x_q, const void *x_k, con
     hipLaunchKernelGGL((kda_decode_kernel<QD, GD, BD, GT, kD, true>), grid, dim3(kThreads), 0, st, x_q, x_k, \
                        x_v, x_row_stride, g, g_row_stride, beta, beta_row_stride, A_log, dt_bias, \
                        scale, lower_bound, flags, state, n_state_slots, state_slots, read_state, \
-                       num_heads, o, o_row_stride, conv_weight, conv_state);                     \
+                       num_heads, o, o_row_stride, conv_weight, conv_state, nullptr, GatedOut{});                     \
     break;
   constexpr int F = SOPHIA_DTYPE_F32, B = SOPHIA_DTYPE_BF16;
   switch (key) {
@@ -377,4 +454,43 @@ extern "C" int sophia_kda_decode_conv_step(const void *x_q, const void *x_k, con
   }
 #undef SOPHIA_DECODE_CONV_CASE
   return check_launch("kda_decode_conv_step");
+}
+
+extern "C" int sophia_kda_decode_mixer_step(
+    const void *x_q, const void *x_k, const void *x_v, int64_t x_row_stride, const float *conv_weight,
+    float *conv_state, const void *g, int64_t g_row_stride, const void *decay_weight, const void *beta,
+    int64_t beta_row_stride, const float *A_log, const float *dt_bias, float scale, float lower_bound,
+    unsigned flags, float *state, int n_state_slots, const int32_t *state_slots, int read_state,
+    const void *out_gate, int64_t out_gate_row_stride, const float *norm_weight, float norm_eps, int batch,
+    int num_heads, int head_dim, void *o, int64_t o_row_stride, void *stream) {
+  SOPHIA_REQUIRE(head_dim == kD, "kda_decode_mixer_step: head_dim must be 128 (got %d)", head_dim);
+  SOPHIA_REQUIRE(batch > 0 && batch <= 65535 && num_heads > 0,
+                 "kda_decode_mixer_step: batch must be 1..65535 and num_heads > 0");
+  SOPHIA_REQUIRE(x_q && x_k && x_v && g && beta && state && o && conv_weight && conv_state && A_log && dt_bias &&
+                     out_gate && norm_weight,
+                 "kda_decode_mixer_step: NULL pointer");
+  SOPHIA_REQUIRE(flags & SOPHIA_KDA_GATE_IN_KERNEL, "kda_decode_mixer_step: the gate runs in the kernel");
+  const int64_t inner = static_cast<int64_t>(num_heads) * kD;
+  SOPHIA_REQUIRE(x_row_stride >= inner && g_row_stride >= (decay_weight ? kD : inner) &&
+                     beta_row_stride >= num_heads && out_gate_row_stride >= inner && o_row_stride >= inner,
+                 "kda_decode_mixer_step: row stride smaller than a row");
+  SOPHIA_REQUIRE(((uintptr_t)state % 16) == 0 && ((uintptr_t)conv_weight % 16) == 0,
+                 "kda_decode_mixer_step: state and conv_weight must be 16-byte aligned");
+  SOPHIA_REQUIRE(!decay_weight || (((uintptr_t)decay_weight % 16) == 0 && ((uintptr_t)g % 16) == 0 && g_row_stride % 8 == 0),
+                 "kda_decode_mixer_step: decay_weight and the low-rank rows must be 16-byte aligned");
+  SOPHIA_REQUIRE(n_state_slots >= 0, "kda_decode_mixer_step: n_state_slots must be >= 0");
+  constexpr int B = SOPHIA_DTYPE_BF16;
+  const GatedOut out{static_cast<const uint16_t *>(out_gate), out_gate_row_stride, norm_weight, norm_eps};
+  const auto run = [&](auto decay) {
+    hipLaunchKernelGGL((kda_decode_kernel<B, B, B, true, kD, true, decay.value, true>), dim3(num_heads, batch),
+                       dim3(kThreads), 0, static_cast<hipStream_t>(stream), x_q, x_k, x_v, x_row_stride, g,
+                       g_row_stride, beta, beta_row_stride, A_log, dt_bias, scale, lower_bound, flags, state,
+                       n_state_slots, state_slots, read_state, num_heads, o, o_row_stride, conv_weight, conv_state,
+                       static_cast<const uint16_t *>(decay_weight), out);
+  };
+  if (decay_weight)
+    run(std::true_type{});
+  else
+    run(std::false_type{});
+  return check_launch("kda_decode_mixer_step");
 }

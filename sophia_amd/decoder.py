@@ -34,7 +34,7 @@ from torch import nn
 
 from .config import ModelArgs
 from . import ops
-from .kda import RMSNorm, RuntimeLinear, SophiaKDA, _require_gpu
+from .kda import RMSNorm, RuntimeLinear, SophiaKDA, _require_gpu, plain_linear
 from .state import LayerCacheSnapshot, RuntimeCacheSnapshot
 
 
@@ -388,8 +388,7 @@ class FeedForward(nn.Module):
         # are one launch.  A projection with hooks or in another module's place
         # is called as a module.
         proj = self.gate_up_proj
-        if type(proj) is RuntimeLinear and proj.bias is None and not (
-                proj._forward_hooks or proj._forward_pre_hooks or proj._backward_hooks or proj._backward_pre_hooks):
+        if plain_linear(proj):
             hidden = ops.linear_situ_glu(x, proj.weight, self.gate_softcap, self.up_softcap)
         else:
             hidden = ops.situ_glu(proj(x), self.gate_softcap, self.up_softcap)

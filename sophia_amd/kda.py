@@ -63,6 +63,13 @@ class RuntimeLinear(nn.Module):
         return ops.linear(x, self.weight, self.bias)
 
 
+def plain_linear(m: nn.Module) -> bool:
+    """Whether ``m`` is a RuntimeLinear that another launch may take the place
+    of: no subclass or replacement, no bias, no hooks."""
+    return type(m) is RuntimeLinear and m.bias is None and not (
+        m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+
+
 class RMSNorm(nn.Module):
     """ops.py:49-64: functional.rms_norm over the last dim, fp32 weight."""
 
@@ -534,6 +541,16 @@ class SophiaKDA(nn.Module):
         if n_decode > 0 and not fused_decode:
             ops.short_conv_step(qkv[n_prefill:], conv_w, conv_state, state_slots=decode_slots,
                                 read_history=True, out=conv_out[n_prefill:], weight_rounded=True)
+        if n_prefill == 0 and fused_decode and ops.decode_mixer_takes(
+                qkv, dd, beta_logits, gate_logits, self.decay_up.weight, self.output_norm.weight):
+            # Decode rows alone: the step's launch also ends with the output norm
+            # and gate and, for few rows, begins with decay_up.
+            own = plain_linear(self.decay_up) and ops.decay_in_step(dd, self.decay_up.weight)
+            return self.o_proj(ops.kda_decode_mixer_step(
+                qkv, conv_w, conv_state, dd if own else self.decay_up(dd).view(n, h, d), beta_logits,
+                self.recurrent_state, gate_logits, self.output_norm.weight, A_log=self.A_log, dt_bias=self.dt_bias,
+                norm_eps=float(self.output_norm.eps), decay_weight=self.decay_up.weight if own else None,
+                lower_bound=self.lower_bound, state_slots=decode_slots))
         decay = self.decay_up(dd).view(n, h, d)
         o = torch.empty((n, h, d), dtype=x2.dtype, device=x2.device)
         gate_args = dict(A_log=self.A_log, dt_bias=self.dt_bias, lower_bound=self.lower_bound)

@@ -594,6 +594,83 @@ def kda_decode_conv_step(x_qkv: torch.Tensor, conv_weight: torch.Tensor, conv_st
     return o
 
 
+def decode_mixer_takes(x_qkv, low, beta, out_gate, weight, norm_weight) -> bool:
+    """Whether ``kda_decode_mixer_step`` may take the place of the launches it
+    stands for: plain values, bf16 rows, an fp32 norm weight of a head of 128."""
+    bf = torch.bfloat16
+    return (_values_only(x_qkv, low, beta, out_gate, weight, norm_weight)
+            and x_qkv.dtype == bf and low.dtype == bf and beta.dtype == bf and out_gate.dtype == bf
+            and norm_weight.dtype == torch.float32 and norm_weight.is_contiguous() and norm_weight.numel() == HEAD_DIM
+            and out_gate.stride(-1) == 1 and all(t.device == x_qkv.device for t in (low, weight, norm_weight)))
+
+
+def decay_in_step(low: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether the decode step forms its decay logits low . weight^T itself: low
+    rank 128, aligned rows, and few of them (each reads the whole weight)."""
+    return (low.size(0) <= ROW_LINEAR_MAX and weight.dtype == torch.bfloat16 and weight.is_contiguous()
+            and weight.size(1) == HEAD_DIM and low.stride(1) == 1 and (low.size(0) <= 1 or low.stride(0) % 8 == 0)
+            and low.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
+
+
+def kda_decode_mixer_step(x_qkv: torch.Tensor, conv_weight: torch.Tensor, conv_state: torch.Tensor,
+                          g: torch.Tensor, beta: torch.Tensor, state: torch.Tensor, out_gate: torch.Tensor,
+                          norm_weight: torch.Tensor, *, A_log, dt_bias, norm_eps: float,
+                          decay_weight: torch.Tensor | None = None, scale: float | None = None,
+                          lower_bound: float = -5.0, state_slots: torch.Tensor | None = None) -> torch.Tensor:
+    """``kda_decode_conv_step`` of bf16 rows with ``gated_head_norm`` of its
+    output (out_gate [B, H * 128] logits) and, with ``decay_weight`` [H * 128,
+    128], the product of the low-rank rows g [B, 128] with it, in one launch
+    (sophia_kda_decode_mixer_step).  Returns [B, H * 128] bf16."""
+    for t, name in ((x_qkv, "x_qkv"), (g, "g"), (beta, "beta"), (out_gate, "out_gate"), (conv_state, "conv_state")):
+        _gpu(t, name)
+    device = x_qkv.device
+    batch, inner = int(x_qkv.size(0)), int(x_qkv.size(1)) // 3
+    heads = inner // HEAD_DIM
+    xs = _rows(x_qkv, "x_qkv", 3 * heads * HEAD_DIM)
+    if decay_weight is not None:
+        gs = _rows(g, "g", HEAD_DIM)
+        if tuple(decay_weight.shape) != (inner, HEAD_DIM) or not decay_in_step(g, decay_weight):
+            raise RuntimeError(f"decay_weight must be contiguous bf16 [{inner}, 128], g at most {ROW_LINEAR_MAX} "
+                               "rows of 128, both 16-byte aligned")
+    else:
+        gs = _heads_rows(g, "g", heads, HEAD_DIM)
+    bs = _rows(beta, "beta", heads)
+    os_ = _rows(out_gate, "out_gate", inner)
+    for t, name in ((g, "g"), (beta, "beta"), (out_gate, "out_gate")):
+        _nrows(t, name, batch)
+    weights = [t for t in (conv_weight, norm_weight, decay_weight) if t is not None]
+    if any(t.device != device for t in [g, beta, out_gate, conv_state, *weights]):
+        raise RuntimeError(f"every operand must be on {device}")
+    if any(t.dtype != torch.bfloat16 for t in (x_qkv, g, beta, out_gate)):
+        raise RuntimeError("x_qkv, g, beta and out_gate must be bf16")
+    if (conv_weight.dtype != torch.float32 or not conv_weight.is_contiguous()
+            or tuple(conv_weight.shape) != (3 * inner, 4)):
+        raise RuntimeError(f"conv_weight must be contiguous fp32 [{3 * inner}, 4] on {device}")
+    if (conv_state.dtype != torch.float32 or not conv_state.is_contiguous()
+            or tuple(conv_state.shape[1:]) != (3 * inner, 3)):
+        raise RuntimeError(f"conv_state must be contiguous fp32 [slots, {3 * inner}, 3]")
+    if norm_weight.dtype != torch.float32 or not norm_weight.is_contiguous() or norm_weight.numel() != HEAD_DIM:
+        raise RuntimeError("norm_weight must be contiguous fp32 [128]")
+    _state(state, "state", heads, device)
+    if int(conv_state.size(0)) != int(state.size(0)):
+        raise RuntimeError("conv_state and state must have the same number of slots")
+    slots = _int32(state_slots, "state_slots", device)
+    _slot_count(slots, batch)
+    if slots is None and int(state.size(0)) < batch:
+        raise RuntimeError("state has fewer slots than the batch")
+    a_log, dtb = _gate_params(True, A_log, dt_bias, heads, device)
+    o = torch.empty((batch, inner), dtype=x_qkv.dtype, device=device)
+    base, esz = x_qkv.data_ptr(), x_qkv.element_size()
+    rc = nat.lib().sophia_kda_decode_mixer_step(
+        base, base + inner * esz, base + 2 * inner * esz, xs, nat.ptr(conv_weight), nat.ptr(conv_state), nat.ptr(g),
+        gs, nat.ptr(decay_weight), nat.ptr(beta), bs, nat.ptr(a_log), nat.ptr(dtb),
+        float(HEAD_DIM ** -0.5 if scale is None else scale), float(lower_bound), _flags(True, True, True),
+        nat.ptr(state), int(state.size(0)), nat.ptr(slots), 1, nat.ptr(out_gate), os_, nat.ptr(norm_weight),
+        float(norm_eps), batch, heads, HEAD_DIM, nat.ptr(o), inner, nat.stream_handle(device))
+    nat.check(rc, "sophia_kda_decode_mixer_step")
+    return o
+
+
 # -------------------------------------------- flash-linear-attention signatures
 def _detached(t):
     """Gate parameters enter the kernels as values (the forward-only kernels
@@ -847,7 +924,7 @@ def _values_only(*tensors) -> bool:
     """True when a call on ``tensors`` computes plain values only: not traced,
     transformed (functorch, forward-mode), under a dispatch or function mode or
     autocast, and with no gradient to record."""
-    if torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda"):
+    if torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing():
         return False
     if (torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
             or torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0):

@@ -571,3 +571,48 @@ def test_decode_conv_step_matches_separate_launches_and_oracle(dtype, batch, hea
                                       dt_bias=dtb, dtype=np.float64)
     assert _rel(_np(o_b)[sample], o_ref) < REL_TOL
     assert _rel(_np(st_b)[slots[sample]], s_ref) < REL_TOL
+
+
+@pytest.mark.parametrize("batch,heads,own", [(1, 1, True), (9, 3, True), (32, 16, True), (9, 3, False), (50, 16, False)])
+def test_decode_mixer_step_equals_separate_launches(batch, heads, own):
+    """sophia_kda_decode_mixer_step against decay_up's product, kda_decode_conv_step
+    and gated_head_norm: states, histories and outputs with the decay given equal
+    bit for bit but for the order of the norm's sum of squares (one bf16 rounding
+    step, 2^-7 of a value); with the product inside, the decay logits may round the
+    other way where their fp32 sums differ in order (1e-2, as the conv step's bf16
+    bar).  x, gate, low rank and beta are slices of one wide row, one slot is out of
+    range (output 0)."""
+    from sophia_amd import ops
+    dev = _dev()
+    gen = torch.Generator().manual_seed(batch)
+    inner, slots_n = heads * 128, batch + 3
+    rnd = lambda *s: torch.randn(*s, generator=gen)  # noqa: E731
+    wide = rnd(batch, 4 * inner + 128 + 8 * ((heads + 7) // 8)).to(torch.bfloat16).to(dev)
+    x, gate, low = wide[:, :3 * inner], wide[:, 3 * inner:4 * inner], wide[:, 4 * inner:4 * inner + 128]
+    beta = wide[:, 4 * inner + 128:4 * inner + 128 + heads]
+    up = (rnd(inner, 128) * 0.05).to(torch.bfloat16).to(dev)
+    taps = (rnd(3 * inner, 4) * 0.3).to(torch.bfloat16).float().to(dev)
+    nw = (1 + 0.1 * rnd(128)).to(dev)
+    kw = dict(A_log=(rnd(heads) * 0.3).to(dev), dt_bias=rnd(inner).to(dev), lower_bound=-5.0,
+              state_slots=torch.randperm(slots_n, generator=gen)[:batch].to(torch.int32).to(dev))
+    if batch > 1:
+        kw["state_slots"][-1] = slots_n + 4
+    s0, c0 = (rnd(slots_n, heads, 128, 128) * 0.1).to(dev), rnd(slots_n, 3 * inner, 3).to(dev)
+    z = (low.float() @ up.float().t()).to(torch.bfloat16).view(batch, heads, 128)
+    sa, ca, sb, cb = s0.clone(), c0.clone(), s0.clone(), c0.clone()
+    o = ops.kda_decode_conv_step(x, taps, ca, z, beta, sa, **kw)
+    ref = ops.gated_head_norm(o, gate, heads, 128, norm_weight=nw, eps=1e-5)
+    y = ops.kda_decode_mixer_step(x, taps, cb, low if own else z, beta, sb, gate, nw, norm_eps=1e-5,
+                                  decay_weight=up if own else None, **kw)
+    assert torch.equal(ca, cb) and y.shape == (batch, inner)
+    if own:
+        assert _rel(_np(y.float()), _np(ref.float())) < 1e-2 and _rel(_np(sb), _np(sa)) < 1e-2
+    else:
+        assert torch.equal(sa, sb)
+        assert bool(((y.float() - ref.float()).abs() <= 2.0 ** -7 * ref.float().abs()).all())
+    if batch > 1:
+        assert bool((y[-1] == 0).all())
+    with pytest.raises(RuntimeError):
+        ops.kda_decode_mixer_step(x, taps, cb, low.float(), beta, sb, gate, nw, norm_eps=1e-5, decay_weight=up, **kw)
+    with pytest.raises(RuntimeError):
+        ops.kda_decode_mixer_step(x, taps, cb, low, beta, sb, gate, nw[:64], norm_eps=1e-5, decay_weight=up, **kw)

@@ -3,7 +3,7 @@
 //
 // Bound by reading the weight once.  One work-group per 16 outputs: its
 // wavefronts split k, each lane loads its share of the 16 weight rows in
-// 16-byte pieces, eight MFMA k-steps at a time before any is used, so that all
+// 16-byte pieces, up to eight MFMA k-steps before any is used, so that all
 // of a work-group's weight bytes (48 KB at k = 1,536) are in flight at once, and the
 // partial 16 x 16 tiles are summed over the wavefronts in order through LDS.
 // A library GEMM of these shapes walks k in LDS tiles.  us per call at 8 rows,
@@ -21,13 +21,16 @@
 // ml/runtime/model) is formed on the fp32 sums of one tile: the projection is
 // neither rounded nor written.
 //
-// For at most eight rows half of a tile's columns would be empty, and 1,536
-// outputs are 96 tiles on 256 CUs.  The half-tile form puts eight outputs in a
-// work-group: A holds their weights over two parts of k (rows 0-7 and 8-15), B
-// the rows of x over the same two parts, and of the product the two diagonal
-// quadrants are the sums over the parts.  Twice the work-groups, the same bytes
-// per load instruction: under the profiler 1,536 x 3,968 9.0 -> 7.3 us, 1,536 x
-// 2,048 5.3 -> 4.8.
+// For at most eight rows half of a tile's columns would be empty.  The half-tile
+// form puts eight outputs in a tile: A holds their weights at two consecutive
+// k-steps (rows 0-7 and 8-15), B the rows of x at the same two, and of the
+// product the two diagonal quadrants are the sums over the even and the odd
+// steps.  A load then takes whole 128-byte lines of eight weight rows instead of
+// half lines of sixteen, x is loaded half as often, and there are twice the
+// tiles to spread over the chip (1,536 outputs are 96 tiles of 16 on 256 CUs).
+// us per call, weights from HBM, whole tiles or library -> half: 1,536 x 3,968 7.9 ->
+// 6.0, 7,936 x 1,536 with its activation 9.2 -> 7.6, 8,384 x 1,536 12.1 -> 7.5, 2,048 x 384
+// 3.8 -> 2.4.
 #include "common.hpp"
 #include "situ.hpp"
 
@@ -37,7 +40,7 @@ namespace sophia {
 namespace {
 
 constexpr int kRlRows = 32;    // most rows of x
-constexpr int kRlBatch = 8;    // k-steps whose loads are issued together
+constexpr int kHlBatch = 8;    // head_linear: k-steps whose loads are issued together
 
 struct RowLinearArgs {
   const uint16_t *x;
@@ -55,41 +58,72 @@ struct RowLinearArgs {
 
 __device__ __forceinline__ bf8 as_bf8(u4 w) { return __builtin_bit_cast(bf8, w); }
 
-// NW wavefronts, NT tiles of outputs (sharing the loads of x), MT tiles of 16
-// rows of x.  HALF: eight outputs per tile for at most eight rows, k split over
-// 2 NW parts, a lane's part by its half of the 16.
+// Sums of a tile's four columns, the partial tiles of the wavefronts, to y.
 template <int NW, int NT, int MT, bool GLU, bool CAP4, bool HALF>
+__device__ __forceinline__ void store_tile(const RowLinearArgs &a, const f4 (&part)[NW][NT * MT][64], int nt, int mt,
+                                           int lane) {
+  const int ln = lane & 15, g = lane >> 4;
+  const int64_t tile = static_cast<int64_t>(blockIdx.x) * NT + nt;
+  if (tile >= a.tiles) return;   // wave-uniform
+  f4 sum = part[0][nt * MT + mt][lane];   // weight rows 4 g + i, row 16 mt + ln
+#pragma unroll
+  for (int p = 1; p < NW; ++p) sum += part[p][nt * MT + mt][lane];
+  constexpr int kRows = HALF ? 8 : 16;   // weight rows of a tile
+  if constexpr (HALF) {
+    // lanes ln < 8, g < 2 hold the even steps' sums, lanes ln + 8, g + 2 the same outputs' of the odd steps
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sum[i] += lane_xor32(dpp_rotate<0x128>(sum[i]));
+  }
+  constexpr int kGroups = kRows / 4 / (GLU ? 2 : 1);   // of four outputs
+  if constexpr (GLU) {
+    // the first half of the tile's weight rows are gate columns, the second their up columns
+    f4 up;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) up[i] = HALF ? lane_xor16(sum[i]) : lane_xor32(sum[i]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sum[i] = situ_value<CAP4>(sum[i], up[i], a.rcg, a.rcu, a.scale);
+  }
+  const int row = 16 * mt + ln;
+  if (g < kGroups && row < a.rows)
+    *reinterpret_cast<u2 *>(a.y + row * a.y_stride + 4 * (kGroups * tile + g)) =
+        u2{pack_bf16x2(sum[0], sum[1]), pack_bf16x2(sum[2], sum[3])};
+}
+
+// NW wavefronts, NT tiles of outputs (sharing the loads of x), MT tiles of 16
+// rows of x; loads of BATCH k-steps (HALF: pairs of steps) issued together.
+template <int NW, int NT, int MT, int BATCH, bool GLU, bool CAP4, bool HALF>
 __global__ __launch_bounds__(NW * 64) void row_linear_kernel(RowLinearArgs a) {
+  static_assert(!HALF || MT == 1, "half tiles are for at most eight rows");
+  constexpr int kRows = HALF ? 8 : 16;   // weight rows of a tile, rows of x
   __shared__ f4 s_part[NW][NT * MT][64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ln = lane & 15, g = lane >> 4;
-  static_assert(!HALF || (MT == 1 && !GLU), "half tiles: at most eight rows, plain outputs");
-  constexpr int kOut = HALF ? 8 : 16;   // outputs per tile
+  const int ln = lane & (kRows - 1), g = lane >> 4;
+  const int odd = HALF ? (lane >> 3) & 1 : 0;   // this lane's step of a pair
   const uint16_t *wp[NT], *xp[MT];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
     const int64_t tile = imin64(static_cast<int64_t>(blockIdx.x) * NT + nt, a.tiles - 1);   // the last again, unused
-    const int64_t wrow = GLU ? (ln < 8 ? 8 * tile + ln : a.hidden + 8 * tile + ln - 8) : kOut * tile + ln % kOut;
+    constexpr int kCols = kRows / 2;   // GLU: gate and up columns of a tile
+    const int64_t wrow = GLU ? (ln < kCols ? kCols * tile + ln : a.hidden + kCols * tile + ln - kCols) : kRows * tile + ln;
     wp[nt] = a.w + wrow * a.w_stride + 8 * g;
   }
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
-    xp[mt] = a.x + static_cast<int64_t>(min(16 * mt + ln % kOut, a.rows - 1)) * a.x_stride + 8 * g;
-  constexpr int kParts = HALF ? 2 * NW : NW;
-  const int per = (a.ksteps + kParts - 1) / kParts;
-  const int s0 = (HALF ? 2 * wave + ln / 8 : wave) * per, s1 = min(s0 + per, a.ksteps);
+    xp[mt] = a.x + static_cast<int64_t>(min(16 * mt + ln, a.rows - 1)) * a.x_stride + 8 * g;
+  const int units = HALF ? (a.ksteps + 1) / 2 : a.ksteps;   // pairs of steps, or steps
+  const int per = (units + NW - 1) / NW;
+  const int s0 = wave * per, s1 = min(s0 + per, units);
   f4 acc[NT][MT];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = f4{0.f, 0.f, 0.f, 0.f};
-  // (HALF: the bounds differ between the lanes' halves, the trip count is the
-  // same; loads past a part's end are inside the row and replaced by zeros.)
-  for (int s = s0; HALF ? s < s0 + per : s < s1; s += kRlBatch) {
-    u4 wr[NT][kRlBatch], xr[MT][kRlBatch];
+  for (int s = s0; s < s1; s += BATCH) {
+    u4 wr[NT][BATCH], xr[MT][BATCH];
 #pragma unroll
-    for (int i = 0; i < kRlBatch; ++i) {
-      const int at = 32 * min(s + i, (HALF ? a.ksteps : s1) - 1);   // past the wave's last step: the last again, unused
+    for (int i = 0; i < BATCH; ++i) {
+      const int unit = min(s + i, s1 - 1);   // past the wave's last: the last again, unused
+      const int at = 32 * (HALF ? min(2 * unit + odd, a.ksteps - 1) : unit);
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) wr[nt][i] = *reinterpret_cast<const u4 *>(wp[nt] + at);
 #pragma unroll
@@ -98,16 +132,12 @@ __global__ __launch_bounds__(NW * 64) void row_linear_kernel(RowLinearArgs a) {
     asm volatile("" ::: "memory");   // (the loads stay a batch: none is sunk to its use)
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < kRlBatch; ++i) {
-      if constexpr (HALF) {
-        if (s + i >= s0 + per) break;   // wave-uniform (s - s0 is)
-        if (s + i >= s1) {
-          xr[0][i] = u4{0, 0, 0, 0};
+    for (int i = 0; i < BATCH; ++i) {
+      if (s + i >= s1) break;   // wave-uniform
+      if (HALF && 2 * (s + i) + odd >= a.ksteps) {   // the step that an odd number of them lacks
+        xr[0][i] = u4{0, 0, 0, 0};
 #pragma unroll
-          for (int nt = 0; nt < NT; ++nt) wr[nt][i] = u4{0, 0, 0, 0};
-        }
-      } else {
-        if (s + i >= s1) break;   // wave-uniform
+        for (int nt = 0; nt < NT; ++nt) wr[nt][i] = u4{0, 0, 0, 0};
       }
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt)
@@ -122,69 +152,60 @@ __global__ __launch_bounds__(NW * 64) void row_linear_kernel(RowLinearArgs a) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) s_part[wave][nt * MT + mt][lane] = acc[nt][mt];
   __syncthreads();
-  static_assert(NT * MT <= NW, "a wavefront sums one tile");
-  if (wave >= NT * MT) return;
-  f4 sum = s_part[0][wave][lane];   // outputs 16 tile + 4 g + i of row 16 mt + ln
-#pragma unroll
-  for (int p = 1; p < NW; ++p) sum += s_part[p][wave][lane];
-  const int row = 16 * (wave % MT) + ln;
-  const int64_t tile = static_cast<int64_t>(blockIdx.x) * NT + wave / MT;
-  if (tile >= a.tiles) return;
-  if constexpr (HALF) {
-    // outputs 8 tile + (4 g + i) % 8: lanes ln < 8, g < 2 hold the sums over the
-    // first parts of k, lanes ln + 8, g + 2 the same outputs' over the second
-#pragma unroll
-    for (int i = 0; i < 4; ++i) sum[i] += lane_xor32(dpp_rotate<0x128>(sum[i]));
-    if (g < 2 && row < a.rows)
-      *reinterpret_cast<u2 *>(a.y + row * a.y_stride + 8 * tile + 4 * g) =
-          u2{pack_bf16x2(sum[0], sum[1]), pack_bf16x2(sum[2], sum[3])};
-  } else if constexpr (GLU) {
-    // rows 4 g + i of the tile: g < 2 gate columns, g + 2 their up columns
-    f4 up;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) up[i] = lane_xor32(sum[i]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) sum[i] = situ_value<CAP4>(sum[i], up[i], a.rcg, a.rcu, a.scale);
-    if (g < 2 && row < a.rows)
-      *reinterpret_cast<u2 *>(a.y + row * a.y_stride + 8 * tile + 4 * g) =
-          u2{pack_bf16x2(sum[0], sum[1]), pack_bf16x2(sum[2], sum[3])};
-  } else if (row < a.rows) {
-    *reinterpret_cast<u2 *>(a.y + row * a.y_stride + 16 * tile + 4 * g) =
-        u2{pack_bf16x2(sum[0], sum[1]), pack_bf16x2(sum[2], sum[3])};
-  }
+  for (int t = wave; t < NT * MT; t += NW)   // (wave-uniform)
+    store_tile<NW, NT, MT, GLU, CAP4, HALF>(a, s_part, t / MT, t % MT, lane);
 }
 
-template <int NW, int NT, int MT, bool GLU, bool CAP4, bool HALF = false>
+template <int NW, int NT, int MT, int BATCH, bool GLU, bool CAP4, bool HALF>
 int launch(const RowLinearArgs &a, hipStream_t st) {
-  hipLaunchKernelGGL((row_linear_kernel<NW, NT, MT, GLU, CAP4, HALF>), dim3(static_cast<unsigned>((a.tiles + NT - 1) / NT)),
-                     dim3(NW * 64), 0, st, a);
+  hipLaunchKernelGGL((row_linear_kernel<NW, NT, MT, BATCH, GLU, CAP4, HALF>),
+                     dim3(static_cast<unsigned>((a.tiles + NT - 1) / NT)), dim3(NW * 64), 0, st, a);
   return check_launch(GLU ? "row_linear_situ_glu" : "row_linear");
 }
 
-// One tile of outputs per work-group while that leaves no CU a second one, else
+// The loads of a batch that a wavefront's share of k does not fill are loads of
+// the same bytes again, so the batch is the share where one holds it (2,048 x 384
+// 3.8 -> 2.4 us, 7,936 x 1,536 9.2 -> 8.6).
+template <int NW, int NT, int MT, bool GLU, bool CAP4, bool HALF>
+int dispatch_batch(const RowLinearArgs &a, int units, hipStream_t st) {
+  const int per = (units + NW - 1) / NW;
+  if constexpr (NW == 4 || (HALF && NT > 1)) {   // else k is long: more than four steps each
+    if (per <= 1) return launch<NW, NT, MT, 1, GLU, CAP4, HALF>(a, st);
+    if (per <= 3) return launch<NW, NT, MT, 3, GLU, CAP4, HALF>(a, st);
+  }
+  if (per <= 6 || NT > 2) return launch<NW, NT, MT, 6, GLU, CAP4, HALF>(a, st);   // (registers)
+  return launch<NW, NT, MT, 8, GLU, CAP4, HALF>(a, st);
+}
+
+// At most eight rows: half tiles, one per work-group while that leaves no CU a
+// second one, else two, and five where two per work-group are more work-groups
+// than two per CU (8,384 x 1,536: 7.5 us with five on 210 CUs, 8.8 with two,
+// 10.1 with four on 262: a second round for six).
+template <bool GLU, bool CAP4>
+int dispatch_half(RowLinearArgs a, hipStream_t st) {
+  a.tiles *= 2;
+  const int units = (a.ksteps + 1) / 2;
+  if (a.tiles > 1024) return dispatch_batch<8, 5, 1, GLU, CAP4, true>(a, units, st);
+  if (a.tiles > 256) return dispatch_batch<8, 2, 1, GLU, CAP4, true>(a, units, st);
+  if (units <= 32) return dispatch_batch<4, 1, 1, GLU, CAP4, true>(a, units, st);
+  return dispatch_batch<8, 1, 1, GLU, CAP4, true>(a, units, st);
+}
+
+// Whole tiles: one per work-group while that leaves no CU a second one, else
 // two, which share their loads of x (7,936 outputs, k = 1,536, 16 rows: 11.0 us
 // with one tile, 9.7 with two, four on 124 CUs 13.8).
 template <int NW, int MT, bool GLU, bool CAP4>
 int dispatch_tiles(const RowLinearArgs &a, hipStream_t st) {
-  if (a.tiles > 256) return launch<NW, 2, MT, GLU, CAP4>(a, st);
-  return launch<NW, 1, MT, GLU, CAP4>(a, st);
+  if (a.tiles > 256) return dispatch_batch<NW, 2, MT, GLU, CAP4, false>(a, a.ksteps, st);
+  return dispatch_batch<NW, 1, MT, GLU, CAP4, false>(a, a.ksteps, st);
 }
 
 // Wavefronts so that one batch holds a wavefront's share of k: 4 up to k =
 // 1,024, 8 up to 2,048, 16 beyond.
 template <bool GLU, bool CAP4>
 int dispatch(const RowLinearArgs &a, hipStream_t st) {
-  const int need = (a.ksteps + kRlBatch - 1) / kRlBatch;
-  // Half tiles while they are at most one per CU; past that whole tiles fill
-  // the chip.  k over 8 parts up to 2,048, over 16 beyond.
-  if constexpr (!GLU) {
-    if (a.rows <= 8 && a.tiles <= 128) {
-      RowLinearArgs half = a;
-      half.tiles = 2 * a.tiles;
-      if (need <= 8) return launch<4, 1, 1, false, false, true>(half, st);
-      return launch<8, 1, 1, false, false, true>(half, st);
-    }
-  }
+  if (a.rows <= 8) return dispatch_half<GLU, CAP4>(a, st);
+  const int need = (a.ksteps + 7) / 8;
   if (a.rows <= 16) {
     if (need <= 4) return dispatch_tiles<4, 1, GLU, CAP4>(a, st);
     if (need <= 8) return dispatch_tiles<8, 1, GLU, CAP4>(a, st);
@@ -222,10 +243,10 @@ __global__ __launch_bounds__(kHlWaves * 64) void head_linear_kernel(HeadLinearAr
   const uint16_t *wp = a.w + (static_cast<int64_t>(h) * a.n + n0 + ln) * k + 8 * g;
   const uint16_t *xp = a.x + min(row, a.rows - 1) * a.x_row + h * a.x_head + 8 * g;
   f4 acc = f4{0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < a.ksteps; s += kRlBatch) {
-    u4 wr[kRlBatch], xr[kRlBatch];
+  for (int s = 0; s < a.ksteps; s += kHlBatch) {
+    u4 wr[kHlBatch], xr[kHlBatch];
 #pragma unroll
-    for (int i = 0; i < kRlBatch; ++i) {
+    for (int i = 0; i < kHlBatch; ++i) {
       const int at = 32 * min(s + i, a.ksteps - 1);
       wr[i] = *reinterpret_cast<const u4 *>(wp + at);
       xr[i] = *reinterpret_cast<const u4 *>(xp + at);
@@ -233,7 +254,7 @@ __global__ __launch_bounds__(kHlWaves * 64) void head_linear_kernel(HeadLinearAr
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < kRlBatch; ++i) {
+    for (int i = 0; i < kHlBatch; ++i) {
       if (s + i >= a.ksteps) break;
       acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf8(wr[i]), as_bf8(xr[i]), acc, 0, 0, 0);
     }

@@ -905,16 +905,17 @@ def _row_linear_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether ``F.linear(x, weight)`` may run on the few-row kernel, and gains
     by it.  It may when nothing else than the values is asked of the call (no
     gradient, trace, transform, mode or autocast) and the layout fits.  It gains
-    up to 32 rows and 512 tiles of outputs: with more rows than that each
-    work-group's reads of x weigh as much as the weight's, and past two tiles per
-    CU the library's GEMM is as fast (8,384 x 1,536: 12.1 us against 11.3 at 8
-    rows, the vocabulary's 65,536: 54 against 39)."""
+    with up to 8 rows at any number of outputs (us, library and kernel: 8,384 x
+    1,536 12.7 and 8.5, the vocabulary's 65,536 43.8 and 43.0), and with up to 32
+    to 512 tiles of outputs (16 rows: 7,936 11.9 and 9.6, but 8,384 12.8 and 14.0):
+    past two tiles per CU each work-group's reads of x weigh as much as the
+    weight's."""
     if not _values_only(x, weight):   # (first: a wrapped tensor has no pointer to look at)
         return False
     k = x.shape[-1]
     if (x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or x.device.type != "cuda"
             or weight.device != x.device or x.numel() > ROW_LINEAR_MAX * k or x.numel() == 0
-            or k % 32 or weight.shape[0] % 16 or weight.shape[0] > 512 * 16):
+            or k % 32 or weight.shape[0] % 16 or (weight.shape[0] > 512 * 16 and x.numel() > 8 * k)):
         return False
     return (weight.is_contiguous() and x.stride(-1) == 1 and x.data_ptr() % 16 == 0
             and weight.data_ptr() % 16 == 0)

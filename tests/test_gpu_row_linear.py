@@ -34,10 +34,12 @@ def _close(y, ref):
 
 # one k-step; k short of, at and past one batch of steps per wavefront with 4,
 # 8 and 16 wavefronts, and past one batch of 16; one and two tiles per
-# work-group, an odd tile left over
+# work-group, an odd tile left over; half tiles (to 8 rows) by one, two and five,
+# an odd number of k-steps
 @pytest.mark.parametrize("n,k", [(16, 32), (48, 96), (2048, 128), (32, 1024), (32, 1056), (1536, 2048), (16, 2080),
-                                 (1536, 3968), (16, 8192), (16 * 257, 64), (16 * 511, 1536)])
-@pytest.mark.parametrize("rows", [1, 8, 16, 17, 32])
+                                 (1536, 3968), (16, 8192), (16 * 257, 64), (16 * 511, 1536), (16 * 524, 96),
+                                 (16 * 513, 3616), (2048, 384)])
+@pytest.mark.parametrize("rows", [1, 8, 9, 16, 17, 32])
 def test_row_linear_matches_float64(rows, n, k):
     from sophia_amd import ops
     dev = _dev()
@@ -48,8 +50,8 @@ def test_row_linear_matches_float64(rows, n, k):
     assert y.shape == (rows, n) and _close(y, x.double() @ w.double().t())
 
 
-@pytest.mark.parametrize("hidden,k", [(8, 32), (24, 160), (3968, 1536), (8 * 259, 64)])
-@pytest.mark.parametrize("rows,cap", [(1, 4.0), (16, 3.0), (19, 4.0), (32, 4.0)])
+@pytest.mark.parametrize("hidden,k", [(8, 32), (24, 160), (3968, 1536), (8 * 259, 64), (8 * 519, 96)])
+@pytest.mark.parametrize("rows,cap", [(1, 4.0), (8, 3.0), (16, 3.0), (19, 4.0), (32, 4.0)])
 def test_row_linear_situ_glu_matches_float64(rows, cap, hidden, k):
     from sophia_amd import ops
     dev = _dev()

@@ -199,11 +199,13 @@ int sophia_row_linear_situ_glu(const void *x, int64_t x_stride, const void *w, i
  * and v_up (ml/runtime/model/attention.py:623-628 folded into latent space).
  * Strides in elements (x: multiples of 8, x and w 16-byte aligned; y: multiples
  * of 4, 8-byte aligned), rows at least as far apart as their heads reach; k a
- * multiple of 32, n of 16.  y may not overlap x or w.
+ * multiple of 32, n of 16.  With ``gate`` (bf16 logits strided as y may be; or
+ * NULL) y is the bf16 product times sigmoid(gate) (attention.py:655-656).  y may
+ * not overlap an input.
  */
 int sophia_head_linear(const void *x, int64_t x_row_stride, int64_t x_head_stride, const void *w, void *y,
-                       int64_t y_row_stride, int64_t y_head_stride, int64_t rows, int heads, int n, int k,
-                       void *stream);
+                       int64_t y_row_stride, int64_t y_head_stride, const void *gate, int64_t gate_row_stride,
+                       int64_t gate_head_stride, int64_t rows, int heads, int n, int k, void *stream);
 
 #ifdef __cplusplus
 }

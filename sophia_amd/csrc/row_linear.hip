@@ -221,13 +221,17 @@ int dispatch(const RowLinearArgs &a, hipStream_t st) {
 // (16 rows, head, 128 outputs), a wavefront per 16 outputs over all of k, its
 // loads eight k-steps at a time.  At 8 rows x 16 heads x 128 x 128 one launch
 // of 5 us takes the place of a batched library GEMM (7.8 us) and the two
-// transposing copies around it (4.6 us each).
+// transposing copies around it (4.6 us each).  With a gate the output is
+// multiplied by its sigmoid (attention.py:655-656), rounded to bf16 before and
+// after as two launches round it: a launch of 4.5 us less.
 struct HeadLinearArgs {
   const uint16_t *x;
   int64_t x_row, x_head;
   const uint16_t *w;
   uint16_t *y;
   int64_t y_row, y_head;
+  const uint16_t *gate;   // logits like y, or NULL
+  int64_t gate_row, gate_head;
   int rows, n, ksteps;
 };
 
@@ -242,6 +246,9 @@ __global__ __launch_bounds__(kHlWaves * 64) void head_linear_kernel(HeadLinearAr
   const int64_t k = 32 * static_cast<int64_t>(a.ksteps);
   const uint16_t *wp = a.w + (static_cast<int64_t>(h) * a.n + n0 + ln) * k + 8 * g;
   const uint16_t *xp = a.x + min(row, a.rows - 1) * a.x_row + h * a.x_head + 8 * g;
+  u2 gate = u2{0, 0};
+  if (a.gate)   // uniform
+    gate = *reinterpret_cast<const u2 *>(a.gate + min(row, a.rows - 1) * a.gate_row + h * a.gate_head + n0 + 4 * g);
   f4 acc = f4{0.f, 0.f, 0.f, 0.f};
   for (int s = 0; s < a.ksteps; s += kHlBatch) {
     u4 wr[kHlBatch], xr[kHlBatch];
@@ -257,6 +264,14 @@ __global__ __launch_bounds__(kHlWaves * 64) void head_linear_kernel(HeadLinearAr
     for (int i = 0; i < kHlBatch; ++i) {
       if (s + i >= a.ksteps) break;
       acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf8(wr[i]), as_bf8(xr[i]), acc, 0, 0, 0);
+    }
+  }
+  if (a.gate) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float logit = __uint_as_float(i % 2 ? gate[i / 2] & 0xffff0000u : gate[i / 2] << 16);
+      acc[i] = as_dtype(acc[i], SOPHIA_DTYPE_BF16) *
+               __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896341f * logit));
     }
   }
   if (row < a.rows)
@@ -310,7 +325,8 @@ extern "C" int sophia_row_linear_situ_glu(const void *x, int64_t x_stride, const
 }
 
 extern "C" int sophia_head_linear(const void *x, int64_t x_row_stride, int64_t x_head_stride, const void *w, void *y,
-                                  int64_t y_row_stride, int64_t y_head_stride, int64_t rows, int heads, int n, int k,
+                                  int64_t y_row_stride, int64_t y_head_stride, const void *gate,
+                                  int64_t gate_row_stride, int64_t gate_head_stride, int64_t rows, int heads, int n, int k,
                                   void *stream) {
   SOPHIA_REQUIRE(rows >= 0 && rows <= 0x7fffffff && heads > 0 && heads <= 65535, "head_linear: bad rows / heads");
   SOPHIA_REQUIRE(k > 0 && k % 32 == 0 && n > 0 && n % 16 == 0 && (n + 127) / 128 <= 65535,
@@ -323,9 +339,14 @@ extern "C" int sophia_head_linear(const void *x, int64_t x_row_stride, int64_t x
   SOPHIA_REQUIRE(reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 &&
                      reinterpret_cast<uintptr_t>(y) % 8 == 0,
                  "head_linear: x and w must be 16-byte and y 8-byte aligned");
+  SOPHIA_REQUIRE(!gate || (gate_head_stride >= n && gate_row_stride >= (heads - 1) * gate_head_stride + n &&
+                           gate_row_stride % 4 == 0 && gate_head_stride % 4 == 0 &&
+                           reinterpret_cast<uintptr_t>(gate) % 8 == 0),
+                 "head_linear: bad gate strides or alignment");
   if (rows == 0) return SOPHIA_OK;
   const HeadLinearArgs a{static_cast<const uint16_t *>(x), x_row_stride, x_head_stride, static_cast<const uint16_t *>(w),
-                         static_cast<uint16_t *>(y), y_row_stride, y_head_stride, static_cast<int>(rows), n, k / 32};
+                         static_cast<uint16_t *>(y), y_row_stride, y_head_stride, static_cast<const uint16_t *>(gate),
+                         gate_row_stride, gate_head_stride, static_cast<int>(rows), n, k / 32};
   const dim3 grid(static_cast<unsigned>((rows + 15) / 16), static_cast<unsigned>(heads),
                   static_cast<unsigned>((n + 127) / 128));
   hipLaunchKernelGGL(head_linear_kernel, grid, dim3(kHlWaves * 64), 0, static_cast<hipStream_t>(stream), a);

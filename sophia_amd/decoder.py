@@ -363,7 +363,12 @@ class SophiaMLA(nn.Module):
             ctx = ops.mla_decode_attn(qa.contiguous(), cache, step["decode_slots"], step["decode_pos"],
                                       d ** -0.5, max_len=int(step["max_decode_len"]))   # [D, h, r]
             if heads_kernel:
-                ops.head_linear(ctx, self.v_up.weight.view(h, d, r), out=out[npre:])
+                # decode rows alone: the output gate on the products as they are formed
+                own = npre == 0 and gate.dtype == x.dtype and gate.stride(0) % 4 == 0 and gate.data_ptr() % 8 == 0 and ops._values_only(gate)
+                ops.head_linear(ctx, self.v_up.weight.view(h, d, r), out=out[npre:],
+                                gate=gate.unflatten(1, (h, d)) if own else None)
+                if own:
+                    return self.o_proj(out.view(n, self.inner_dim))
             else:
                 o = torch.bmm(ctx.transpose(0, 1).contiguous(), self._v_up_t(x.dtype))
                 out[npre:] = o.transpose(0, 1)

@@ -978,11 +978,13 @@ def row_linear_situ_glu(x: torch.Tensor, weight: torch.Tensor, gate_softcap: flo
     return h
 
 
-def head_linear(x: torch.Tensor, weight: torch.Tensor, *, out: torch.Tensor | None = None) -> torch.Tensor:
+def head_linear(x: torch.Tensor, weight: torch.Tensor, *, out: torch.Tensor | None = None,
+                gate: torch.Tensor | None = None) -> torch.Tensor:
     """Per-head projection (sophia_head_linear): out[r, h] = x[r, h] . weight[h]^T
     in bf16, x [rows, heads, k] with dense last dim, weight [heads, n, k]
     contiguous, k a multiple of 32, n of 16.  Returns [rows, heads, n] (or
-    ``out``, whose rows and heads may be strided)."""
+    ``out``, whose rows and heads may be strided); with ``gate`` (bf16 logits
+    [rows, heads, n]) times its sigmoid, as ``gated_head_norm`` of the result."""
     _gpu(x, "x")
     _gpu(weight, "weight")
     rows, heads, k = (int(v) for v in x.shape)
@@ -993,11 +995,17 @@ def head_linear(x: torch.Tensor, weight: torch.Tensor, *, out: torch.Tensor | No
     y = out if out is not None else torch.empty((rows, heads, n), dtype=x.dtype, device=x.device)
     if y.dtype != x.dtype or tuple(y.shape) != (rows, heads, n) or y.stride(2) != 1 or y.device != x.device:
         raise RuntimeError(f"out must be bf16 [{rows}, {heads}, {n}]")
+    if gate is not None and (gate.dtype != x.dtype or tuple(gate.shape) != (rows, heads, n) or gate.stride(2) != 1
+                             or gate.device != x.device):
+        raise RuntimeError(f"gate must be bf16 [{rows}, {heads}, {n}]")
     xh = x.stride(1) if heads > 1 else k
     yh = y.stride(1) if heads > 1 else n
+    gh = n if gate is None or heads == 1 else gate.stride(1)
+    gr = gate.stride(0) if gate is not None and rows > 1 else (heads - 1) * gh + n
     rc = nat.lib().sophia_head_linear(
         x.data_ptr(), x.stride(0) if rows > 1 else (heads - 1) * xh + k, xh, weight.data_ptr(), y.data_ptr(),
-        y.stride(0) if rows > 1 else (heads - 1) * yh + n, yh, rows, heads, n, k, nat.stream_handle(x.device))
+        y.stride(0) if rows > 1 else (heads - 1) * yh + n, yh, nat.ptr(gate), gr, gh, rows, heads, n, k,
+        nat.stream_handle(x.device))
     nat.check(rc, "sophia_head_linear")
     return y
 

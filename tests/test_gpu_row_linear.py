@@ -153,5 +153,11 @@ def test_head_linear_matches_float64(rows, heads, n, k):
     ref = torch.einsum("rhk,hnk->rhn", wide[:, :, 8:].double(), w.double())
     assert _close(y, ref) and _close(ops.head_linear(wide.to(dev)[:, :, 8:], w.to(dev)), ref)
     assert bool((big[0] == 3).all() and (big[-1] == 3).all() and (big[1:-1, :, n:] == 3).all())
+    gate = torch.randn(rows, heads * n + 4, generator=g).to(torch.bfloat16).to(dev)[:, 4:].unflatten(1, (heads, n))
+    gated = ops.head_linear(wide.to(dev)[:, :, 8:], w.to(dev), gate=gate)
+    plain = ops.head_linear(wide.to(dev)[:, :, 8:], w.to(dev))
+    assert _close(gated, plain.double().cpu() * torch.sigmoid(gate.double().cpu()))
     with pytest.raises(RuntimeError):
         ops.head_linear(wide.to(dev)[:, :, 8:].float(), w.to(dev))
+    with pytest.raises(RuntimeError):
+        ops.head_linear(wide.to(dev)[:, :, 8:], w.to(dev), gate=gate.float())

@@ -92,6 +92,7 @@ struct BwdArgs {
   // outputs: dq, dk, dv of element type grad_dtype, the others fp32
   void *dq, *dk, *dv;
   int grad_dtype;
+  int grad_heads;   // heads in a row of dq, dk, dv
   float *dg, *dbeta, *dh0, *dA_log, *ddt_bias;
   // workspace
   float *qh, *kh, *gl, *bt;        // prepared q^, k^, alpha = e^g, beta
@@ -452,7 +453,7 @@ __global__ __launch_bounds__(kChainThreads) void kda_bwd_chain_kernel(BwdArgs a)
               dst[((static_cast<int64_t>(slice) * a.total + tok) * a.num_heads + h) * kD + row] = rsum;
             }
             if (c.rg == 0) {
-              store_elem(a.dv, (tok * a.num_heads + h) * kD + c.col, a.grad_dtype, cur.bt * du);
+              store_elem(a.dv, (tok * a.grad_heads + h) * kD + c.col, a.grad_dtype, cur.bt * du);
               if (l32 == 3 * kRows) a.dbp[(static_cast<int64_t>(slice) * a.total + tok) * a.num_heads + h] = rsum;
             }
           }
@@ -514,8 +515,9 @@ __global__ __launch_bounds__(kD) void kda_bwd_post_kernel(BwdArgs a) {
     dq = (lq < 1e-12f ? dyq : dyq - yq * ((s_red[0][0] + s_red[1][0]) / nq)) / nq;
     dk = (lk < 1e-12f ? dkh : dkh - yk * ((s_red[0][1] + s_red[1][1]) / nk)) / nk;
   }
-  store_elem(a.dq, o, a.grad_dtype, dq);
-  store_elem(a.dk, o, a.grad_dtype, dk);
+  const int64_t go = (tok * a.grad_heads + h) * kD + c;
+  store_elem(a.dq, go, a.grad_dtype, dq);
+  store_elem(a.dk, go, a.grad_dtype, dk);
   // alpha = e^g: dg = dalpha alpha; through the gate, dz = dg lb s (1 - s) e^A_log
   float dgv = dal * a.gl[o];
   if (a.flags & SOPHIA_KDA_GATE_IN_KERNEL) {
@@ -549,7 +551,7 @@ __device__ __forceinline__ void covered_rows(const BwdArgs &a, int64_t &lo, int6
 // them in its state-scan kernel).
 constexpr int kZeroBlocks = 64;
 __global__ __launch_bounds__(256) void kda_bwd_zero_outside_kernel(BwdArgs a) {
-  zero_rows_outside(a.cu, a.n_seqs, a.total, a.num_heads, a.dq, a.dk, a.dv, a.grad_dtype, a.dg, a.dbeta,
+  zero_rows_outside(a.cu, a.n_seqs, a.total, a.num_heads, a.dq, a.dk, a.dv, a.grad_dtype, a.grad_heads, a.dg, a.dbeta,
                     static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x, static_cast<int64_t>(kZeroBlocks) * 256);
 }
 
@@ -703,6 +705,12 @@ extern "C" int sophia_kda_chunk_bwd(const void *q, const void *k, const void *v,
   SOPHIA_REQUIRE(cu_seqlens && workspace &&
                      (total_tokens == 0 || (q && k && v && g && beta && d_out && dq && dk && dv && dg && dbeta)),
                  "kda_chunk_bwd: NULL pointer");
+  if ((flags & SOPHIA_KDA_BWD_GRAD_PACKED) && total_tokens > 0) {
+    const size_t part = static_cast<size_t>(num_heads) * kD * ((flags & SOPHIA_KDA_BWD_GRAD_BF16) ? 2 : 4);
+    SOPHIA_REQUIRE(static_cast<uint8_t *>(dk) == static_cast<uint8_t *>(dq) + part &&
+                       static_cast<uint8_t *>(dv) == static_cast<uint8_t *>(dk) + part,
+                   "kda_chunk_bwd: packed dq, dk, dv must follow each other in one row");
+  }
   const bool gate = (flags & SOPHIA_KDA_GATE_IN_KERNEL) != 0;
   SOPHIA_REQUIRE(!gate || (A_log && dt_bias), "kda_chunk_bwd: gate in kernel needs A_log and dt_bias");
   SOPHIA_REQUIRE(gate || (!dA_log && !ddt_bias),
@@ -736,6 +744,7 @@ extern "C" int sophia_kda_chunk_bwd(const void *q, const void *k, const void *v,
   a.dht = d_final_state;
   a.dq = dq; a.dk = dk; a.dv = dv; a.dg = dg; a.dbeta = dbeta; a.dh0 = d_initial_state;
   a.grad_dtype = (flags & SOPHIA_KDA_BWD_GRAD_BF16) ? SOPHIA_DTYPE_BF16 : SOPHIA_DTYPE_F32;
+  a.grad_heads = (flags & SOPHIA_KDA_BWD_GRAD_PACKED) ? 3 * num_heads : num_heads;
   a.dA_log = dA_log; a.ddt_bias = ddt_bias;
   a.qh = carve(tok * kD * 4);
   a.kh = carve(tok * kD * 4);
@@ -784,7 +793,7 @@ extern "C" int sophia_kda_chunk_bwd(const void *q, const void *k, const void *v,
     ChunkBwdIO io{q, k, v, qkv_row_stride, qkv_dtype, g, g_row_stride, g_dtype, beta, beta_row_stride,
                   beta_dtype, A_log, dt_bias, scale, lower_bound, flags, cu_seqlens, n_seqs, total_tokens,
                   num_heads, initial_state, d_out, d_out_row_stride, d_out_dtype, d_final_state,
-                  dq, dk, dg, dbeta, dv, d_initial_state, a.grad_dtype};
+                  dq, dk, dg, dbeta, dv, d_initial_state, a.grad_dtype, a.grad_heads};
     if (const int rc = chunk_bwd_run(io, scratch, st)) return rc;
   }
   if (recurrent && total_tokens > 0) {

@@ -1780,6 +1780,7 @@ struct BwdChunkArgs {
   float *dg, *dbeta;                   // gradients of g, beta (fp32)
   void *dv;                            // gradient of v (element type grad_dtype)
   int grad_dtype;
+  int grad_heads;                      // heads in a row of dq, dk, dv
 };
 
 // One (sequence, head, NVB value columns) of the forward scan that keeps S0
@@ -1882,7 +1883,7 @@ __global__ __launch_bounds__(kScanThreads) void kda_bwd_states_kernel(BwdChunkAr
   __shared__ __attribute__((aligned(16))) uint8_t sUb[2 * 8 * 64 * 16];
   const ScanArgs &p = a.p;
   if (p.total > 0)   // rows no sequence covers: zero gradients (no other kernel writes them)
-    zero_rows_outside(p.cu, p.n_seqs, p.total, p.num_heads, a.dq, a.dk, a.dv, a.grad_dtype, a.dg, a.dbeta,
+    zero_rows_outside(p.cu, p.n_seqs, p.total, p.num_heads, a.dq, a.dk, a.dv, a.grad_dtype, a.grad_heads, a.dg, a.dbeta,
                       static_cast<int64_t>(blockIdx.x) * kScanThreads + threadIdx.x,
                       static_cast<int64_t>(gridDim.x) * kScanThreads);
   int item, half;
@@ -2150,6 +2151,7 @@ __global__ __launch_bounds__(kGradThreads) void kda_bwd_grad_kernel(BwdChunkArgs
   const int rb = 16 * w;
   const int st0 = w >> 1;   // T^T[m][k] = T[k][m] vanishes for k < m: row blocks 2, 3 skip K-step 0
   const auto tok_off = [&](int r) { return (tok0 + r) * static_cast<int64_t>(H) + h; };
+  const auto grad_off = [&](int r) { return (tok0 + r) * static_cast<int64_t>(a.grad_heads) + h; };
   const int64_t vrow = static_cast<int64_t>(h) * kD;
   const float *S0 = a.s0 + it * (kD * kD);
   const float *dS1 = a.ds1 + it * (kD * kD);
@@ -2356,7 +2358,7 @@ __global__ __launch_bounds__(kGradThreads) void kda_bwd_grad_kernel(BwdChunkArgs
       const int r = rb + 4 * gq + e;
       const float bt = sBt[r];
       dbr[e] += dxu[k][e] * vown[k][e];
-      if (r < len) store_elem(a.dv, tok_off(r) * kD + c, GD, bt * dxu[k][e]);
+      if (r < len) store_elem(a.dv, grad_off(r) * kD + c, GD, bt * dxu[k][e]);
     }
   }
   lds_barrier();   // dU is read; dA_qk and dU U^T are complete
@@ -2707,8 +2709,9 @@ __global__ __launch_bounds__(kGradThreads) void kda_bwd_grad_kernel(BwdChunkArgs
       }
       const int64_t o = tok_off(r) * kD + blk_c;
       *reinterpret_cast<f4 *>(&a.dg[o]) = d;
-      store4(a.dq, o, GD, dqs - qv[q] * (sIq[r] * sq));
-      store4(a.dk, o, GD, dks * rk - kv[q] * (sIk[r] * rk * rk * rk * sk));
+      const int64_t go = grad_off(r) * kD + blk_c;
+      store4(a.dq, go, GD, dqs - qv[q] * (sIq[r] * sq));
+      store4(a.dk, go, GD, dks * rk - kv[q] * (sIk[r] * rk * rk * rk * sk));
     }
   }
 }
@@ -2867,7 +2870,7 @@ int chunk_bwd_run(const ChunkBwdIO &io, void *scratch, hipStream_t st) {
   a.beta = io.beta; a.beta_stride = io.beta_stride; a.beta_dtype = io.beta_dtype;
   a.A_log = io.A_log; a.dt_bias = io.dt_bias; a.scale = io.scale; a.lb = io.lb; a.flags = io.flags;
   a.dout = io.dout; a.do_stride = io.do_stride; a.do_dtype = io.do_dtype;
-  a.dq = io.dq; a.dk = io.dk; a.dg = io.dg; a.dbeta = io.dbeta; a.dv = io.dv; a.grad_dtype = io.grad_dtype;
+  a.dq = io.dq; a.dk = io.dk; a.dg = io.dg; a.dbeta = io.dbeta; a.dv = io.dv; a.grad_dtype = io.grad_dtype; a.grad_heads = io.grad_heads;
   hipLaunchKernelGGL(kda_bwd_states_kernel, dim3(static_cast<unsigned>(sblocks)), dim3(kScanThreads), 0, st, a);
   if (const int rc = check_launch("kda_bwd_states")) return rc;
   hipLaunchKernelGGL(kda_bwd_rscan_kernel, dim3(static_cast<unsigned>(sblocks)), dim3(kScanThreads), 0, st, a);

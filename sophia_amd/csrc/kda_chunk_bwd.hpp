@@ -35,7 +35,8 @@ struct ChunkBwdIO {
   int64_t do_stride;
   int do_dtype;
   const float *dht;         // [n_seqs][H][128][128] or NULL
-  // outputs: gradients of q, k, v [total][H][128] (element type grad_dtype),
+  // outputs: gradients of q, k, v [total][H][128] (rows of grad_heads heads,
+  // element type grad_dtype),
   // of g (the gate's input, or the log-decay itself without the gate in the
   // kernel) [total][H][128] and beta [total][H] (fp32), and of the initial
   // states (fp32, or NULL)
@@ -44,6 +45,7 @@ struct ChunkBwdIO {
   void *dv;
   float *dh0;
   int grad_dtype;
+  int grad_heads;           // heads in a row of dq, dk, dv: H, or 3 H where they are interleaved
 };
 
 // Rows outside every sequence (before cu[0], or from cu[n_seqs] on, both
@@ -51,7 +53,8 @@ struct ChunkBwdIO {
 // `t` of `threads` takes every threads-th element of those rows (usually
 // none).
 __device__ __forceinline__ void zero_rows_outside(const int32_t *cu, int n_seqs, int64_t total, int num_heads,
-                                                  void *dq, void *dk, void *dv, int grad_dtype, float *dg,
+                                                  void *dq, void *dk, void *dv, int grad_dtype, int grad_heads,
+                                                  float *dg,
                                                   float *dbeta, int64_t t, int64_t threads) {
   const int64_t lo = cu[0] < 0 ? 0 : (cu[0] > total ? total : cu[0]);
   const int64_t hi = cu[n_seqs] < lo ? lo : (cu[n_seqs] > total ? total : cu[n_seqs]);
@@ -61,9 +64,10 @@ __device__ __forceinline__ void zero_rows_outside(const int32_t *cu, int n_seqs,
     const int64_t r = i / per_row;
     const int64_t row = r < lo ? r : hi + (r - lo);
     const int64_t e = row * per_row + (i - r * per_row);
-    store_elem(dq, e, grad_dtype, 0.f);
-    store_elem(dk, e, grad_dtype, 0.f);
-    store_elem(dv, e, grad_dtype, 0.f);
+    const int64_t ge = row * grad_heads * 128 + (i - r * per_row);
+    store_elem(dq, ge, grad_dtype, 0.f);
+    store_elem(dk, ge, grad_dtype, 0.f);
+    store_elem(dv, ge, grad_dtype, 0.f);
     dg[e] = 0.f;
     if (i - r * per_row < num_heads) dbeta[row * num_heads + (i - r * per_row)] = 0.f;
   }

@@ -432,8 +432,12 @@ class SophiaKDA(nn.Module):
                                            step=(seqlen == 1 and cached and self.use_cache))
         shape4 = (bsz, seqlen, self.num_heads, self.head_dim)
         # Strided views of the conv output (no copies): the kernels take row
-        # strides.  One unbind: its backward writes the gradient of qkv once.
-        q, k, v = qkv.view(bsz, seqlen, 3, self.num_heads, self.head_dim).unbind(2)
+        # strides, and the backward's gradients of q, k and v are one row's parts.
+        qkv = qkv.view(bsz, seqlen, 3, self.num_heads, self.head_dim)
+        if _needs_grad(qkv) and ops._plain_dispatch():
+            q, k, v = ops.UnbindHeads.apply(qkv)
+        else:
+            q, k, v = qkv.unbind(2)
         decay = self.decay_up(dd).view(shape4)
         beta_logits = beta_logits.reshape(bsz, seqlen, self.num_heads)
         if pad_mask is not None:

@@ -401,7 +401,7 @@ def kda_chunk_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Te
                   use_beta_sigmoid: bool = True, initial_state: torch.Tensor | None = None,
                   d_final_state: torch.Tensor | None = None,
                   cu_seqlens_cpu: torch.Tensor | None = None, recurrent: bool = False,
-                  grad_dtype: torch.dtype = torch.float32):
+                  grad_dtype: torch.dtype = torch.float32, grad_packed: bool = False):
     """Gradients of ``kda_chunk_fwd`` (no cache slots: one state per sequence).
 
     The HIP counterpart of FlashKDA's chunk_kda_train_bwd plus l2norm_bwd and
@@ -412,7 +412,8 @@ def kda_chunk_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Te
     [N, H, 128, 128], dA_log [H] and ddt_bias [H * 128] (empty without the
     in-kernel gate); ``grad_dtype=torch.bfloat16`` writes dq, dk and dv as
     bf16 instead (the fp32 gradients rounded to nearest even), the element
-    type a bf16 forward's q, k, v carry.  A host ``cu_seqlens`` (or ``cu_seqlens_cpu``) is checked
+    type a bf16 forward's q, k, v carry; ``grad_packed`` returns dq, dk and dv
+    as the parts [:, 0], [:, 1], [:, 2] of one [total, 3, H, 128] buffer.  A host ``cu_seqlens`` (or ``cu_seqlens_cpu``) is checked
     to rise from 0 to the token count.  The chunk form runs by default (bf16
     MFMA operands, fp32 accumulation and state, the forward's arithmetic);
     ``recurrent=True`` runs the per-token recurrence in fp32 instead.
@@ -457,9 +458,12 @@ def kda_chunk_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Te
     if scale is None:
         scale = HEAD_DIM ** -0.5
     f32 = dict(dtype=torch.float32, device=device)
-    dq = torch.empty((total, heads, HEAD_DIM), dtype=grad_dtype, device=device)
-    dk = torch.empty_like(dq)
-    dv = torch.empty_like(dq)
+    if grad_packed:
+        dq, dk, dv = torch.empty((total, 3, heads, HEAD_DIM), dtype=grad_dtype, device=device).unbind(1)
+    else:
+        dq = torch.empty((total, heads, HEAD_DIM), dtype=grad_dtype, device=device)
+        dk = torch.empty_like(dq)
+        dv = torch.empty_like(dq)
     dg = torch.empty((total, heads, HEAD_DIM), **f32)
     dbeta = torch.empty((total, heads), **f32)
     dh0 = torch.empty((n, heads, HEAD_DIM, HEAD_DIM), **f32)
@@ -473,7 +477,8 @@ def kda_chunk_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Te
         nat.dtype_code(g.dtype), nat.ptr(beta), bs, nat.dtype_code(beta.dtype), nat.ptr(a_log),
         nat.ptr(dtb), float(scale), float(lower_bound),
         _flags(use_qk_l2norm, use_gate, use_beta_sigmoid) | (nat.BWD_RECURRENT if recurrent else 0)
-        | (nat.BWD_GRAD_BF16 if grad_dtype == torch.bfloat16 else 0),
+        | (nat.BWD_GRAD_BF16 if grad_dtype == torch.bfloat16 else 0)
+        | (nat.BWD_GRAD_PACKED if grad_packed else 0),
         nat.ptr(cu), n, total, heads, HEAD_DIM,
         nat.ptr(initial_state), nat.ptr(d_out), ds, nat.dtype_code(d_out.dtype),
         nat.ptr(d_final_state), nat.ptr(dq), nat.ptr(dk), nat.ptr(dv), nat.ptr(dg),
@@ -780,6 +785,46 @@ def _grad_like(grad: torch.Tensor, meta):
     return grad.view(meta[0]).to(meta[1])
 
 
+def _parts_of_rows(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
+    """Whether q, k and v are three consecutive parts of the rows of one buffer:
+    the same strides, with rows (the dimension before the heads) 3 H 128 apart
+    and each part H 128 elements after the one before."""
+    part = int(q.size(-2)) * int(q.size(-1))
+    rows = [(int(n), int(s)) for n, s in zip(q.shape[:-2], q.stride()[:-2])]
+    step = 3 * part
+    for n, s in reversed(rows):
+        if n > 1 and s != step:
+            return False
+        step *= n
+    return (q.numel() > 0 and q.dtype == k.dtype == v.dtype and q.shape == k.shape == v.shape
+            and q.stride() == k.stride() == v.stride() and q.stride()[-2:] == (q.size(-1), 1)
+            and q.untyped_storage().data_ptr() == k.untyped_storage().data_ptr() == v.untyped_storage().data_ptr()
+            and k.storage_offset() == q.storage_offset() + part and v.storage_offset() == k.storage_offset() + part)
+
+
+class UnbindHeads(torch.autograd.Function):
+    """q, k, v [B, T, H, D] of fused rows [B, T, 3, H, D]: ``x.unbind(2)`` whose
+    backward takes gradients that lie as parts of one row, as the KDA backward
+    writes them, for the gradient of x without a copy; others are stacked."""
+
+    @staticmethod
+    def forward(ctx, x):
+        ctx.set_materialize_grads(False)
+        ctx.like = (x.shape, x.dtype, x.device)
+        return x.unbind(2)
+
+    @staticmethod
+    def backward(ctx, dq, dk, dv):
+        shape, dtype, device = ctx.like
+        grads = [dq, dk, dv]
+        if all(d is not None for d in grads) and not torch.compiler.is_compiling() and _parts_of_rows(*grads):
+            b, t, three, h, d = shape
+            row = three * h * d
+            return dq.as_strided(shape, (t * row, row, h * d, d, 1), dq.storage_offset())
+        one = shape[:2] + shape[3:]
+        return torch.stack([torch.zeros(one, dtype=dtype, device=device) if d is None else d for d in grads], 2)
+
+
 class ChunkKDAFunction(torch.autograd.Function):
     """FlashKDAFunction (ml/training/pretrain/engine/sm120_concurrent_ffn.py:
     209-373) over the HIP kernels: the forward is the chunk prefill
@@ -820,10 +865,15 @@ class ChunkKDAFunction(torch.autograd.Function):
         if do is None:
             do = torch.zeros((q.size(0), q.size(1), HEAD_DIM), dtype=torch.float32, device=q.device)
         dht = None if dht is None else dht.float().contiguous()
-        # bf16 q, k, v take their gradients as bf16 from the kernel (no casts)
-        dq, dk, dv, dg, db, dh0, da, dbias = torch_ops.kda_chunk_bwd(
-            q, k, v, g, beta, cu, do.contiguous(), a_log, dtb, scale, lb, use_l2, use_gate,
-            use_sig, h0, dht, ctx.cu_cpu, False, q.dtype == torch.bfloat16)
+        # bf16 q, k, v take their gradients as bf16 from the kernel (no casts),
+        # and parts of one row theirs as parts of one row (no gathering copy)
+        more = (q, k, v, g, beta, cu, do.contiguous(), a_log, dtb, scale, lb, use_l2, use_gate,
+                use_sig, h0, dht, ctx.cu_cpu, False, q.dtype == torch.bfloat16)
+        if _parts_of_rows(q, k, v) and not torch.compiler.is_compiling():
+            dqkv, dg, db, dh0, da, dbias = torch_ops.kda_chunk_bwd_packed(*more)
+            dq, dk, dv = dqkv.unbind(1)
+        else:
+            dq, dk, dv, dg, db, dh0, da, dbias = torch_ops.kda_chunk_bwd(*more)
         return (dq.to(q.dtype), dk.to(k.dtype), dv.to(v.dtype), dg.to(g.dtype), db.to(beta.dtype),
                 _grad_like(da, A_log) if use_gate else None,
                 _grad_like(dbias, dt_bias) if use_gate else None, None,
@@ -921,14 +971,20 @@ def _row_linear_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
             and weight.data_ptr() % 16 == 0)
 
 
+def _plain_dispatch() -> bool:
+    """True outside of tracing, functorch transforms, forward-mode and dispatch
+    or function modes."""
+    return not (torch.compiler.is_compiling() or torch.jit.is_tracing()
+                or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+                or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch.autograd.forward_ad._current_level >= 0)
+
+
 def _values_only(*tensors) -> bool:
     """True when a call on ``tensors`` computes plain values only: not traced,
     transformed (functorch, forward-mode), under a dispatch or function mode or
     autocast, and with no gradient to record."""
-    if torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing():
-        return False
-    if (torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
-            or torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0):
+    if torch.is_autocast_enabled("cuda") or not _plain_dispatch():
         return False
     if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
         return False

@@ -126,6 +126,38 @@ def _(q, k, v, g, beta, cu_seqlens, d_out, A_log, dt_bias, scale, lower_bound, u
             q.new_empty((heads * dim if use_gate else 0,), **f32))
 
 
+@torch.library.custom_op(f"{_LIB}::kda_chunk_bwd_packed", mutates_args=(), device_types="cuda")
+def kda_chunk_bwd_packed(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,
+                         beta: torch.Tensor, cu_seqlens: torch.Tensor, d_out: torch.Tensor,
+                         A_log: Optional[torch.Tensor], dt_bias: Optional[torch.Tensor], scale: float,
+                         lower_bound: float, use_qk_l2norm: bool, use_gate: bool, use_beta_sigmoid: bool,
+                         initial_state: Optional[torch.Tensor], d_final_state: Optional[torch.Tensor],
+                         cu_seqlens_cpu: Optional[torch.Tensor], recurrent: bool = False,
+                         grad_bf16: bool = False) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor,
+                                                           torch.Tensor, torch.Tensor]:
+    """``kda_chunk_bwd`` with dq, dk and dv as the parts of one [total, 3, H, 128] tensor."""
+    dq, _, _, *others = ops.kda_chunk_bwd(
+        q, k, v, g, beta, cu_seqlens, d_out, A_log=A_log, dt_bias=dt_bias, scale=scale, lower_bound=lower_bound,
+        use_qk_l2norm=use_qk_l2norm, use_gate=use_gate, use_beta_sigmoid=use_beta_sigmoid,
+        initial_state=initial_state, d_final_state=d_final_state, cu_seqlens_cpu=cu_seqlens_cpu,
+        recurrent=recurrent, grad_dtype=torch.bfloat16 if grad_bf16 else torch.float32, grad_packed=True)
+    total, heads, dim = dq.shape
+    return dq.as_strided((total, 3, heads, dim), (3 * heads * dim, heads * dim, dim, 1), 0), *others
+
+
+@kda_chunk_bwd_packed.register_fake
+def _(q, k, v, g, beta, cu_seqlens, d_out, A_log, dt_bias, scale, lower_bound, use_qk_l2norm,
+      use_gate, use_beta_sigmoid, initial_state, d_final_state, cu_seqlens_cpu, recurrent=False,
+      grad_bf16=False):
+    total, heads, dim = q.shape
+    n = cu_seqlens.shape[0] - 1
+    f32 = dict(dtype=torch.float32)
+    return (q.new_empty((total, 3, heads, dim), dtype=torch.bfloat16 if grad_bf16 else torch.float32),
+            q.new_empty((total, heads, dim), **f32), q.new_empty((total, heads), **f32),
+            q.new_empty((n, heads, dim, dim), **f32), q.new_empty((heads if use_gate else 0,), **f32),
+            q.new_empty((heads * dim if use_gate else 0,), **f32))
+
+
 @torch.library.custom_op(f"{_LIB}::kda_decode_step", mutates_args=("state",), device_types="cuda")
 def kda_decode_step(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,
                     beta: torch.Tensor, state: torch.Tensor, A_log: Optional[torch.Tensor],
@@ -235,5 +267,5 @@ torch.library.register_autograd(f"{_LIB}::gated_head_norm", _gated_head_norm_bac
                                 setup_context=_gated_head_norm_setup)
 
 
-__all__ = ["gated_head_norm", "gated_head_norm_bwd", "kda_chunk_bwd", "kda_chunk_fwd", "kda_decode_step",
+__all__ = ["gated_head_norm", "gated_head_norm_bwd", "kda_chunk_bwd", "kda_chunk_bwd_packed", "kda_chunk_fwd", "kda_decode_step",
            "short_conv", "short_conv_bwd", "short_conv_fwd", "short_conv_step"]

@@ -322,6 +322,32 @@ def test_bf16_gradients_are_the_fp32_gradients_rounded(recurrent):
         assert torch.equal(b16[i].view(torch.int32), f32[i].view(torch.int32)), f"d{name}"
     with pytest.raises(RuntimeError, match="grad_dtype"):
         ops.kda_chunk_bwd(*args, grad_dtype=torch.float16, **kw)
+    for dtype, want in ((torch.float32, f32), (torch.bfloat16, b16)):   # parts of one row: the same bits elsewhere
+        got = ops.kda_chunk_bwd(*args, grad_dtype=dtype, grad_packed=True, **kw)
+        assert ops._parts_of_rows(*got[:3])
+        for i in range(8):
+            assert torch.equal(got[i], want[i]), i
+
+
+def test_unbind_heads_backward():
+    """Gradients that are parts of one row come back as that row without a copy;
+    separate, missing, reordered, offset or batch-strided ones are stacked."""
+    x = torch.randn(2, 5, 3, 2, 128, requires_grad=True)
+    buf = torch.randn(2, 5, 3, 2, 128)
+    q, k, v = buf.unbind(2)
+    wide = torch.randn(2, 7, 3, 2, 128)[:, :5].unbind(2)
+    forms = {"row": (q, k, v), "separate": tuple(t.clone() for t in (q, k, v)), "reordered": (k, q, v),
+             "wide": wide, "heads apart": tuple(t.transpose(2, 3).contiguous().transpose(2, 3) for t in (q, k, v))}
+    for name, grads in forms.items():
+        got, = torch.autograd.grad(ops.UnbindHeads.apply(x), x, grads)
+        assert torch.equal(got, torch.stack(grads, 2)), name
+        assert (got.data_ptr() == buf.data_ptr()) == (name == "row"), name
+    outs = ops.UnbindHeads.apply(x)
+    got, = torch.autograd.grad([outs[0], outs[2]], x, [q, v])
+    assert torch.equal(got, torch.stack([q, torch.zeros_like(k), v], 2))
+    assert not ops._parts_of_rows(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2))
+    one = torch.randn(1, 1, 3, 2, 128).unbind(2)   # strides of single rows do not count
+    assert ops._parts_of_rows(*one)
 
 
 def test_chunk_bwd_matches_torch_autograd_restatement():

@@ -762,8 +762,18 @@ def chunk_kda(q, k, v, g, beta, *, scale=None, initial_state=None, output_final_
                                and initial_state.is_contiguous()) else initial_state.float().contiguous()
     ht = torch.empty((n, heads, HEAD_DIM, HEAD_DIM), dtype=torch.float32, device=q.device) \
         if output_final_state else None
-    # Through the sophia::kda_chunk_fwd custom op, so that torch.compile traces
-    # the call as one node.
+    # Plain values go straight to the kernels; else through the
+    # sophia::kda_chunk_fwd custom op, so that torch.compile, tracers and modes
+    # see the call as one node.  Its dispatch takes longer on the host than a
+    # short prompt's kernels on the GPU.
+    given = [t for t in (q, k, v, g, beta, cu, A_log, dt_bias, h0) if isinstance(t, torch.Tensor)]
+    if _values_only(*given) and all(t.device == q.device and t.is_cuda for t in given[:6]):
+        o = kda_chunk_fwd(flat(q, HEAD_DIM), flat(k, HEAD_DIM), flat(v, HEAD_DIM), flat(g, HEAD_DIM),
+                          beta.reshape(total, heads), cu, A_log=A_log, dt_bias=dt_bias, scale=scale, lower_bound=lb,
+                          use_qk_l2norm=bool(use_qk_l2norm_in_kernel), use_gate=bool(use_gate_in_kernel),
+                          use_beta_sigmoid=bool(use_beta_sigmoid_in_kernel), initial_state=h0, final_state=ht,
+                          cu_seqlens_cpu=cu_seqlens_cpu)
+        return o.view(bsz, seqlen, heads, HEAD_DIM), ht
     o = torch_ops.kda_chunk_fwd(
         flat(q, HEAD_DIM), flat(k, HEAD_DIM), flat(v, HEAD_DIM), flat(g, HEAD_DIM),
         beta.reshape(total, heads), cu, _detached(A_log), _detached(dt_bias),

@@ -228,3 +228,38 @@ def test_chunk_kda_state_v_first_is_the_transposed_state():
     (ops.chunk_kda(q, k, v, g, b, initial_state=a1, **kw)[0] * w).sum().backward()
     (ops.chunk_kda(q, k, v, g, b, initial_state=a2, state_v_first=True, **kw)[0] * w).sum().backward()
     assert torch.equal(a1.grad, a2.grad.transpose(-1, -2))
+
+
+def test_chunk_kda_direct_call_equals_the_custom_op():
+    """chunk_kda's direct call for plain values against the traced form's custom
+    op: the same bits with and without offsets, state and gate; on a host tensor,
+    under a dispatch mode and with a gradient it goes the way it went."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from sophia_amd import ops
+    dev = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(5)
+    T, H = 150, 2
+    q, k, v, z = (torch.randn(1, T, H, 128, generator=g).to(torch.bfloat16).to(dev) for _ in range(4))
+    beta = torch.randn(1, T, H, generator=g).to(torch.bfloat16).to(dev)
+    a, b = torch.randn(H, generator=g).to(dev), torch.randn(H * 128, generator=g).to(dev)
+    seen = []
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    flags = dict(use_qk_l2norm_in_kernel=True, use_gate_in_kernel=True, use_beta_sigmoid_in_kernel=True, safe_gate=True,
+                 A_log=a, dt_bias=b, output_final_state=True)
+    cu = torch.tensor([0, 40, 150], dtype=torch.int32)
+    for more in (dict(), dict(cu_seqlens=cu.to(dev)), dict(cu_seqlens=cu.to(dev), cu_seqlens_cpu=cu),
+                 dict(cu_seqlens=cu, initial_state=torch.randn(2, H, 128, 128, generator=g).to(dev))):
+        got = ops.chunk_kda(q, k, v, z, beta, **flags, **more)
+        with Mode():
+            want = ops.chunk_kda(q, k, v, z, beta, **flags, **more)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    assert any("kda_chunk_fwd" in name for name in seen)
+    with pytest.raises(RuntimeError):
+        ops.chunk_kda(*(t.cpu() for t in (q, k, v, z, beta)), **flags)
+    with pytest.raises(RuntimeError):
+        ops.chunk_kda(q, k, v.cpu(), z, beta, **flags)

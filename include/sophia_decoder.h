@@ -172,6 +172,16 @@ int sophia_causal_attention(const void *q, int64_t q_stride, const void *k, int6
                             int heads, int head_dim, float scale, int dtype, void *stream);
 
 /*
+ * Rows out[r] = parts[0][r] | parts[1][r] | ..., up to SOPHIA_JOIN_PARTS parts of
+ * any element type: the gradient of a mixer's fused projection from those of its
+ * parts.  widths and row_strides are in bytes, multiples of 16, parts and out
+ * 16-byte aligned; a NULL part is zeros.  out is dense and overlaps no part.
+ */
+#define SOPHIA_JOIN_PARTS 6
+int sophia_join_columns(const void *const *parts, const int64_t *row_strides, const int64_t *widths, int n_parts,
+                        void *out, int64_t rows, void *stream);
+
+/*
  * Projections of a few rows (a decode step's): y = x . w^T with x [rows, k],
  * w [n, k] and y [rows, n] in bf16 (RuntimeLinear.forward,
  * ml/runtime/model/runtime_linear.py:32-33, without a bias), fp32 sums rounded

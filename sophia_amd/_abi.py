@@ -79,6 +79,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "sophia_gated_head_norm_bwd_workspace_size": (_sz, [_i64, _i32, _i32]),
     "sophia_gated_head_norm_bwd": (_i32, [_vp, _i64, _vp, _i64, _i32, _vp, _i64, _vp, _f32, _vp, _i64,
                                           _vp, _i64, _vp, _i64, _i32, _i32, _i32, _vp, _sz, _vp]),
+    "sophia_join_columns": (_i32, [_vp, _vp, _vp, _i32, _vp, _i64, _vp]),
     "sophia_row_linear": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _vp]),
     "sophia_row_linear_situ_glu": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _f32, _f32, _vp]),
     "sophia_head_linear": (_i32, [_vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp, _i64, _i64, _i64, _i32, _i32, _i32,

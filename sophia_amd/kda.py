@@ -336,11 +336,14 @@ class SophiaKDA(nn.Module):
         y = ops.linear(x2, self._input_weight(x2.dtype))
         i, r, h = self.inner_dim, self.decay_rank, self.num_heads
         g = i if self.output_gate_full_rank else self.output_gate_rank
-        # One split, whose backward writes the gradient of y once; a slice per
-        # part would each write a whole zero-padded row set and add it up.
+        # One split, whose backward writes the gradient of y once (in one launch
+        # where it may); a slice per part would each write a whole zero-padded
+        # row set and add it up.
         sizes = [3 * i, g, r, h]
         pad = int(y.size(1)) - sum(sizes)
-        qkv, gate, dd, beta = y.split(sizes + [pad] if pad else sizes, 1)[:4]
+        sizes = sizes + [pad] if pad else sizes
+        split = _needs_grad(y) and ops._plain_dispatch()
+        qkv, gate, dd, beta = (ops.SplitColumns.apply(y, sizes) if split else y.split(sizes, 1))[:4]
         if not self.output_gate_full_rank:
             gate = self.output_gate_up(gate)
         return qkv, dd, beta, gate

@@ -16,6 +16,7 @@ FlashKDA seam (sm120_concurrent_ffn.py:375-423), so they drop into
 
 from __future__ import annotations
 
+import ctypes
 import torch
 
 from . import _native as nat
@@ -413,8 +414,9 @@ def kda_chunk_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Te
     in-kernel gate); ``grad_dtype=torch.bfloat16`` writes dq, dk and dv as
     bf16 instead (the fp32 gradients rounded to nearest even), the element
     type a bf16 forward's q, k, v carry; ``grad_packed`` returns dq, dk and dv
-    as the parts [:, 0], [:, 1], [:, 2] of one [total, 3, H, 128] buffer.  A host ``cu_seqlens`` (or ``cu_seqlens_cpu``) is checked
-    to rise from 0 to the token count.  The chunk form runs by default (bf16
+    as the parts [:, 0], [:, 1], [:, 2] of one [total, 3, H, 128] buffer.  A
+    host ``cu_seqlens`` (or ``cu_seqlens_cpu``) is checked to rise from 0 to the
+    token count.  The chunk form runs by default (bf16
     MFMA operands, fp32 accumulation and state, the forward's arithmetic);
     ``recurrent=True`` runs the per-token recurrence in fp32 instead.
     """
@@ -793,6 +795,43 @@ def _grad_like(grad: torch.Tensor, meta):
     if meta is None:
         return None
     return grad.view(meta[0]).to(meta[1])
+
+
+class SplitColumns(torch.autograd.Function):
+    """``y.split(sizes, 1)`` whose backward joins the parts' gradients in one
+    launch (sophia_join_columns), zeros where a part has none; types, strides or
+    widths that it does not take are concatenated."""
+
+    @staticmethod
+    def forward(ctx, y, sizes):
+        ctx.set_materialize_grads(False)
+        ctx.like = (int(y.size(0)), tuple(int(n) for n in sizes), y.dtype, y.device)
+        return y.split(sizes, 1)
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, *grads):
+        rows, sizes, dtype, device = ctx.like
+        if all(d is None for d in grads):
+            return None, None
+        size = dtype.itemsize
+        if (device.type == "cuda" and len(sizes) <= 6 and all(n * size % 16 == 0 for n in sizes) and _plain_dispatch()
+                and all(d is None or (type(d) is torch.Tensor and d.dtype == dtype and d.device == device
+                                      and d.stride(1) == 1 and d.data_ptr() % 16 == 0
+                                      and (rows <= 1 or (d.stride(0) >= n and d.stride(0) * size % 16 == 0)))
+                        for d, n in zip(grads, sizes))):
+            out = torch.empty((rows, sum(sizes)), dtype=dtype, device=device)
+            count = len(sizes)
+            rc = nat.lib().sophia_join_columns(
+                (ctypes.c_void_p * count)(*(None if d is None else d.data_ptr() for d in grads)),
+                (ctypes.c_int64 * count)(*(n * size if d is None or rows <= 1 else d.stride(0) * size
+                                           for d, n in zip(grads, sizes))),
+                (ctypes.c_int64 * count)(*(n * size for n in sizes)), count, out.data_ptr(), rows,
+                nat.stream_handle(device))
+            nat.check(rc, "sophia_join_columns")
+            return out, None
+        parts = [torch.zeros((rows, n), dtype=dtype, device=device) if d is None else d for d, n in zip(grads, sizes)]
+        return torch.cat(parts, 1), None
 
 
 def _parts_of_rows(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:

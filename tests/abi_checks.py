@@ -147,6 +147,15 @@ def check_host_side(lib, nat) -> None:
     assert rc == nat.SOPHIA_ERR_INVALID and "multiple of 16" in nat.last_error()
     rc = lib.sophia_row_linear_situ_glu(16, 64, 32, 64, 48, 16, 4, 16, 64, 0.0, 25.0, None)
     assert rc == nat.SOPHIA_ERR_INVALID and "soft caps" in nat.last_error()
+    # Decode steps and joined columns: sizes, strides and alignment before any launch.
+    rc = lib.sophia_kda_decode_mixer_step(16, 16, 16, 128, 16, 16, 16, 128, None, 16, 1, 16, 16, 0.1, -5.0, 7, 16, 1,
+                                          None, 1, 16, 128, 16, 1e-5, 1, 1, 64, 16, 128, None)
+    assert rc == nat.SOPHIA_ERR_INVALID and "head_dim" in nat.last_error()
+    rc = lib.sophia_kda_decode_mixer_step(16, 16, 16, 128, 16, 16, 24, 128, 16, 16, 1, 16, 16, 0.1, -5.0, 7, 16, 1,
+                                          None, 1, 16, 128, 16, 1e-5, 1, 1, 128, 16, 128, None)
+    assert rc == nat.SOPHIA_ERR_INVALID and "low-rank" in nat.last_error()
+    rc = lib.sophia_join_columns(None, None, None, 7, None, 1, None)
+    assert rc == nat.SOPHIA_ERR_INVALID and "parts" in nat.last_error()
     # Causal attention: bf16 and head_dim 128 only.
     rc = lib.sophia_causal_attention(16, 2048, 32, 2048, 48, 2048, 64, 2048, 80, None, 2, 100, 0, 64,
                                      16, 128, 0.08, 0, None)

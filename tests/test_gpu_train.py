@@ -236,3 +236,23 @@ def test_mixer_parameter_gradients_match_float64_autograd(seqlen):
     err_x = _rel(xd.grad, x64.grad)
     print(f"T={seqlen} dx: rel err {err_x:.2e} (worst parameter {worst:.2e})", flush=True)
     assert err_x <= TOL_MIXER
+
+
+@pytest.mark.parametrize("rows,sizes,dtype", [(1, [8], torch.bfloat16), (5, [24, 8, 16, 8], torch.bfloat16),
+                                              (70, [2048, 264, 8, 128, 16], torch.float32),
+                                              (9, [8, 12, 4], torch.bfloat16), (3, [8] * 7, torch.bfloat16)])
+def test_split_columns_backward_joins(rows, sizes, dtype):
+    """Gradients of the parts joined bit for bit: dense, slices of wider rows,
+    missing ones; widths off 16 bytes and too many parts are concatenated."""
+    from sophia_amd import ops
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    y = torch.randn(rows, sum(sizes), device="cuda").to(dtype).requires_grad_(True)
+    outs = ops.SplitColumns.apply(y, sizes)
+    assert all(torch.equal(a, b) for a, b in zip(outs, y.split(sizes, 1)))
+    wide = [torch.randn(rows, n + 16, device="cuda").to(dtype)[:, 8:8 + n] for n in sizes]
+    for grads in ([g.contiguous() for g in wide], wide, [g.t().contiguous().t() for g in wide]):
+        got, = torch.autograd.grad(outs, y, grads, retain_graph=True)
+        assert torch.equal(got, torch.cat(grads, 1))
+    got, = torch.autograd.grad(outs[0], y, wide[0])
+    assert torch.equal(got, torch.cat([wide[0]] + [torch.zeros_like(g) for g in wide[1:]], 1))

@@ -71,11 +71,6 @@ extern "C" {
  * (each the fp32 gradient rounded to nearest even), the element type a bf16
  * forward's q, k, v carry; dg, dbeta and the state gradients stay fp32. */
 #define SOPHIA_KDA_BWD_GRAD_BF16 32u
-/* Backward switch (sophia_kda_chunk_bwd): dq, dk and dv are the three parts of
- * one [total, 3, H, 128] buffer (dk = dq + H * 128 elements, dv = dk + H * 128),
- * the layout of the fused q | k | v rows, so that their gradient needs no
- * gathering copy. */
-#define SOPHIA_KDA_BWD_GRAD_PACKED 64u
 
 /* Message of the last failing call on this thread ("" if none). */
 const char *sophia_last_error(void);
@@ -328,8 +323,10 @@ int sophia_kda_conv_chunk_fwd(const void *x_q, const void *x_k, const void *x_v,
  *                     dtype SOPHIA_DTYPE_F32 or _BF16.
  *   d_final_state   : [n_seqs, H, 128, 128] fp32 gradient of the final states,
  *                     or NULL (zeros).
- * Outputs, fp32 (dq, dk, dv bf16 with SOPHIA_KDA_BWD_GRAD_BF16), dense (dq,
- * dk, dv interleaved with SOPHIA_KDA_BWD_GRAD_PACKED):
+ * Outputs, fp32 (dq, dk, dv bf16 with SOPHIA_KDA_BWD_GRAD_BF16), dense; or dq,
+ * dk and dv as the three parts of one [total, 3, H, 128] buffer, the layout of
+ * fused q | k | v rows: pointers with dk = dq + H * 128 and dv = dk + H * 128
+ * elements, which dense outputs of more than one row cannot have, say so.
  *   dq, dk, dv, dg  : [total, H, 128]   (dg with respect to the g input: the
  *                                        decay logits when the gate is applied
  *                                        in the kernel, else the log-decay)

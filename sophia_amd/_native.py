@@ -30,7 +30,6 @@ from ._abi import (  # noqa: F401
     SCAN_NO_SEGMENTS,
     BWD_RECURRENT,
     BWD_GRAD_BF16,
-    BWD_GRAD_PACKED,
 )
 
 _HERE = os.path.dirname(os.path.abspath(__file__))

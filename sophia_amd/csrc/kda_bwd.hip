@@ -705,12 +705,6 @@ extern "C" int sophia_kda_chunk_bwd(const void *q, const void *k, const void *v,
   SOPHIA_REQUIRE(cu_seqlens && workspace &&
                      (total_tokens == 0 || (q && k && v && g && beta && d_out && dq && dk && dv && dg && dbeta)),
                  "kda_chunk_bwd: NULL pointer");
-  if ((flags & SOPHIA_KDA_BWD_GRAD_PACKED) && total_tokens > 0) {
-    const size_t part = static_cast<size_t>(num_heads) * kD * ((flags & SOPHIA_KDA_BWD_GRAD_BF16) ? 2 : 4);
-    SOPHIA_REQUIRE(static_cast<uint8_t *>(dk) == static_cast<uint8_t *>(dq) + part &&
-                       static_cast<uint8_t *>(dv) == static_cast<uint8_t *>(dk) + part,
-                   "kda_chunk_bwd: packed dq, dk, dv must follow each other in one row");
-  }
   const bool gate = (flags & SOPHIA_KDA_GATE_IN_KERNEL) != 0;
   SOPHIA_REQUIRE(!gate || (A_log && dt_bias), "kda_chunk_bwd: gate in kernel needs A_log and dt_bias");
   SOPHIA_REQUIRE(gate || (!dA_log && !ddt_bias),
@@ -744,7 +738,11 @@ extern "C" int sophia_kda_chunk_bwd(const void *q, const void *k, const void *v,
   a.dht = d_final_state;
   a.dq = dq; a.dk = dk; a.dv = dv; a.dg = dg; a.dbeta = dbeta; a.dh0 = d_initial_state;
   a.grad_dtype = (flags & SOPHIA_KDA_BWD_GRAD_BF16) ? SOPHIA_DTYPE_BF16 : SOPHIA_DTYPE_F32;
-  a.grad_heads = (flags & SOPHIA_KDA_BWD_GRAD_PACKED) ? 3 * num_heads : num_heads;
+  // Parts of one row (dense buffers of more than one row would overlap there).
+  const uintptr_t part = static_cast<uintptr_t>(num_heads) * kD * (a.grad_dtype == SOPHIA_DTYPE_BF16 ? 2 : 4);
+  const uintptr_t q0 = reinterpret_cast<uintptr_t>(dq);
+  const bool packed = reinterpret_cast<uintptr_t>(dk) == q0 + part && reinterpret_cast<uintptr_t>(dv) == q0 + 2 * part;
+  a.grad_heads = packed ? 3 * num_heads : num_heads;
   a.dA_log = dA_log; a.ddt_bias = ddt_bias;
   a.qh = carve(tok * kD * 4);
   a.kh = carve(tok * kD * 4);

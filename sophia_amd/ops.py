@@ -479,8 +479,7 @@ def kda_chunk_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Te
         nat.dtype_code(g.dtype), nat.ptr(beta), bs, nat.dtype_code(beta.dtype), nat.ptr(a_log),
         nat.ptr(dtb), float(scale), float(lower_bound),
         _flags(use_qk_l2norm, use_gate, use_beta_sigmoid) | (nat.BWD_RECURRENT if recurrent else 0)
-        | (nat.BWD_GRAD_BF16 if grad_dtype == torch.bfloat16 else 0)
-        | (nat.BWD_GRAD_PACKED if grad_packed else 0),
+        | (nat.BWD_GRAD_BF16 if grad_dtype == torch.bfloat16 else 0),
         nat.ptr(cu), n, total, heads, HEAD_DIM,
         nat.ptr(initial_state), nat.ptr(d_out), ds, nat.dtype_code(d_out.dtype),
         nat.ptr(d_final_state), nat.ptr(dq), nat.ptr(dk), nat.ptr(dv), nat.ptr(dg),

@@ -548,11 +548,11 @@ class SophiaKDA(nn.Module):
         if n_decode > 0 and not fused_decode:
             ops.short_conv_step(qkv[n_prefill:], conv_w, conv_state, state_slots=decode_slots,
                                 read_history=True, out=conv_out[n_prefill:], weight_rounded=True)
-        if n_prefill == 0 and fused_decode and ops.decode_mixer_takes(
+        if n_prefill == 0 and fused_decode and plain_linear(self.decay_up) and ops.decode_mixer_takes(
                 qkv, dd, beta_logits, gate_logits, self.decay_up.weight, self.output_norm.weight):
             # Decode rows alone: the step's launch also ends with the output norm
             # and gate and, for few rows, begins with decay_up.
-            own = plain_linear(self.decay_up) and ops.decay_in_step(dd, self.decay_up.weight)
+            own = ops.decay_in_step(dd, self.decay_up.weight)
             return self.o_proj(ops.kda_decode_mixer_step(
                 qkv, conv_w, conv_state, dd if own else self.decay_up(dd).view(n, h, d), beta_logits,
                 self.recurrent_state, gate_logits, self.output_norm.weight, A_log=self.A_log, dt_bias=self.dt_bias,

@@ -221,3 +221,38 @@ def test_mixer_with_trained_parameter_values_matches_oracle():
     err_s = _rel(_np(mod.recurrent_state[:1]), cache["recurrent"])
     print(f"trained-value mixer: output {err_y:.2e}, state {err_s:.2e}")
     assert err_y < REL_TOL and err_s < REL_TOL
+
+
+@pytest.mark.parametrize("rows", [3, 40])
+def test_decode_rows_with_another_decay_module(rows):
+    """Decode rows run in one launch with the module's own decay_up; one with a
+    hook or another module in its place is called, with the same results."""
+    from sophia_amd.config import ModelArgs
+    from sophia_amd.kda import RuntimeLinear, SophiaKDA
+    torch.manual_seed(rows)
+    with torch.device("cuda"):
+        m = SophiaKDA(ModelArgs(use_cache=True, max_batch_size=rows))
+    for mod in m.modules():
+        if isinstance(mod, RuntimeLinear):
+            mod.weight.data = mod.weight.data.to(torch.bfloat16)
+    x = torch.randn(rows, m.dim, device="cuda", dtype=torch.bfloat16)
+    slots = torch.arange(rows, dtype=torch.int32, device="cuda")
+    cu = torch.zeros(1, dtype=torch.int32, device="cuda")
+    state, conv = torch.randn_like(m.recurrent_state) * 0.1, torch.randn_like(m.conv_state)
+
+    def step():
+        m.recurrent_state.copy_(state)
+        m.conv_state.copy_(conv)
+        with torch.no_grad():
+            return m.forward_mixed(x, 0, cu, None, slots).float(), m.recurrent_state.clone()
+
+    y, s = step()
+    calls = []
+    handle = m.decay_up.register_forward_hook(lambda *a: calls.append(1))
+    yh, sh = step()
+    handle.remove()
+    m.decay_up = torch.nn.Sequential(m.decay_up)
+    yr, sr = step()
+    assert len(calls) == 1
+    for got, want in ((yh, y), (yr, y), (sh, s), (sr, s)):
+        assert float((got - want).norm()) <= 1e-2 * float(want.norm())

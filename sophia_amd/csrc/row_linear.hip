@@ -6,10 +6,10 @@
 // 16-byte pieces, up to eight MFMA k-steps before any is used, so that all
 // of a work-group's weight bytes (48 KB at k = 1,536) are in flight at once, and the
 // partial 16 x 16 tiles are summed over the wavefronts in order through LDS.
-// A library GEMM of these shapes walks k in LDS tiles.  us per call at 8 rows,
-// weights from HBM, library -> this: 1,536 x 3,968 15.2 -> 8.1, 1,536 x 2,048 8.2 ->
-// 5.2, 2,560 x 1,536 7.2 -> 5.1, 7,936 x 1,536 10.7 -> 8.8 (with its activation, 15.7
-// -> 9.4), 2,048 x 128 3.4 -> 3.1.
+// A library GEMM of these shapes walks k in LDS tiles.  us per call at 16 rows,
+// weights from HBM, library -> this: 1,536 x 3,968 19.5 -> 10.7, 2,560 x 1,536 9.4 ->
+// 5.9, 7,936 x 1,536 11.9 -> 9.6; at 8 rows, in half tiles, 19.3 -> 6.8, 9.4 -> 5.2,
+// 11.9 -> 8.1 and 8,384 x 1,536 12.7 -> 8.5.
 //
 // The tile is W . x^T on v_mfma_f32_16x16x32_bf16 (A = 16 weight rows, B = 16
 // rows of x; lanes of rows past the last read the last row, unused): a lane
@@ -28,8 +28,8 @@
 // steps.  A load then takes whole 128-byte lines of eight weight rows instead of
 // half lines of sixteen, x is loaded half as often, and there are twice the
 // tiles to spread over the chip (1,536 outputs are 96 tiles of 16 on 256 CUs).
-// us per call, weights from HBM, whole tiles or library -> half: 1,536 x 3,968 7.9 ->
-// 6.0, 7,936 x 1,536 with its activation 9.2 -> 7.6, 8,384 x 1,536 12.1 -> 7.5, 2,048 x 384
+// us per call in a loop of launches, whole tiles -> half: 1,536 x 3,968 7.9 -> 6.0,
+// 7,936 x 1,536 with its activation 9.2 -> 7.6, 8,384 x 1,536 14.0 -> 7.5, 2,048 x 384
 // 3.8 -> 2.4.
 #include "common.hpp"
 #include "situ.hpp"

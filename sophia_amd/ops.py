@@ -1008,11 +1008,13 @@ def _row_linear_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
     to 512 tiles of outputs (16 rows: 7,936 11.9 and 9.6, but 8,384 12.8 and 14.0):
     past two tiles per CU each work-group's reads of x weigh as much as the
     weight's."""
-    if not _values_only(x, weight):   # (first: a wrapped tensor has no pointer to look at)
-        return False
     k = x.shape[-1]
+    if torch.compiler.is_compiling() or x.numel() > ROW_LINEAR_MAX * k:   # (first: most other calls end here)
+        return False
+    if not _values_only(x, weight):   # (before any look at a pointer: a wrapped tensor has none)
+        return False
     if (x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or x.device.type != "cuda"
-            or weight.device != x.device or x.numel() > ROW_LINEAR_MAX * k or x.numel() == 0
+            or weight.device != x.device or x.numel() == 0
             or k % 32 or weight.shape[0] % 16 or (weight.shape[0] > 512 * 16 and x.numel() > 8 * k)):
         return False
     return (weight.is_contiguous() and x.stride(-1) == 1 and x.data_ptr() % 16 == 0

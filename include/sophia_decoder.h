@@ -217,6 +217,14 @@ int sophia_head_linear(const void *x, int64_t x_row_stride, int64_t x_head_strid
                        int64_t y_row_stride, int64_t y_head_stride, const void *gate, int64_t gate_row_stride,
                        int64_t gate_head_stride, int64_t rows, int heads, int n, int k, void *stream);
 
+/*
+ * sophia_head_linear without a gate of head blocks w [heads, k, n] (contiguous):
+ * y[r, h, :] = x[r, h, :] . w[h], k_up's blocks as its weight holds them.
+ */
+int sophia_head_linear_kn(const void *x, int64_t x_row_stride, int64_t x_head_stride, const void *w, void *y,
+                          int64_t y_row_stride, int64_t y_head_stride, int64_t rows, int heads, int n, int k,
+                          void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -83,6 +83,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "sophia_row_linear_situ_glu": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _f32, _f32, _vp]),
     "sophia_head_linear": (_i32, [_vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp, _i64, _i64, _i64, _i32, _i32, _i32,
                                   _vp]),
+    "sophia_head_linear_kn": (_i32, [_vp, _i64, _i64, _vp, _vp, _i64, _i64, _i64, _i32, _i32, _i32, _vp]),
     "sophia_mla_decode_workspace_size": (_sz, [_i64, _i32, _i32]),
     "sophia_causal_attention": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _i32,
                                        _i64, _i64, _i32, _i32, _i32, _f32, _i32, _vp]),

@@ -163,6 +163,13 @@ __device__ __forceinline__ float wave_sum_dpp(float v) {
   return v + dpp_rotate<0x121>(v);
 }
 
+// Transposing LDS read: the 16 lanes of a group read four rows of 16 elements
+// (lane j: row j / 4, elements 4 (j % 4) .. + 3) and lane j gets column j.
+__device__ __forceinline__ u2 lds_read_tr(const uint16_t *p) {
+  return __builtin_bit_cast(u2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                    (__attribute__((address_space(3))) s4 *)(p)));
+}
+
 // Butterfly sum over the whole 64-lane wavefront.
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll

@@ -932,13 +932,6 @@ __device__ __forceinline__ f16v mfma32x32(const bf8 &a, const bf8 &b, const f16v
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
-// Transposing LDS read: the 16 lanes of a group read four rows of 16 elements
-// (lane j: row j / 4, elements 4 (j % 4) .. + 3) and lane j gets column j.
-__device__ __forceinline__ u2 lds_read_tr(const uint16_t *p) {
-  return __builtin_bit_cast(u2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                    (__attribute__((address_space(3))) s4 *)(p)));
-}
-
 // NARROW: 64 rows of k and v span less than 2 GiB, so that a lane's byte offsets
 // within a block are 32-bit constants added to a scalar base (64-bit products
 // per row and block took a quarter of the vector instructions).

@@ -224,6 +224,13 @@ int dispatch(const RowLinearArgs &a, hipStream_t st) {
 // transposing copies around it (4.6 us each).  With a gate the output is
 // multiplied by its sigmoid (attention.py:655-656), rounded to bf16 before and
 // after as two launches round it: a launch of 4.5 us less.
+//
+// KN: w[h] lies as [k, n], k_up's block as its weight holds it (the product
+// contracts over the head's rows).  128 of its rows at a time go to LDS as whole
+// lines and come back by transposing reads, four of a column per lane: the same
+// operands, steps and sums as over a transposed copy, no copy to keep in step
+// with the weight, and whole lines of it (16 heads x 128 x 128 in a loop of
+// launches: 8 rows 4.2 us over the copy, 2.4 here; 1,024 rows 16.1 and 6.8).
 struct HeadLinearArgs {
   const uint16_t *x;
   int64_t x_row, x_head;
@@ -236,34 +243,74 @@ struct HeadLinearArgs {
 };
 
 constexpr int kHlWaves = 8;
+constexpr int kHlCols = 16 * kHlWaves;   // outputs of a work-group
+constexpr int kHlK = 128;                // KN: rows of w in LDS at a time
+constexpr int kHlLd = kHlCols + 8;       // bf16 row stride there
 
+// KN: rows k0 .. k0 + kHlK - 1 of w[h] (past the last: the last again, unused),
+// the columns of this work-group (past the last: the last again, unused).
+__device__ __forceinline__ void stage_head_rows(const HeadLinearArgs &a, int h, int col0, int k0, uint16_t *s_w) {
+  constexpr int kChunks = kHlCols / 8, kRows = kHlWaves * 64 / kChunks;   // 16-byte chunks of a row, rows at a time
+  const int c = threadIdx.x % kChunks, r = threadIdx.x / kChunks;
+  const int64_t k = 32 * static_cast<int64_t>(a.ksteps);
+  const uint16_t *wp = a.w + static_cast<int64_t>(h) * k * a.n + min(col0 + 8 * c, a.n - 8);
+  u4 v[kHlK / kRows];
+#pragma unroll
+  for (int i = 0; i < kHlK / kRows; ++i)
+    v[i] = *reinterpret_cast<const u4 *>(wp + imin64(k0 + r + i * kRows, k - 1) * a.n);
+#pragma unroll
+  for (int i = 0; i < kHlK / kRows; ++i) *reinterpret_cast<u4 *>(s_w + (r + i * kRows) * kHlLd + 8 * c) = v[i];
+}
+
+template <bool KN>
 __global__ __launch_bounds__(kHlWaves * 64) void head_linear_kernel(HeadLinearArgs a) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ln = lane & 15, g = lane >> 4;
-  const int h = blockIdx.y, n0 = 16 * (blockIdx.z * kHlWaves + wave);
-  if (n0 >= a.n) return;   // wave-uniform; no barrier below
+  const int h = blockIdx.y, n0 = kHlCols * blockIdx.z + 16 * wave;
+  if (!KN && n0 >= a.n) return;   // wave-uniform; no barrier below
   const int row = blockIdx.x * 16 + ln;
-  const int64_t k = 32 * static_cast<int64_t>(a.ksteps);
-  const uint16_t *wp = a.w + (static_cast<int64_t>(h) * a.n + n0 + ln) * k + 8 * g;
   const uint16_t *xp = a.x + min(row, a.rows - 1) * a.x_row + h * a.x_head + 8 * g;
   u2 gate = u2{0, 0};
-  if (a.gate)   // uniform
+  if (a.gate && n0 < a.n)   // uniform
     gate = *reinterpret_cast<const u2 *>(a.gate + min(row, a.rows - 1) * a.gate_row + h * a.gate_head + n0 + 4 * g);
   f4 acc = f4{0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < a.ksteps; s += kHlBatch) {
-    u4 wr[kHlBatch], xr[kHlBatch];
+  if constexpr (KN) {
+    __shared__ __attribute__((aligned(16))) uint16_t s_w[kHlK * kHlLd];
+    // rows 8 g + ln / 4 of a step (and four on) at this wavefront's columns: A's lane (output ln, k 8 g ..)
+    const uint16_t *sp = s_w + (8 * g + (ln >> 2)) * kHlLd + 16 * wave + 4 * (ln & 3);
+    constexpr int kSteps = kHlK / 32;
+    for (int s = 0; s < a.ksteps; s += kSteps) {
+      u4 xr[kSteps];
 #pragma unroll
-    for (int i = 0; i < kHlBatch; ++i) {
-      const int at = 32 * min(s + i, a.ksteps - 1);
-      wr[i] = *reinterpret_cast<const u4 *>(wp + at);
-      xr[i] = *reinterpret_cast<const u4 *>(xp + at);
+      for (int i = 0; i < kSteps; ++i) xr[i] = *reinterpret_cast<const u4 *>(xp + 32 * min(s + i, a.ksteps - 1));
+      if (s > 0) __syncthreads();   // the rows before are read
+      stage_head_rows(a, h, kHlCols * blockIdx.z, 32 * s, s_w);
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < kSteps; ++i) {
+        if (s + i >= a.ksteps) break;   // uniform
+        const u2 lo = lds_read_tr(sp + 32 * i * kHlLd), hi = lds_read_tr(sp + (32 * i + 4) * kHlLd);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf8(u4{lo.x, lo.y, hi.x, hi.y}), as_bf8(xr[i]), acc, 0, 0, 0);
+      }
     }
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
+    if (n0 >= a.n) return;   // (after the last barrier)
+  } else {
+    const uint16_t *wp = a.w + (static_cast<int64_t>(h) * a.n + n0 + ln) * (32 * static_cast<int64_t>(a.ksteps)) + 8 * g;
+    for (int s = 0; s < a.ksteps; s += kHlBatch) {
+      u4 wr[kHlBatch], xr[kHlBatch];
 #pragma unroll
-    for (int i = 0; i < kHlBatch; ++i) {
-      if (s + i >= a.ksteps) break;
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf8(wr[i]), as_bf8(xr[i]), acc, 0, 0, 0);
+      for (int i = 0; i < kHlBatch; ++i) {
+        const int at = 32 * min(s + i, a.ksteps - 1);
+        wr[i] = *reinterpret_cast<const u4 *>(wp + at);
+        xr[i] = *reinterpret_cast<const u4 *>(xp + at);
+      }
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < kHlBatch; ++i) {
+        if (s + i >= a.ksteps) break;
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf8(wr[i]), as_bf8(xr[i]), acc, 0, 0, 0);
+      }
     }
   }
   if (a.gate) {
@@ -324,10 +371,11 @@ extern "C" int sophia_row_linear_situ_glu(const void *x, int64_t x_stride, const
   return dispatch<true, false>(a, static_cast<hipStream_t>(stream));
 }
 
-extern "C" int sophia_head_linear(const void *x, int64_t x_row_stride, int64_t x_head_stride, const void *w, void *y,
-                                  int64_t y_row_stride, int64_t y_head_stride, const void *gate,
-                                  int64_t gate_row_stride, int64_t gate_head_stride, int64_t rows, int heads, int n, int k,
-                                  void *stream) {
+namespace {
+template <bool KN>
+int head_linear(const void *x, int64_t x_row_stride, int64_t x_head_stride, const void *w, void *y, int64_t y_row_stride,
+                int64_t y_head_stride, const void *gate, int64_t gate_row_stride, int64_t gate_head_stride, int64_t rows,
+                int heads, int n, int k, void *stream) {
   SOPHIA_REQUIRE(rows >= 0 && rows <= 0x7fffffff && heads > 0 && heads <= 65535, "head_linear: bad rows / heads");
   SOPHIA_REQUIRE(k > 0 && k % 32 == 0 && n > 0 && n % 16 == 0 && (n + 127) / 128 <= 65535,
                  "head_linear: k must be a positive multiple of 32 and n of 16");
@@ -349,6 +397,22 @@ extern "C" int sophia_head_linear(const void *x, int64_t x_row_stride, int64_t x
                          gate_row_stride, gate_head_stride, static_cast<int>(rows), n, k / 32};
   const dim3 grid(static_cast<unsigned>((rows + 15) / 16), static_cast<unsigned>(heads),
                   static_cast<unsigned>((n + 127) / 128));
-  hipLaunchKernelGGL(head_linear_kernel, grid, dim3(kHlWaves * 64), 0, static_cast<hipStream_t>(stream), a);
+  hipLaunchKernelGGL(head_linear_kernel<KN>, grid, dim3(kHlWaves * 64), 0, static_cast<hipStream_t>(stream), a);
   return check_launch("head_linear");
+}
+}  // namespace
+
+extern "C" int sophia_head_linear(const void *x, int64_t x_row_stride, int64_t x_head_stride, const void *w, void *y,
+                                  int64_t y_row_stride, int64_t y_head_stride, const void *gate,
+                                  int64_t gate_row_stride, int64_t gate_head_stride, int64_t rows, int heads, int n, int k,
+                                  void *stream) {
+  return head_linear<false>(x, x_row_stride, x_head_stride, w, y, y_row_stride, y_head_stride, gate, gate_row_stride,
+                            gate_head_stride, rows, heads, n, k, stream);
+}
+
+extern "C" int sophia_head_linear_kn(const void *x, int64_t x_row_stride, int64_t x_head_stride, const void *w, void *y,
+                                     int64_t y_row_stride, int64_t y_head_stride, int64_t rows, int heads, int n, int k,
+                                     void *stream) {
+  return head_linear<true>(x, x_row_stride, x_head_stride, w, y, y_row_stride, y_head_stride, nullptr, n,
+                           static_cast<int64_t>(heads) * n, rows, heads, n, k, stream);
 }

@@ -64,8 +64,6 @@ class SophiaMLA(nn.Module):
             int(args.max_batch_size), int(args.max_seq_len), self.kv_rank), persistent=False)
         self._v_t = None
         self._v_t_key = None
-        self._k_t = None
-        self._k_t_key = None
         self._in_w = None
         self._in_w_key = None
 
@@ -96,18 +94,6 @@ class SophiaMLA(nn.Module):
             self._v_t = w.detach().view(h, d, r).to(dtype).transpose(1, 2).contiguous()
             self._v_t_key = key
         return self._v_t
-
-    def _k_up_t(self, dtype: torch.dtype) -> torch.Tensor:
-        """k_up's weight as [heads, kv_rank, head_dim] (the per-head blocks
-        transposed), as the decode rows' key product takes it; kept until the
-        weight changes."""
-        w = self.k_up.weight
-        h, d, r = self.num_heads, self.head_dim, self.kv_rank
-        key = (w.data_ptr(), w._version, w.dtype, dtype)
-        if self._k_t_key != key:
-            self._k_t = w.detach().view(h, d, r).to(dtype).transpose(1, 2).contiguous()
-            self._k_t_key = key
-        return self._k_t
 
     # ------------------------------------------------------------- caches
     def ensure_batch_capacity(self, batch_size: int) -> None:
@@ -349,23 +335,25 @@ class SophiaMLA(nn.Module):
                          cu_k=cu_k, cu_host=step["cu_prefill_host"], cu_k_host=cu_k_host)
         if nd > 0:
             # the per-head products on the head kernel where only their values
-            # are asked for (bf16 weights, whole MFMA steps), else batched GEMMs
-            heads_kernel = (x.dtype == torch.bfloat16 and r % 32 == 0 and d % 32 == 0
-                            and self.v_up.weight.dtype == torch.bfloat16 and self.v_up.weight.is_contiguous()
-                            and q.stride(0) % 8 == 0
-                            and ops._values_only(q, self.k_up.weight, self.v_up.weight))
+            # are asked for (bf16 weights, whole MFMA steps), else batched GEMMs.
+            # It reads both weights as they lie: an edit of them in place, by
+            # whatever means, is seen by the next step and by replays.
+            w_k, w_v = self.k_up.weight, self.v_up.weight
+            heads_kernel = (x.dtype == torch.bfloat16 and r % 32 == 0 and d % 32 == 0 and q.stride(0) % 8 == 0
+                            and all(w.dtype == torch.bfloat16 and w.is_contiguous() for w in (w_k, w_v))
+                            and ops._values_only(q, w_k, w_v))
             if heads_kernel:
-                qa = ops.head_linear(q[npre:], self._k_up_t(x.dtype))                       # [D, h, r]
+                qa = ops.head_linear(q[npre:], w_k.view(h, d, r), weight_kn=True)           # [D, h, r]
             else:
-                w_k = self.k_up.weight.view(h, d, r).to(x.dtype)
-                qa = torch.bmm(q[npre:].transpose(0, 1).contiguous(), w_k).transpose(0, 1)   # [D, h, r]
+                qa = torch.bmm(q[npre:].transpose(0, 1).contiguous(),
+                               w_k.view(h, d, r).to(x.dtype)).transpose(0, 1)               # [D, h, r]
             # softmax over cached latents 0..pos and their weighted sum, one kernel
             ctx = ops.mla_decode_attn(qa.contiguous(), cache, step["decode_slots"], step["decode_pos"],
                                       d ** -0.5, max_len=int(step["max_decode_len"]))   # [D, h, r]
             if heads_kernel:
                 # decode rows alone: the output gate on the products as they are formed
                 own = npre == 0 and gate.dtype == x.dtype and gate.stride(0) % 4 == 0 and gate.data_ptr() % 8 == 0 and ops._values_only(gate)
-                ops.head_linear(ctx, self.v_up.weight.view(h, d, r), out=out[npre:],
+                ops.head_linear(ctx, w_v.view(h, d, r), out=out[npre:],
                                 gate=gate.unflatten(1, (h, d)) if own else None)
                 if own:
                     return self.o_proj(out.view(n, self.inner_dim))

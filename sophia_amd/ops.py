@@ -1085,19 +1085,24 @@ def row_linear_situ_glu(x: torch.Tensor, weight: torch.Tensor, gate_softcap: flo
 
 
 def head_linear(x: torch.Tensor, weight: torch.Tensor, *, out: torch.Tensor | None = None,
-                gate: torch.Tensor | None = None) -> torch.Tensor:
+                gate: torch.Tensor | None = None, weight_kn: bool = False) -> torch.Tensor:
     """Per-head projection (sophia_head_linear): out[r, h] = x[r, h] . weight[h]^T
     in bf16, x [rows, heads, k] with dense last dim, weight [heads, n, k]
     contiguous, k a multiple of 32, n of 16.  Returns [rows, heads, n] (or
     ``out``, whose rows and heads may be strided); with ``gate`` (bf16 logits
-    [rows, heads, n]) times its sigmoid, as ``gated_head_norm`` of the result."""
+    [rows, heads, n]) times its sigmoid, as ``gated_head_norm`` of the result.
+    ``weight_kn``: weight is [heads, k, n] (sophia_head_linear_kn; no gate)."""
     _gpu(x, "x")
     _gpu(weight, "weight")
     rows, heads, k = (int(v) for v in x.shape)
-    n = int(weight.size(1))
-    if tuple(weight.shape) != (heads, n, k) or not weight.is_contiguous() or x.stride(2) != 1 \
-            or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or weight.device != x.device:
-        raise RuntimeError(f"head_linear takes bf16 x [rows, {heads}, {k}] and contiguous weight [{heads}, n, {k}]")
+    n = int(weight.size(2 if weight_kn else 1))
+    if tuple(weight.shape) != ((heads, k, n) if weight_kn else (heads, n, k)) or not weight.is_contiguous() \
+            or x.stride(2) != 1 or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 \
+            or weight.device != x.device:
+        form = f"[{heads}, {k}, n]" if weight_kn else f"[{heads}, n, {k}]"
+        raise RuntimeError(f"head_linear takes bf16 x [rows, {heads}, {k}] and contiguous weight {form}")
+    if weight_kn and gate is not None:
+        raise RuntimeError("head_linear takes no gate with weight_kn")
     y = out if out is not None else torch.empty((rows, heads, n), dtype=x.dtype, device=x.device)
     if y.dtype != x.dtype or tuple(y.shape) != (rows, heads, n) or y.stride(2) != 1 or y.device != x.device:
         raise RuntimeError(f"out must be bf16 [{rows}, {heads}, {n}]")
@@ -1106,12 +1111,17 @@ def head_linear(x: torch.Tensor, weight: torch.Tensor, *, out: torch.Tensor | No
         raise RuntimeError(f"gate must be bf16 [{rows}, {heads}, {n}]")
     xh = x.stride(1) if heads > 1 else k
     yh = y.stride(1) if heads > 1 else n
+    xr = x.stride(0) if rows > 1 else (heads - 1) * xh + k
+    yr = y.stride(0) if rows > 1 else (heads - 1) * yh + n
+    if weight_kn:
+        rc = nat.lib().sophia_head_linear_kn(x.data_ptr(), xr, xh, weight.data_ptr(), y.data_ptr(), yr, yh, rows, heads,
+                                             n, k, nat.stream_handle(x.device))
+        nat.check(rc, "sophia_head_linear_kn")
+        return y
     gh = n if gate is None or heads == 1 else gate.stride(1)
     gr = gate.stride(0) if gate is not None and rows > 1 else (heads - 1) * gh + n
-    rc = nat.lib().sophia_head_linear(
-        x.data_ptr(), x.stride(0) if rows > 1 else (heads - 1) * xh + k, xh, weight.data_ptr(), y.data_ptr(),
-        y.stride(0) if rows > 1 else (heads - 1) * yh + n, yh, nat.ptr(gate), gr, gh, rows, heads, n, k,
-        nat.stream_handle(x.device))
+    rc = nat.lib().sophia_head_linear(x.data_ptr(), xr, xh, weight.data_ptr(), y.data_ptr(), yr, yh, nat.ptr(gate), gr,
+                                      gh, rows, heads, n, k, nat.stream_handle(x.device))
     nat.check(rc, "sophia_head_linear")
     return y
 

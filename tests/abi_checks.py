@@ -147,6 +147,10 @@ def check_host_side(lib, nat) -> None:
     assert rc == nat.SOPHIA_ERR_INVALID and "multiple of 16" in nat.last_error()
     rc = lib.sophia_row_linear_situ_glu(16, 64, 32, 64, 48, 16, 4, 16, 64, 0.0, 25.0, None)
     assert rc == nat.SOPHIA_ERR_INVALID and "soft caps" in nat.last_error()
+    rc = lib.sophia_head_linear_kn(16, 256, 128, 24, 48, 256, 128, 4, 2, 128, 128, None)
+    assert rc == nat.SOPHIA_ERR_INVALID and "aligned" in nat.last_error()
+    rc = lib.sophia_head_linear_kn(16, 256, 128, 32, 48, 256, 128, 4, 2, 128, 48, None)
+    assert rc == nat.SOPHIA_ERR_INVALID and "multiple of 32" in nat.last_error()
     # Decode steps and joined columns: sizes, strides and alignment before any launch.
     rc = lib.sophia_kda_decode_mixer_step(16, 16, 16, 128, 16, 16, 16, 128, None, 16, 1, 16, 16, 0.1, -5.0, 7, 16, 1,
                                           None, 1, 16, 128, 16, 1e-5, 1, 1, 64, 16, 128, None)

@@ -251,6 +251,55 @@ def test_mixed_step_graph_replays_match_eager():
             model(torch.zeros(1, 3, dtype=torch.long, device=dev), start_pos=0)
 
 
+def _mla_decode(dev, rows=5, **kw):
+    """An MLA layer with bf16 weights, a filled latent cache, and a decode-only step."""
+    from sophia_amd.config import ModelArgs
+    from sophia_amd.decoder import SophiaMLA
+    from sophia_amd.kda import RuntimeLinear
+    torch.manual_seed(11)
+    with torch.device(dev):
+        m = SophiaMLA(ModelArgs(dim=256, num_heads=2, mla_q_rank=64, mla_kv_rank=32, max_seq_len=40,
+                                max_batch_size=rows, **kw))
+    for mod in m.modules():
+        if isinstance(mod, RuntimeLinear):
+            mod.weight.data = mod.weight.data.mul_(4).to(torch.bfloat16)
+    m.latent_cache.normal_()
+    x = torch.randn(rows, 256, device=dev).to(torch.bfloat16)
+    step = dict(n_prefill_rows=0, rectangular=False, decode_slots=torch.arange(rows, dtype=torch.int32, device=dev),
+                decode_pos=torch.arange(10, 10 + rows, device=dev), max_decode_len=40)
+    return m, x, step
+
+
+def test_mla_decode_rows_see_up_weights_edited_in_place():
+    """k_up and v_up edited through ``.data`` (no version count) after a step and
+    after a capture: the next eager step and the replays use the edited weights."""
+    dev = _dev()
+    m, x, step = _mla_decode(dev)
+    with torch.no_grad():
+        first = m.forward_mixed(x, step).clone()
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            m.forward_mixed(x, step)
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = m.forward_mixed(x, step)
+        for lin, factor in ((m.k_up, -3.0), (m.v_up, 2.0)):
+            lin.weight.data.mul_(factor)
+            other, _, _ = _mla_decode(dev)
+            other.load_state_dict(m.state_dict())
+            other.latent_cache.copy_(m.latent_cache)
+            for mod, src in ((other.k_up, m.k_up), (other.v_up, m.v_up)):
+                mod.weight.data = src.weight.data.clone()
+            want = other.forward_mixed(x, step)
+            assert not torch.equal(want, first)
+            assert torch.equal(m.forward_mixed(x, step), want)
+            for _ in range(2):
+                graph.replay()
+                assert torch.equal(out, want)
+
+
 FULL_DIMS = dict(vocab_size=1024, n_layers=4, ffn_hidden=3968, mla_q_rank=384, mla_kv_rank=128,
                  dim=1536, num_heads=16, max_seq_len=256, max_batch_size=4)
 

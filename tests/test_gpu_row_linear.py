@@ -161,3 +161,22 @@ def test_head_linear_matches_float64(rows, heads, n, k):
         ops.head_linear(wide.to(dev)[:, :, 8:].float(), w.to(dev))
     with pytest.raises(RuntimeError):
         ops.head_linear(wide.to(dev)[:, :, 8:], w.to(dev), gate=gate.float())
+
+
+@pytest.mark.parametrize("rows,heads,n,k", [(1, 1, 16, 32), (8, 16, 128, 128), (17, 3, 144, 96), (5, 2, 32, 320),
+                                            (33, 2, 272, 256)])
+def test_head_linear_of_rows_first_weights_equals_the_transposed_copy(rows, heads, n, k):
+    """weight_kn takes w [heads, k, n] as it lies: bit for bit head_linear of its
+    transposed copy (the same operands in the same steps), with outputs and rows
+    that end inside a tile, k short of, at and past the rows held in LDS."""
+    from sophia_amd import ops
+    dev = _dev()
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, heads, k + 8, generator=g).to(torch.bfloat16).to(dev)[:, :, 8:]
+    w = (torch.randn(heads, k, n, generator=g) * k ** -0.5).to(torch.bfloat16).to(dev)
+    big = torch.full((rows + 2, heads, n + 4), 3.0, dtype=torch.bfloat16, device=dev)
+    y = ops.head_linear(x, w, out=big[1:-1, :, :n], weight_kn=True)
+    assert torch.equal(y, ops.head_linear(x, w.transpose(1, 2).contiguous()))
+    assert bool((big[0] == 3).all() and (big[-1] == 3).all() and (big[1:-1, :, n:] == 3).all())
+    with pytest.raises(RuntimeError):
+        ops.head_linear(x, w.transpose(1, 2).contiguous() if n != k else w[:, 1:], weight_kn=True)

@@ -865,7 +865,7 @@ class UnbindHeads(torch.autograd.Function):
     def backward(ctx, dq, dk, dv):
         shape, dtype, device = ctx.like
         grads = [dq, dk, dv]
-        if all(d is not None for d in grads) and not torch.compiler.is_compiling() and _parts_of_rows(*grads):
+        if all(d is not None for d in grads) and _plain_dispatch() and _parts_of_rows(*grads):
             b, t, three, h, d = shape
             row = three * h * d
             return dq.as_strided(shape, (t * row, row, h * d, d, 1), dq.storage_offset())
@@ -917,7 +917,7 @@ class ChunkKDAFunction(torch.autograd.Function):
         # and parts of one row theirs as parts of one row (no gathering copy)
         more = (q, k, v, g, beta, cu, do.contiguous(), a_log, dtb, scale, lb, use_l2, use_gate,
                 use_sig, h0, dht, ctx.cu_cpu, False, q.dtype == torch.bfloat16)
-        if _parts_of_rows(q, k, v) and not torch.compiler.is_compiling():
+        if _plain_dispatch() and _parts_of_rows(q, k, v):   # (traced and wrapped tensors have no storage to look at)
             dqkv, dg, db, dh0, da, dbias = torch_ops.kda_chunk_bwd_packed(*more)
             dq, dk, dv = dqkv.unbind(1)
         else:

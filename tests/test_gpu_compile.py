@@ -68,6 +68,48 @@ def test_opcheck_custom_ops():
                                                          2, 128, 1e-5))
 
 
+@pytest.mark.parametrize("recurrent,grad_bf16", [(False, True), (True, False)])
+def test_opcheck_chunk_bwd(recurrent, grad_bf16):
+    """The backward ops, dq, dk, dv dense and as parts of one tensor."""
+    from sophia_amd import torch_ops  # noqa: F401
+    dev = _dev()
+    a = _kda_args(dev)
+    cu = torch.tensor([0, 50, 70], dtype=torch.int32, device=dev)
+    d_out = torch.randn(70, 2, 128, device=dev)
+    h0, dht = (torch.randn(2, 2, 128, 128, device=dev) * 0.05 for _ in range(2))
+    args = (a["q"], a["k"], a["v"], a["g"], a["beta"], cu, d_out, a["A_log"], a["dt_bias"], 0.088, -5.0, True, True,
+            True, h0, dht, cu.cpu(), recurrent, grad_bf16)
+    torch.library.opcheck(torch.ops.sophia.kda_chunk_bwd.default, args)
+    torch.library.opcheck(torch.ops.sophia.kda_chunk_bwd_packed.default, args)
+    dq, dk, dv, *rest = torch.ops.sophia.kda_chunk_bwd(*args)
+    dqkv, *rest_p = torch.ops.sophia.kda_chunk_bwd_packed(*args)
+    assert torch.equal(dqkv, torch.stack([dq, dk, dv], 1)) and all(map(torch.equal, rest, rest_p))
+
+
+def test_compiled_mixer_training_matches_eager():
+    """SophiaKDA forward and backward under torch.compile(fullgraph=True): the
+    output and every gradient of the eager module (whose q, k, v gradients are
+    written as parts of one row; the compiled form writes them apart)."""
+    from sophia_amd.config import ModelArgs
+    from sophia_amd.kda import SophiaKDA
+    dev = _dev()
+    torch.manual_seed(3)
+    eager = SophiaKDA(ModelArgs(dim=256, num_heads=2, use_cache=False)).to(dev).train()
+    twin = copy.deepcopy(eager)
+    compiled = torch.compile(twin, backend="aot_eager", fullgraph=True)
+    x = torch.randn(2, 70, 256, device=dev)
+    dy = torch.randn(2, 70, 256, device=dev)
+    got = {}
+    for name, fn, mod in (("eager", eager, eager), ("compiled", compiled, twin)):
+        xi = x.clone().requires_grad_(True)
+        y = fn(xi)
+        y.backward(dy)
+        got[name] = [y.detach(), xi.grad] + [p.grad for p in mod.parameters()]
+    for i, (e, c) in enumerate(zip(got["eager"], got["compiled"])):
+        # the same kernels; sums over tokens of the weights' gradients may be taken in another order
+        assert float((c - e).norm()) <= 1e-5 * float(e.norm()), i
+
+
 def test_compiled_chunk_kda_seam_matches_eager():
     """The FLA-signature prefill seam compiles with no graph break."""
     from sophia_amd import ops

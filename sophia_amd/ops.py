@@ -865,7 +865,9 @@ class UnbindHeads(torch.autograd.Function):
     def backward(ctx, dq, dk, dv):
         shape, dtype, device = ctx.like
         grads = [dq, dk, dv]
-        if all(d is not None for d in grads) and _plain_dispatch() and _parts_of_rows(*grads):
+        # (gradients with a history of their own are stacked: the one-row view would keep dq's alone)
+        history = torch.is_grad_enabled() and any(d is not None and d.requires_grad for d in grads)
+        if all(d is not None for d in grads) and not history and _plain_dispatch() and _parts_of_rows(*grads):
             b, t, three, h, d = shape
             row = three * h * d
             return dq.as_strided(shape, (t * row, row, h * d, d, 1), dq.storage_offset())

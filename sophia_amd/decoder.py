@@ -334,14 +334,11 @@ class SophiaMLA(nn.Module):
             self._causal(q[:npre], k, v, step["cu_prefill"], int(step["max_prefill_len"]), out[:npre],
                          cu_k=cu_k, cu_host=step["cu_prefill_host"], cu_k_host=cu_k_host)
         if nd > 0:
-            # the per-head products on the head kernel where only their values
-            # are asked for (bf16 weights, whole MFMA steps), else batched GEMMs.
-            # It reads both weights as they lie: an edit of them in place, by
-            # whatever means, is seen by the next step and by replays.
+            # the per-head products on the head kernel where it takes them, else
+            # batched GEMMs.  It reads both weights as they lie: an edit of them
+            # in place, by whatever means, is seen by the next step and by replays.
             w_k, w_v = self.k_up.weight, self.v_up.weight
-            heads_kernel = (x.dtype == torch.bfloat16 and r % 32 == 0 and d % 32 == 0 and q.stride(0) % 8 == 0
-                            and all(w.dtype == torch.bfloat16 and w.is_contiguous() for w in (w_k, w_v))
-                            and ops._values_only(q, w_k, w_v))
+            heads_kernel = ops.head_linear_takes(q, w_k, w_v)
             if heads_kernel:
                 qa = ops.head_linear(q[npre:], w_k.view(h, d, r), weight_kn=True)           # [D, h, r]
             else:

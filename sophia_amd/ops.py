@@ -1086,6 +1086,17 @@ def row_linear_situ_glu(x: torch.Tensor, weight: torch.Tensor, gate_softcap: flo
     return h
 
 
+def head_linear_takes(x: torch.Tensor, *weights: torch.Tensor) -> bool:
+    """Whether ``head_linear`` may take products of x [rows, heads, k] with
+    ``weights`` where only their values are asked for: bf16, whole MFMA steps
+    (rows and columns of a head), contiguous 16-byte aligned weights, aligned
+    rows and heads of x."""
+    return (_values_only(x, *weights) and x.dtype == torch.bfloat16 and x.stride(2) == 1 and x.stride(0) % 8 == 0
+            and x.stride(1) % 8 == 0 and x.data_ptr() % 16 == 0
+            and all(w.dtype == torch.bfloat16 and w.device == x.device and w.is_contiguous() and w.data_ptr() % 16 == 0
+                    and w.size(1) % 32 == 0 and w.size(0) // x.size(1) % 32 == 0 for w in weights))
+
+
 def head_linear(x: torch.Tensor, weight: torch.Tensor, *, out: torch.Tensor | None = None,
                 gate: torch.Tensor | None = None, weight_kn: bool = False) -> torch.Tensor:
     """Per-head projection (sophia_head_linear): out[r, h] = x[r, h] . weight[h]^T

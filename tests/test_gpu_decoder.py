@@ -300,6 +300,23 @@ def test_mla_decode_rows_see_up_weights_edited_in_place():
                 assert torch.equal(out, want)
 
 
+def test_mla_decode_rows_take_a_misaligned_weight():
+    """v_up as a contiguous view at an odd offset of a flat buffer (as flattened
+    parameters lie): the step takes it, with the aligned weight's result."""
+    dev = _dev()
+    m, x, step = _mla_decode(dev)
+    with torch.no_grad():
+        want = m.forward_mixed(x, step).float()
+        w = m.v_up.weight.data
+        flat = torch.zeros(w.numel() + 8, dtype=w.dtype, device=dev)
+        flat[1:1 + w.numel()].copy_(w.flatten())
+        m.v_up.weight.data = flat[1:1 + w.numel()].view_as(w)
+        assert m.v_up.weight.data_ptr() % 16 == 2
+        got = m.forward_mixed(x, step).float()
+    # bf16 roundings of the products and of the gate's in- and output in another order
+    assert float((got - want).norm()) <= 1e-2 * float(want.norm())
+
+
 FULL_DIMS = dict(vocab_size=1024, n_layers=4, ffn_hidden=3968, mla_q_rank=384, mla_kv_rank=128,
                  dim=1536, num_heads=16, max_seq_len=256, max_batch_size=4)
 

@@ -1,0 +1,46 @@
+"""The rules that take a call to a kernel of its own, on the CPU: forms that the
+kernel refuses must stay on the general path."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from sophia_amd import ops
+
+
+def _at_offset(t, elements):
+    """t as a contiguous view `elements` into a flat buffer (parameters of one
+    flat buffer lie like this)."""
+    flat = torch.zeros(t.numel() + elements + 8, dtype=t.dtype)
+    flat = flat[(-flat.data_ptr() // t.element_size()) % 8:]   # 16-byte aligned
+    view = flat[elements:elements + t.numel()].view(t.shape)
+    view.copy_(t)
+    return view
+
+
+@pytest.mark.parametrize("which", ["x", "k_up", "v_up"])
+def test_head_linear_rule_looks_at_alignment(which):
+    """The per-head kernel needs 16-byte aligned rows and weights."""
+    x = torch.randn(5, 2, 128).to(torch.bfloat16)
+    w = {"k_up": torch.randn(256, 32).to(torch.bfloat16), "v_up": torch.randn(256, 32).to(torch.bfloat16)}
+    with torch.no_grad():
+        for offset in (0, 8, 1, 4):
+            args = {"x": x, **w}
+            args[which] = _at_offset(args[which], offset)
+            assert ops.head_linear_takes(args["x"], args["k_up"], args["v_up"]) == (offset % 8 == 0), offset
+
+
+def test_head_linear_rule_forms():
+    """Other types, strides, widths, and calls that ask for more than values."""
+    x, w = torch.randn(5, 2, 128).to(torch.bfloat16), torch.randn(256, 32).to(torch.bfloat16)
+    with torch.no_grad():
+        assert ops.head_linear_takes(x, w, w)
+        wide = torch.zeros(5, 264, dtype=torch.bfloat16)
+        assert ops.head_linear_takes(wide[:, :256].view(5, 2, 128), w)
+        assert not ops.head_linear_takes(torch.zeros(5, 260, dtype=torch.bfloat16)[:, :256].view(5, 2, 128), w)
+        assert not ops.head_linear_takes(x.float(), w, w) and not ops.head_linear_takes(x, w.float(), w)
+        assert not ops.head_linear_takes(x, w.t().contiguous().t())
+        assert not ops.head_linear_takes(x, torch.zeros(256, 48, dtype=torch.bfloat16))
+        assert not ops.head_linear_takes(x[:, :, :48], torch.zeros(96, 32, dtype=torch.bfloat16))
+    assert not ops.head_linear_takes(x, w.clone().requires_grad_(True))

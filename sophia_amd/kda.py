@@ -65,9 +65,12 @@ class RuntimeLinear(nn.Module):
 
 def plain_linear(m: nn.Module) -> bool:
     """Whether ``m`` is a RuntimeLinear that another launch may take the place
-    of: no subclass or replacement, no bias, no hooks."""
-    return type(m) is RuntimeLinear and m.bias is None and not (
-        m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+    of: no subclass, replacement or ``forward`` of its own, no bias, and no
+    hooks, neither its own nor those registered for every module."""
+    hooks = torch.nn.modules.module
+    return type(m) is RuntimeLinear and m.bias is None and "forward" not in m.__dict__ and not (
+        m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+        or hooks._has_any_global_hook())
 
 
 class RMSNorm(nn.Module):

@@ -1016,7 +1016,7 @@ def _row_linear_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
     if not _values_only(x, weight):   # (before any look at a pointer: a wrapped tensor has none)
         return False
     if (x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or x.device.type != "cuda"
-            or weight.device != x.device or x.numel() == 0
+            or weight.device != x.device or x.numel() == 0 or weight.shape[0] == 0
             or k % 32 or weight.shape[0] % 16 or (weight.shape[0] > 512 * 16 and x.numel() > 8 * k)):
         return False
     return (weight.is_contiguous() and x.stride(-1) == 1 and x.data_ptr() % 16 == 0

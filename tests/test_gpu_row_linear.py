@@ -91,6 +91,8 @@ def test_linear_rule_and_general_path_agree():
         with torch.autograd.forward_ad.dual_level():
             dual = torch.autograd.forward_ad.make_dual(x.clone(), torch.ones_like(x))
             assert ops._few_rows(dual, w) is None
+        empty = ops.linear(x, w[:0])
+        assert empty.shape == (12, 0) and empty.dtype == torch.bfloat16
     wg = w.clone().requires_grad_(True)
     y = ops.linear(x, wg)
     y.float().sum().backward()

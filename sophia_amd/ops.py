@@ -986,6 +986,7 @@ def fused_recurrent_kda(q, k, v, g, beta, *, A_log=None, dt_bias=None, scale=Non
 
 # ------------------------------------------------------------------ projections of a few rows
 ROW_LINEAR_MAX = 32   # rows the few-row projection kernel takes
+_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
 
 
 def row_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
@@ -1011,8 +1012,6 @@ def _row_linear_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
     past two tiles per CU each work-group's reads of x weigh as much as the
     weight's."""
     k = x.shape[-1]
-    if torch.compiler.is_compiling() or x.numel() > ROW_LINEAR_MAX * k:   # (first: most other calls end here)
-        return False
     if not _values_only(x, weight):   # (before any look at a pointer: a wrapped tensor has none)
         return False
     if (x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or x.device.type != "cuda"
@@ -1040,13 +1039,21 @@ def _values_only(*tensors) -> bool:
         return False
     if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
         return False
-    return all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)
+    return all(type(t) in _PLAIN_TYPES for t in tensors)
 
 
 def _few_rows(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor | None:
     """x as the [rows, k] view (or copy) that the few-row kernel takes, or None
     where ``F.linear`` runs."""
-    if weight.dim() != 2 or x.dim() < 2 or x.shape[-1] != weight.shape[1] or not _row_linear_takes(x, weight):
+    # What a tracer's proxy, a nested or a sparse tensor cannot answer is not
+    # asked of them, and what ends most other calls comes first.
+    if torch.compiler.is_compiling() or type(x) not in _PLAIN_TYPES or type(weight) not in _PLAIN_TYPES:
+        return None
+    if weight.dim() != 2 or x.numel() > ROW_LINEAR_MAX * weight.shape[1]:
+        return None
+    if x.is_nested or x.layout is not torch.strided or weight.layout is not torch.strided:
+        return None
+    if x.dim() < 2 or x.shape[-1] != weight.shape[1] or not _row_linear_takes(x, weight):
         return None
     rows = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
     if rows.size(0) > 1 and (rows.stride(0) % 8 or rows.stride(0) < rows.size(1)):

@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from sophia_amd import ops
+from sophia_amd.kda import RuntimeLinear
 
 
 def _at_offset(t, elements):
@@ -44,3 +45,20 @@ def test_head_linear_rule_forms():
         assert not ops.head_linear_takes(x, torch.zeros(256, 48, dtype=torch.bfloat16))
         assert not ops.head_linear_takes(x[:, :, :48], torch.zeros(96, 32, dtype=torch.bfloat16))
     assert not ops.head_linear_takes(x, w.clone().requires_grad_(True))
+
+
+def test_linear_of_other_tensors():
+    """Proxies of a symbolic trace, nested and sparse tensors reach F.linear."""
+    torch.manual_seed(0)
+    m = RuntimeLinear(64, 32)
+    x = torch.randn(3, 64)
+    want = torch.nn.functional.linear(x, m.weight)
+    assert torch.equal(torch.fx.symbolic_trace(m)(x), want)
+    nested = m(torch.nested.nested_tensor([x[:2], x[1:]]))
+    assert torch.allclose(nested[0], want[:2], atol=1e-5) and torch.allclose(nested[1], want[1:], atol=1e-5)
+    for form in (x.to_sparse(), x.to_sparse_csr()):
+        assert torch.allclose(ops.linear(form, m.weight), want, atol=1e-5)
+    half = x.to(torch.bfloat16)
+    for other in (half.to_sparse(), torch.nested.nested_tensor([half]), half[0]):
+        assert ops._few_rows(other, m.weight.detach().to(torch.bfloat16)) is None
+    assert ops._few_rows(half, m.weight.detach().to(torch.bfloat16).to_sparse()) is None

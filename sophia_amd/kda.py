@@ -60,7 +60,10 @@ class RuntimeLinear(nn.Module):
             nn.init.zeros_(self.bias)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return ops.linear(x, self.weight, self.bias)
+        if torch.jit.is_scripting():   # (a script holds the projection itself)
+            return F.linear(x, self.weight, self.bias)
+        else:
+            return ops.linear(x, self.weight, self.bias)
 
 
 def plain_linear(m: nn.Module) -> bool:

@@ -62,3 +62,10 @@ def test_linear_of_other_tensors():
     for other in (half.to_sparse(), torch.nested.nested_tensor([half]), half[0]):
         assert ops._few_rows(other, m.weight.detach().to(torch.bfloat16)) is None
     assert ops._few_rows(half, m.weight.detach().to(torch.bfloat16).to_sparse()) is None
+
+
+@pytest.mark.parametrize("bias", [False, True])
+def test_runtime_linear_scripts(bias):
+    m = RuntimeLinear(64, 32, bias=bias)
+    x = torch.randn(3, 64)
+    assert torch.equal(torch.jit.script(m)(x), torch.nn.functional.linear(x, m.weight, m.bias))

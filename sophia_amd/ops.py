@@ -986,6 +986,7 @@ def fused_recurrent_kda(q, k, v, g, beta, *, A_log=None, dt_bias=None, scale=Non
 
 # ------------------------------------------------------------------ projections of a few rows
 ROW_LINEAR_MAX = 32   # rows the few-row projection kernel takes
+_CUS = 256            # compute units of the card
 _PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
 
 
@@ -1002,21 +1003,40 @@ def row_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     return y
 
 
-def _row_linear_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
+def row_linear_gains(rows: int, n: int, k: int, glu: bool = False) -> bool:
+    """Whether the few-row kernel is the faster form of a projection (``glu``:
+    with its activation).  us, library and kernel, weights from HBM:
+
+    Up to 8 rows (half tiles), while five tiles per work-group leave no CU a
+    second work-group: 1 row of 10,240 x 4,096 26.9 and 22.5, 8 rows of 8,384 x
+    1,536 11.6 and 7.7, 8,192 x 4,096 16.4 and 15.5; but 12,288 x 2,048 16.6 and
+    23.3, 8,192 x 6,144 26.7 and 29.0, the vocabulary's 65,536 x 1,536 42.0 and 41.1.
+
+    Past 8 rows the reads of x weigh as much as the weight's once there are two
+    tiles per CU: 16 rows of 8,192 x 2,048 13.2 and 11.4, 8,384 x 1,536 12.8 and
+    14.0, 32 rows of 4,096 x 1,536 9.8 and 7.9, 4,112 x 1,280 8.9 and 9.7 (the saved
+    launch of an activation is worth 2.5).  Past k = 2,048 sixteen wavefronts
+    share a tile: 16 rows of 4,096 x 3,968 18.8 and 11.7, x 4,608 17.7 and 18.9,
+    4,112 x 3,072 12.3 and 13.7.  There the library divides k by 256 where it can:
+    32 rows of 1,536 x 3,968 18.1 and 15.7, but x 3,840 11.6 and 15.3."""
+    if rows <= 8:
+        return n <= 5 * 8 * _CUS and k <= 4096
+    if k <= 2048:
+        return n <= (2 if rows <= 16 or glu else 1) * 16 * _CUS
+    return n <= 16 * _CUS and k <= 4096 and (rows <= 16 or k % 256 != 0)
+
+
+def _row_linear_takes(x: torch.Tensor, weight: torch.Tensor, glu: bool) -> bool:
     """Whether ``F.linear(x, weight)`` may run on the few-row kernel, and gains
     by it.  It may when nothing else than the values is asked of the call (no
-    gradient, trace, transform, mode or autocast) and the layout fits.  It gains
-    with up to 8 rows at any number of outputs (us, library and kernel: 8,384 x
-    1,536 12.7 and 8.5, the vocabulary's 65,536 43.8 and 43.0), and with up to 32
-    to 512 tiles of outputs (16 rows: 7,936 11.9 and 9.6, but 8,384 12.8 and 14.0):
-    past two tiles per CU each work-group's reads of x weigh as much as the
-    weight's."""
+    gradient, trace, transform, mode or autocast) and the layout fits."""
     k = x.shape[-1]
     if not _values_only(x, weight):   # (before any look at a pointer: a wrapped tensor has none)
         return False
+    n, size = weight.shape[0], x.numel()
     if (x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or x.device.type != "cuda"
-            or weight.device != x.device or x.numel() == 0 or weight.shape[0] == 0
-            or k % 32 or weight.shape[0] % 16 or (weight.shape[0] > 512 * 16 and x.numel() > 8 * k)):
+            or weight.device != x.device or size == 0 or n == 0 or k % 32 or n % 16
+            or not row_linear_gains(size // k, n, k, glu)):
         return False
     return (weight.is_contiguous() and x.stride(-1) == 1 and x.data_ptr() % 16 == 0
             and weight.data_ptr() % 16 == 0)
@@ -1042,7 +1062,7 @@ def _values_only(*tensors) -> bool:
     return all(type(t) in _PLAIN_TYPES for t in tensors)
 
 
-def _few_rows(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor | None:
+def _few_rows(x: torch.Tensor, weight: torch.Tensor, glu: bool = False) -> torch.Tensor | None:
     """x as the [rows, k] view (or copy) that the few-row kernel takes, or None
     where ``F.linear`` runs."""
     # What a tracer's proxy, a nested or a sparse tensor cannot answer is not
@@ -1053,7 +1073,7 @@ def _few_rows(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor | None:
         return None
     if x.is_nested or x.layout is not torch.strided or weight.layout is not torch.strided:
         return None
-    if x.dim() < 2 or x.shape[-1] != weight.shape[1] or not _row_linear_takes(x, weight):
+    if x.dim() < 2 or x.shape[-1] != weight.shape[1] or not _row_linear_takes(x, weight, glu):
         return None
     rows = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
     if rows.size(0) > 1 and (rows.stride(0) % 8 or rows.stride(0) < rows.size(1)):
@@ -1072,7 +1092,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
 
 def linear_situ_glu(x: torch.Tensor, weight: torch.Tensor, gate_softcap: float, up_softcap: float) -> torch.Tensor:
     """``situ_glu(F.linear(x, weight), ...)``: for a few rows in one launch."""
-    rows = _few_rows(x, weight)
+    rows = _few_rows(x, weight, glu=True)
     if rows is None:
         return situ_glu(torch.nn.functional.linear(x, weight), gate_softcap, up_softcap)
     h = row_linear_situ_glu(rows, weight, gate_softcap, up_softcap)

@@ -69,3 +69,16 @@ def test_runtime_linear_scripts(bias):
     m = RuntimeLinear(64, 32, bias=bias)
     x = torch.randn(3, 64)
     assert torch.equal(torch.jit.script(m)(x), torch.nn.functional.linear(x, m.weight, m.bias))
+
+
+def test_row_linear_rule_leaves_what_the_library_does_faster():
+    """Shapes measured slower on the few-row kernel than in the library, beside
+    ones measured faster (rows, outputs, k)."""
+    slower = [(1, 10256, 4096), (8, 12288, 2048), (8, 16384, 3968), (1, 65536, 2048), (8, 8192, 6144), (9, 512, 6144),
+              (16, 4112, 3072), (16, 1536, 4608), (17, 4112, 3968), (24, 4096, 2560), (32, 512, 3072),
+              (32, 8192, 3968), (32, 6144, 1280), (17, 8192, 8192)]
+    faster = [(1, 8384, 1536), (8, 10240, 4096), (8, 1536, 3968), (9, 8192, 2048), (16, 7936, 1536), (16, 4096, 4096),
+              (17, 2048, 384), (32, 1536, 2048), (32, 1536, 3968), (24, 4096, 3200), (32, 4096, 1536)]
+    assert [c for c in slower if ops.row_linear_gains(*c)] == []
+    assert [c for c in faster if not ops.row_linear_gains(*c)] == []
+    assert ops.row_linear_gains(32, 7936, 1536, glu=True) and not ops.row_linear_gains(17, 8192, 3968, glu=True)

@@ -76,9 +76,11 @@ def dtype_code(dtype: torch.dtype) -> int:
     raise RuntimeError(f"sophia_amd kernels take float32 or bfloat16 tensors, got {dtype}")
 
 
-def ptr(t: torch.Tensor | None):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+# Addresses go to the library as plain integers: its argument types make the
+# pointers, and an object made for each is host time of every call.
+def ptr(t: torch.Tensor | None) -> int | None:
+    return None if t is None else t.data_ptr()
 
 
-def stream_handle(device: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+def stream_handle(device: torch.device) -> int:
+    return torch.cuda.current_stream(device).cuda_stream

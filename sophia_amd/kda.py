@@ -349,7 +349,7 @@ class SophiaKDA(nn.Module):
         pad = int(y.size(1)) - sum(sizes)
         sizes = sizes + [pad] if pad else sizes
         split = _needs_grad(y) and ops._plain_dispatch()
-        qkv, gate, dd, beta = (ops.SplitColumns.apply(y, sizes) if split else y.split(sizes, 1))[:4]
+        qkv, gate, dd, beta = (ops.SplitColumns.apply(y, sizes) if split else y.split_with_sizes(sizes, 1))[:4]
         if not self.output_gate_full_rank:
             gate = self.output_gate_up(gate)
         return qkv, dd, beta, gate

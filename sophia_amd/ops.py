@@ -26,7 +26,7 @@ CHUNK_SIZE = 64
 
 
 def _gpu(t: torch.Tensor, name: str) -> None:
-    if not isinstance(t, torch.Tensor) or t.device.type != "cuda":
+    if not isinstance(t, torch.Tensor) or not t.is_cuda:
         raise RuntimeError(f"{name} must be a tensor on a ROCm GPU (sophia_amd has no CPU path)")
 
 
@@ -986,7 +986,9 @@ def fused_recurrent_kda(q, k, v, g, beta, *, A_log=None, dt_bias=None, scale=Non
 
 # ------------------------------------------------------------------ projections of a few rows
 ROW_LINEAR_MAX = 32   # rows the few-row projection kernel takes
+_ROW_LINEAR_K = 4096  # the largest k at which it gains
 _CUS = 256            # compute units of the card
+_is_compiling, _forward_ad = torch.compiler.is_compiling, torch.autograd.forward_ad
 _PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
 
 
@@ -1020,46 +1022,48 @@ def row_linear_gains(rows: int, n: int, k: int, glu: bool = False) -> bool:
     4,112 x 3,072 12.3 and 13.7.  There the library divides k by 256 where it can:
     32 rows of 1,536 x 3,968 18.1 and 15.7, but x 3,840 11.6 and 15.3."""
     if rows <= 8:
-        return n <= 5 * 8 * _CUS and k <= 4096
+        return n <= 5 * 8 * _CUS and k <= _ROW_LINEAR_K
     if k <= 2048:
         return n <= (2 if rows <= 16 or glu else 1) * 16 * _CUS
-    return n <= 16 * _CUS and k <= 4096 and (rows <= 16 or k % 256 != 0)
+    return n <= 16 * _CUS and k <= _ROW_LINEAR_K and (rows <= 16 or k % 256 != 0)
 
 
-def _row_linear_takes(x: torch.Tensor, weight: torch.Tensor, glu: bool) -> bool:
-    """Whether ``F.linear(x, weight)`` may run on the few-row kernel, and gains
-    by it.  It may when nothing else than the values is asked of the call (no
-    gradient, trace, transform, mode or autocast) and the layout fits."""
-    k = x.shape[-1]
+def _row_linear_takes(x: torch.Tensor, weight: torch.Tensor, n: int, k: int, glu: bool) -> bool:
+    """Whether ``F.linear(x, weight)`` (weight [n, k]) may run on the few-row
+    kernel, and gains by it.  It may when nothing else than the values is asked
+    of the call (no gradient, trace, transform, mode or autocast) and the layout
+    fits."""
     if not _values_only(x, weight):   # (before any look at a pointer: a wrapped tensor has none)
         return False
-    n, size = weight.shape[0], x.numel()
-    if (x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or x.device.type != "cuda"
-            or weight.device != x.device or size == 0 or n == 0 or k % 32 or n % 16
-            or not row_linear_gains(size // k, n, k, glu)):
-        return False
-    return (weight.is_contiguous() and x.stride(-1) == 1 and x.data_ptr() % 16 == 0
-            and weight.data_ptr() % 16 == 0)
+    size = x.numel()
+    return (x.dtype is torch.bfloat16 and weight.dtype is torch.bfloat16 and x.is_cuda and weight.device == x.device
+            and size > 0 and n > 0 and k % 32 == 0 and n % 16 == 0 and row_linear_gains(size // k, n, k, glu)
+            and weight.is_contiguous() and x.stride(-1) == 1 and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
 
 
 def _plain_dispatch() -> bool:
     """True outside of tracing, functorch transforms, forward-mode and dispatch
     or function modes."""
-    return not (torch.compiler.is_compiling() or torch.jit.is_tracing()
-                or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
-                or torch._C._functorch.peek_interpreter_stack() is not None
-                or torch.autograd.forward_ad._current_level >= 0)
+    c = torch._C
+    return not (_is_compiling() or c._is_tracing() or c._len_torch_dispatch_stack() or c._len_torch_function_stack()
+                or c._functorch.peek_interpreter_stack() is not None or _forward_ad._current_level >= 0)
 
 
 def _values_only(*tensors) -> bool:
     """True when a call on ``tensors`` computes plain values only: not traced,
     transformed (functorch, forward-mode), under a dispatch or function mode or
-    autocast, and with no gradient to record."""
-    if torch.is_autocast_enabled("cuda") or not _plain_dispatch():
+    autocast, and with no gradient to record.  (Plain loops: every projection of
+    a few rows asks this, and generators were a third of its 2.6 us.)"""
+    for t in tensors:
+        if type(t) not in _PLAIN_TYPES:
+            return False
+    if not _plain_dispatch() or torch.is_autocast_enabled("cuda"):
         return False
-    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
-        return False
-    return all(type(t) in _PLAIN_TYPES for t in tensors)
+    if torch.is_grad_enabled():
+        for t in tensors:
+            if t.requires_grad:
+                return False
+    return True
 
 
 def _few_rows(x: torch.Tensor, weight: torch.Tensor, glu: bool = False) -> torch.Tensor | None:
@@ -1067,13 +1071,16 @@ def _few_rows(x: torch.Tensor, weight: torch.Tensor, glu: bool = False) -> torch
     where ``F.linear`` runs."""
     # What a tracer's proxy, a nested or a sparse tensor cannot answer is not
     # asked of them, and what ends most other calls comes first.
-    if torch.compiler.is_compiling() or type(x) not in _PLAIN_TYPES or type(weight) not in _PLAIN_TYPES:
+    if _is_compiling() or type(x) not in _PLAIN_TYPES or x.numel() > ROW_LINEAR_MAX * _ROW_LINEAR_K:
         return None
-    if weight.dim() != 2 or x.numel() > ROW_LINEAR_MAX * weight.shape[1]:
+    if type(weight) not in _PLAIN_TYPES or weight.dim() != 2:
+        return None
+    n, k = weight.shape
+    if x.numel() > ROW_LINEAR_MAX * k:
         return None
     if x.is_nested or x.layout is not torch.strided or weight.layout is not torch.strided:
         return None
-    if x.dim() < 2 or x.shape[-1] != weight.shape[1] or not _row_linear_takes(x, weight, glu):
+    if x.dim() < 2 or x.shape[-1] != k or not _row_linear_takes(x, weight, n, k, glu):
         return None
     rows = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
     if rows.size(0) > 1 and (rows.stride(0) % 8 or rows.stride(0) < rows.size(1)):

@@ -898,18 +898,23 @@ __global__ __launch_bounds__(256) void mla_decode_merge_kernel(MlaArgs a) {
 // matched by the V^T reads).
 //
 // What bounds it: short sequences wait for memory (16 x 1,024 tokens x 16 heads
-// read and write 268 MB, 67 us at 4 TB/s, before any block is used twice; 177 ->
-// 125 us), long ones the vector instructions of the softmax (an exponential per
-// score at a quarter of the rate; 8 x 4,096 tokens 588 us, 936 TFLOP/s, 37 % of
-// the matrix peak; 1 x 8,192 379 -> 291 us).  Against 16x16x32 tiles, V
+// read and write 268 MB, 67 us at 4 TB/s, before any block is used twice; 163 ->
+// 114 us), long ones the vector instructions of the softmax (an exponential per
+// score at a quarter of the rate; 8 x 4,096 tokens 832 -> 615 us, 894 TFLOP/s, 36 %
+// of the matrix peak; 1 x 8,192 379 -> 297 us).  Against 16x16x32 tiles, V
 // transposed by matrix products and a register round trip for K and V: half the
 // vector instructions per score, and no registers held by the copies.  Measured
-// and not kept: key blocks from the last one down (132 us; each query block
-// then fetches its own keys first), 64-bit row products in the copies (131 us).
+// and not kept: key blocks from the last one down (7 us more; each query block
+// then fetches its own keys first), 64-bit row products in the copies (6 us more),
+// rescaling in every block (2 us more, and 66 us instead of 58 for 128 + 64 + 500
+// queries after 1,000 + 3,000 + 20 keys), and a reference point up to 2^8 behind
+// the running maximum: 4 us less, but the largest probability of a row is then
+// rounded to bf16 where it is exactly 1 otherwise, and the error against float64
+// grows by 3 % (0.00200 -> 0.00205; the running maximum's is that of the kernel
+// before it).
 constexpr int kFaD = 128;          // head dim
 constexpr int kFaQ = 128;          // queries per work-group
 constexpr int kFaK = 64;           // keys per block
-constexpr float kFaSlack = 8.f;    // see the running maximum
 
 struct FaArgs {
   const uint16_t *q, *k, *v;       // bf16 rows: token t, head h at t * stride + h * 128
@@ -1060,12 +1065,12 @@ __device__ __forceinline__ void causal_attn(const FaArgs &a) {
 #pragma unroll
     for (int i = 1; i < 32; ++i) mx = fmaxf(mx, st[i >> 4][i & 15]);
     mx = fmaxf(mx, lane_xor32(mx));
-    // The reference point m_run follows the maximum only where a score rises
-    // more than 2^kFaSlack above it (the exact same quotient, P up to 2^kFaSlack): after
-    // the first blocks the accumulators then need no rescaling.  m_run is finite
-    // once key 0 has been seen, and key 0 is in the first block.
+    // m_run is the running maximum itself, so that the largest probability is
+    // exactly 1 in bf16 (see above); where no row of the wavefront rose, nothing
+    // is rescaled.  m_run is finite once key 0 has been seen, and key 0 is in the
+    // first block.
     mx *= a.scale_log2;
-    if (__any(mx > m_run + kFaSlack)) {
+    if (__any(mx > m_run)) {
       const float m_new = fmaxf(m_run, mx);
       const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
       m_run = m_new;

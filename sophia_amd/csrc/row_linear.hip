@@ -173,8 +173,14 @@ int dispatch_batch(const RowLinearArgs &a, int units, hipStream_t st) {
     if (per <= 1) return launch<NW, NT, MT, 1, GLU, CAP4, HALF>(a, st);
     if (per <= 3) return launch<NW, NT, MT, 3, GLU, CAP4, HALF>(a, st);
   }
-  if (per <= 6 || NT > 2) return launch<NW, NT, MT, 6, GLU, CAP4, HALF>(a, st);   // (registers)
-  return launch<NW, NT, MT, 8, GLU, CAP4, HALF>(a, st);
+  // Past 128 registers of loads in a batch of eight (16 wavefronts have 128 each, two tiles each way take 16 of
+  // them per step) they spilled: 32 rows of 8,192 x 3,968 33.3 us with eight, 28.4 with six, x 6,144 57.3 and 35.6.
+  if constexpr (NT > 2 || NW * NT * MT > 32) {
+    return launch<NW, NT, MT, 6, GLU, CAP4, HALF>(a, st);
+  } else {
+    if (per <= 6) return launch<NW, NT, MT, 6, GLU, CAP4, HALF>(a, st);
+    return launch<NW, NT, MT, 8, GLU, CAP4, HALF>(a, st);
+  }
 }
 
 // At most eight rows: half tiles, one per work-group while that leaves no CU a

@@ -40,6 +40,7 @@ namespace sophia {
 namespace {
 
 constexpr int kRlRows = 32;    // most rows of x
+constexpr int kCus = 256;      // compute units of the card
 constexpr int kHlBatch = 8;    // head_linear: k-steps whose loads are issued together
 
 struct RowLinearArgs {
@@ -186,13 +187,15 @@ int dispatch_batch(const RowLinearArgs &a, int units, hipStream_t st) {
 // At most eight rows: half tiles, one per work-group while that leaves no CU a
 // second one, else two, and five where two per work-group are more work-groups
 // than two per CU (8,384 x 1,536: 7.5 us with five on 210 CUs, 8.8 with two,
-// 10.1 with four on 262: a second round for six).
+// 10.1 with four on 262: a second round for six).  Past five per CU the second
+// round comes with five too (8 rows: 10,240 x 1,536 8.4 us, 10,256 x 1,536 11.6),
+// and a library GEMM is the faster form of most shapes.
 template <bool GLU, bool CAP4>
 int dispatch_half(RowLinearArgs a, hipStream_t st) {
   a.tiles *= 2;
   const int units = (a.ksteps + 1) / 2;
-  if (a.tiles > 1024) return dispatch_batch<8, 5, 1, GLU, CAP4, true>(a, units, st);
-  if (a.tiles > 256) return dispatch_batch<8, 2, 1, GLU, CAP4, true>(a, units, st);
+  if (a.tiles > 4 * kCus) return dispatch_batch<8, 5, 1, GLU, CAP4, true>(a, units, st);
+  if (a.tiles > kCus) return dispatch_batch<8, 2, 1, GLU, CAP4, true>(a, units, st);
   if (units <= 32) return dispatch_batch<4, 1, 1, GLU, CAP4, true>(a, units, st);
   return dispatch_batch<8, 1, 1, GLU, CAP4, true>(a, units, st);
 }
@@ -202,7 +205,7 @@ int dispatch_half(RowLinearArgs a, hipStream_t st) {
 // with one tile, 9.7 with two, four on 124 CUs 13.8).
 template <int NW, int MT, bool GLU, bool CAP4>
 int dispatch_tiles(const RowLinearArgs &a, hipStream_t st) {
-  if (a.tiles > 256) return dispatch_batch<NW, 2, MT, GLU, CAP4, false>(a, a.ksteps, st);
+  if (a.tiles > kCus) return dispatch_batch<NW, 2, MT, GLU, CAP4, false>(a, a.ksteps, st);
   return dispatch_batch<NW, 1, MT, GLU, CAP4, false>(a, a.ksteps, st);
 }
 

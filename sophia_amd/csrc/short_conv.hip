@@ -789,7 +789,8 @@ extern "C" int sophia_short_conv_bwd(const void *x, int64_t x_row_stride, const 
     return set_error(SOPHIA_ERR_WORKSPACE, "short_conv_bwd: workspace %zu bytes < required %zu", workspace_bytes,
                      need);
   const int groups = conv_bwd_groups(total_tokens);
-  SOPHIA_REQUIRE(groups / 4 < 65535, "short_conv_bwd: too many tokens for one launch");
+  // (the entry point's range, 33.5 million tokens; the grid itself is checked below)
+  SOPHIA_REQUIRE(groups < 4 * 65535, "short_conv_bwd: too many tokens for one launch");
   ConvBwdArgs a{x, x_row_stride, dy, dy_row_stride, dx, dx_row_stride, weight, conv_state, n_state_slots,
                 state_slots, cu_seqlens, n_seqs, total_tokens, channels, read_history, static_cast<float *>(workspace),
                 dweight, groups, (channels / kBVec + kBLanes - 1) / kBLanes};

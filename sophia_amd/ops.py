@@ -1031,12 +1031,14 @@ def row_linear_gains(rows: int, n: int, k: int, glu: bool = False) -> bool:
 def _row_linear_takes(x: torch.Tensor, weight: torch.Tensor, n: int, k: int, glu: bool) -> bool:
     """Whether ``F.linear(x, weight)`` (weight [n, k]) may run on the few-row
     kernel, and gains by it.  It may when nothing else than the values is asked
-    of the call (no gradient, trace, transform, mode or autocast) and the layout
-    fits."""
+    of the call (no gradient, trace, transform, mode or autocast), the layout
+    fits and the tensors lie on the current device (F.linear changes to theirs,
+    a launch of ours goes to the current one)."""
     if not _values_only(x, weight):   # (before any look at a pointer: a wrapped tensor has none)
         return False
     size = x.numel()
     return (x.dtype is torch.bfloat16 and weight.dtype is torch.bfloat16 and x.is_cuda and weight.device == x.device
+            and x.get_device() == torch.cuda.current_device()
             and size > 0 and n > 0 and k % 32 == 0 and n % 16 == 0 and row_linear_gains(size // k, n, k, glu)
             and weight.is_contiguous() and x.stride(-1) == 1 and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
 

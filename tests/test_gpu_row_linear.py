@@ -107,6 +107,18 @@ def test_linear_rule_and_general_path_agree():
     assert seen == [None]
 
 
+def test_linear_of_another_device_stays_with_the_library(monkeypatch):
+    """Tensors of a device that is not the current one: F.linear changes to it, a
+    launch of the kernel would go to the current device."""
+    from sophia_amd import ops
+    dev = _dev()
+    x, w = (t.to(dev) for t in _data(12, 64, 96))
+    with torch.no_grad():
+        assert ops._few_rows(x, w) is not None
+        monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+        assert ops._few_rows(x, w) is None
+
+
 @pytest.mark.parametrize("rows", [5, 40])
 def test_feed_forward_few_rows_and_graph(rows):
     """FeedForward with the one-launch projection and activation (5 rows) and

@@ -126,7 +126,7 @@ __device__ __forceinline__ void load_depth(const MixArgs &a, int64_t row, int b,
 // template arguments so that the per-block sums, and for bf16 the values
 // themselves (4 VGPRs per chunk and block), stay in registers between the
 // score pass and the mix pass; fp32 values are read again (cache hits).
-template <int DEPTH, int CPT, bool BF16>
+template <int DEPTH, int CPT, bool BF16, bool PLAIN>
 __global__ __launch_bounds__(256) void attn_res_mix_kernel(MixArgs a) {
   constexpr int kDt = BF16 ? SOPHIA_DTYPE_BF16 : SOPHIA_DTYPE_F32;
   __shared__ float red[2 * DEPTH + 1][4];
@@ -144,6 +144,9 @@ __global__ __launch_bounds__(256) void attn_res_mix_kernel(MixArgs a) {
   // the score norm's weight): one memory round trip.  For the few rows of a
   // decode step that, and sums without the LDS crossbar, are most of the kernel's
   // length: 8 rows, depth 8 with the residual: 6.7 -> 5.4 us; 2,048 rows 18.9 -> 16.4.
+  // PLAIN (of a single block, neither residual nor norm) leaves them out: they
+  // would be as many loads as there are others (2,048 rows of 4,096 bf16 columns
+  // 7.9 us, 9.0 with them; under a branch the others' 6.4 us at 1,536 became 6.7).
   const uint8_t *res_row = static_cast<const uint8_t *>(a.residual != nullptr ? a.residual : a.partial) +
                            row * (a.residual != nullptr ? a.residual_stride : a.partial_stride) * (BF16 ? 2 : 4);
   const float *onw = a.out_norm_w != nullptr ? a.out_norm_w : a.norm_w;
@@ -156,13 +159,14 @@ __global__ __launch_bounds__(256) void attn_res_mix_kernel(MixArgs a) {
 #pragma unroll
       for (int b = 0; b < DEPTH; ++b)
         raw[b][k] = *reinterpret_cast<const u4 *>(static_cast<const uint16_t *>(depth_value(a, row, b)) + 8 * c);
-      rres[k] = *reinterpret_cast<const u4 *>(reinterpret_cast<const uint16_t *>(res_row) + 8 * c);
+      if constexpr (!PLAIN)
+        rres[k] = *reinterpret_cast<const u4 *>(reinterpret_cast<const uint16_t *>(res_row) + 8 * c);
     }
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       wn[k][i] = *reinterpret_cast<const f4 *>(a.norm_w + 8 * c + 4 * i);
       wq4[k][i] = *reinterpret_cast<const f4 *>(a.query_w + 8 * c + 4 * i);
-      wo[k][i] = *reinterpret_cast<const f4 *>(onw + 8 * c + 4 * i);
+      if constexpr (!PLAIN) wo[k][i] = *reinterpret_cast<const f4 *>(onw + 8 * c + 4 * i);
     }
   }
   asm volatile("" ::: "memory");   // (none is sunk to its use)
@@ -171,7 +175,7 @@ __global__ __launch_bounds__(256) void attn_res_mix_kernel(MixArgs a) {
   for (int k = 0; k < CPT; ++k) {
     const int c = tid + k * blockDim.x;
     if (c < chunks) {
-      if (a.residual != nullptr) {  // uniform: partial <- partial + residual, written out once
+      if (!PLAIN && a.residual != nullptr) {  // uniform: partial <- partial + residual, written out once
         float v[8];
         if constexpr (BF16) {
           float r[8];
@@ -261,7 +265,7 @@ __global__ __launch_bounds__(256) void attn_res_mix_kernel(MixArgs a) {
       for (int i = 0; i < 8; ++i) sq = fmaf(o[k][i], o[k][i], sq);
     }
   }
-  if (a.out_norm_w != nullptr) {  // uniform over the grid
+  if (!PLAIN && a.out_norm_w != nullptr) {  // uniform over the grid
     sq = wave_sum_dpp(sq);
     if (lane == 0) red[2 * DEPTH][wave] = sq;
     lds_barrier();
@@ -619,6 +623,10 @@ __global__ __launch_bounds__(1024) void gated_head_norm_dw_reduce_kernel(GateBwd
 // once; 64 bytes of a row per instruction fetch a line twice: 84 us).  240 rows
 // of U[1, 4096) keys, 251 MB: 100 -> 69 us, 3.7 TB/s, where a plain reduction of
 // 1 GiB reads 3.9 TB/s on the same card.
+// Rows of at most 16 keys take 0.2 us more than with one tile in flight (5.6 ->
+// 5.8; 512 rows 6.7 -> 7.4), 128 rows and more of 100 keys 0.5 (7.8 -> 8.4).  Paths
+// of their own for the last tiles, without the loads that nothing uses: not kept
+// (100 keys 7.0 -> 7.8 us: the code is then twice as long; 600 keys 9.7 -> 10.4).
 struct MlaArgs {
   const void *qa;        // [rows, heads, R]
   int64_t qa_stride;     // elements between rows
@@ -1264,11 +1272,15 @@ extern "C" int sophia_attn_res_mix(const void *partial, int64_t partial_stride, 
   const int threads = ((chunks + per_thread - 1) / per_thread + 63) / 64 * 64;
   const dim3 grid(static_cast<unsigned>(rows)), block(threads);
   const hipStream_t st = static_cast<hipStream_t>(stream);
+  const bool plain = n_blocks == 0 && residual == nullptr && out_norm_weight == nullptr;
   const int key = (n_blocks + 1) * 4 + (per_thread - 1) * 2 + (dtype == SOPHIA_DTYPE_BF16 ? 1 : 0);
   switch (key) {
 #define SOPHIA_MIX_CASE(d, cpt, bf)                                                              \
   case d * 4 + (cpt - 1) * 2 + bf:                                                                \
-    hipLaunchKernelGGL((attn_res_mix_kernel<d, cpt, bf != 0>), grid, block, 0, st, a);           \
+    if (plain)                                                                                    \
+      hipLaunchKernelGGL((attn_res_mix_kernel<d, cpt, bf != 0, d == 1>), grid, block, 0, st, a);  \
+    else                                                                                          \
+      hipLaunchKernelGGL((attn_res_mix_kernel<d, cpt, bf != 0, false>), grid, block, 0, st, a);   \
     break;
 #define SOPHIA_MIX_DEPTH(d) \
   SOPHIA_MIX_CASE(d, 1, 0) SOPHIA_MIX_CASE(d, 1, 1) SOPHIA_MIX_CASE(d, 2, 0) SOPHIA_MIX_CASE(d, 2, 1)

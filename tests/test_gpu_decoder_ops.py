@@ -75,6 +75,20 @@ def test_attn_res_mix_matches_fp64_reference(dtype, rows, n_blocks, dim, normed)
     _check(y, _mix_ref(partial, completed, w, q, 1e-5, wo, 1e-5), dtype)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,dim", [(300, 2056), (7, 1536), (2, 4096)])
+def test_attn_res_mix_of_one_block_is_the_block(dtype, rows, dim):
+    """The form without residual, norm or completed blocks: a softmax over one
+    score is 1, so the result is the block, bit for bit."""
+    from sophia_amd import ops
+    dev = _dev()
+    g = torch.Generator(device="cpu").manual_seed(rows + dim)
+    partial = torch.randn(rows, dim, generator=g).to(dev, dtype)
+    w, q = torch.rand(dim, generator=g).to(dev), torch.randn(dim, generator=g).to(dev)
+    y = ops.attn_res_mix(partial, partial.new_empty(rows, 0, dim), w, q, 1e-5)
+    assert torch.equal(y, partial)
+
+
 def test_attn_res_mix_matches_oracle_on_strided_store_views():
     """Leading dims [B, S], completed a narrow view of a wider depth store and
     partial a strided slice, as the decoder passes them; checked against the

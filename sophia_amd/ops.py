@@ -992,12 +992,28 @@ _is_compiling, _forward_ad = torch.compiler.is_compiling, torch.autograd.forward
 _PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
 
 
+def _row_linear_operands(x: torch.Tensor, weight: torch.Tensor) -> None:
+    """What the few-row kernels assume of x [rows, k] and weight [n, k] (the
+    library itself sees addresses and sizes alone)."""
+    if x.dim() != 2 or weight.dim() != 2 or x.size(1) != weight.size(1):
+        raise RuntimeError(f"x [rows, k] and weight [n, k] must share k, got {tuple(x.shape)} and {tuple(weight.shape)}")
+    if not weight.is_contiguous() or x.stride(1) != 1:
+        raise RuntimeError("weight must be contiguous and the rows of x dense")
+    _gpu(x, "x")
+    if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or weight.device != x.device:
+        raise RuntimeError("x and weight must be bf16 on one device")
+
+
 def row_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """``F.linear(x, weight)`` of at most ROW_LINEAR_MAX rows in bf16
     (sophia_row_linear): x [rows, k] with dense rows, weight [n, k] contiguous,
     k a multiple of 32, n of 16.  Returns [rows, n]."""
-    rows, k = int(x.size(0)), int(x.size(1))
-    n = int(weight.size(0))
+    _row_linear_operands(x, weight)
+    return _row_linear(x, weight)
+
+
+def _row_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    (rows, k), n = x.shape, weight.shape[0]
     y = torch.empty((rows, n), dtype=x.dtype, device=x.device)
     rc = nat.lib().sophia_row_linear(x.data_ptr(), x.stride(0) if rows > 1 else k, weight.data_ptr(), k, y.data_ptr(),
                                      n, rows, n, k, nat.stream_handle(x.device))
@@ -1095,7 +1111,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
     rows = _few_rows(x, weight) if bias is None else None
     if rows is None:
         return torch.nn.functional.linear(x, weight, bias)
-    y = row_linear(rows, weight)
+    y = _row_linear(rows, weight)
     return y if x.dim() == 2 else y.view(*x.shape[:-1], weight.shape[0])
 
 
@@ -1104,7 +1120,7 @@ def linear_situ_glu(x: torch.Tensor, weight: torch.Tensor, gate_softcap: float, 
     rows = _few_rows(x, weight, glu=True)
     if rows is None:
         return situ_glu(torch.nn.functional.linear(x, weight), gate_softcap, up_softcap)
-    h = row_linear_situ_glu(rows, weight, gate_softcap, up_softcap)
+    h = _row_linear_situ_glu(rows, weight, gate_softcap, up_softcap)
     return h if x.dim() == 2 else h.view(*x.shape[:-1], h.size(1))
 
 
@@ -1112,8 +1128,14 @@ def row_linear_situ_glu(x: torch.Tensor, weight: torch.Tensor, gate_softcap: flo
     """``situ_glu(F.linear(x, weight), ...)`` of at most ROW_LINEAR_MAX rows in
     one launch (sophia_row_linear_situ_glu), the activation formed on the fp32
     sums: x [rows, k], weight [2H, k] ([gate | up], H a multiple of 8)."""
-    rows, k = int(x.size(0)), int(x.size(1))
-    hidden = int(weight.size(0)) // 2
+    _row_linear_operands(x, weight)
+    if weight.size(0) % 2:
+        raise RuntimeError("weight must have an even number of rows")
+    return _row_linear_situ_glu(x, weight, gate_softcap, up_softcap)
+
+
+def _row_linear_situ_glu(x: torch.Tensor, weight: torch.Tensor, gate_softcap: float, up_softcap: float) -> torch.Tensor:
+    (rows, k), hidden = x.shape, weight.shape[0] // 2
     h = torch.empty((rows, hidden), dtype=x.dtype, device=x.device)
     rc = nat.lib().sophia_row_linear_situ_glu(
         x.data_ptr(), x.stride(0) if rows > 1 else k, weight.data_ptr(), k, h.data_ptr(), hidden, rows, hidden, k,

@@ -82,3 +82,21 @@ def test_row_linear_rule_leaves_what_the_library_does_faster():
     assert [c for c in slower if ops.row_linear_gains(*c)] == []
     assert [c for c in faster if not ops.row_linear_gains(*c)] == []
     assert ops.row_linear_gains(32, 7936, 1536, glu=True) and not ops.row_linear_gains(17, 8192, 3968, glu=True)
+
+
+@pytest.mark.parametrize("form", [ops.row_linear, lambda x, w: ops.row_linear_situ_glu(x, w, 4.0, 25.0)])
+def test_row_linear_refuses_operands_that_do_not_fit(form):
+    """Called directly: a weight of another k (the kernel would read past it),
+    other strides and dimensions, and host tensors raise before any launch."""
+    x, w = torch.zeros(4, 96, dtype=torch.bfloat16), torch.zeros(32, 96, dtype=torch.bfloat16)
+    for other in (w[:, :64].contiguous(), torch.zeros(32, dtype=torch.bfloat16), w.view(2, 16, 96)):
+        with pytest.raises(RuntimeError, match="share k"):
+            form(x, other)
+    with pytest.raises(RuntimeError, match="share k"):
+        form(x.view(2, 2, 96), w)
+    with pytest.raises(RuntimeError, match="contiguous"):
+        form(x, w.t().contiguous().t())
+    with pytest.raises(RuntimeError, match="dense"):
+        form(x.t().contiguous().t(), w)
+    with pytest.raises(RuntimeError, match="GPU"):
+        form(x, w)
